@@ -1,5 +1,5 @@
 // Launcher declarations: one explicit instantiation per working precision
-// lives in sdns_f32.hip / sdns_f64.hip; the C-ABI layer (sdns_abi.hip) calls
+// lives in sdns_part.hip; the C-ABI layer (sdns_abi.hip) calls
 // these with runtime line lengths.  Every launcher returns 0, or -1 when the
 // length has no compiled kernel.
 #pragma once

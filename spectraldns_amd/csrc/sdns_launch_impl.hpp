@@ -1,5 +1,5 @@
-// Launcher bodies (size dispatch) and elementwise kernels.  Included once per
-// working precision by sdns_f32.hip / sdns_f64.hip.
+// Launcher bodies (size dispatch) and elementwise kernels, instantiated per pass
+// group and working precision by sdns_part.hip.
 #pragma once
 #include <type_traits>
 
@@ -741,14 +741,22 @@ template <typename Rt> int launch_errnorm(const void* err, const void* u0, const
 
 }  // namespace sdns
 
-#define SDNS_INSTANTIATE(Rt)                                                                     \
+// Explicit instantiations, one group per translation unit (sdns_part.hip).
+#define SDNS_PART_P1(Rt) \
+  namespace sdns { template int launch_p1<Rt>(int, int, const P1Args<Rt>&, hipStream_t); }
+#define SDNS_PART_P2(Rt) \
+  namespace sdns { template int launch_p2<Rt>(int, int, const P2Args<Rt>&, hipStream_t); }
+#define SDNS_PART_P3(Rt) \
+  namespace sdns { template int launch_p3<Rt>(int, int, const P3Args<Rt>&, hipStream_t); }
+#define SDNS_PART_P5(Rt) \
+  namespace sdns { template int launch_p5<Rt>(int, int, int, const P5Args<Rt>&, hipStream_t, int*); }
+#define SDNS_PART_LINES(Rt)                                                                      \
   namespace sdns {                                                                               \
-  template int launch_p1<Rt>(int, int, const P1Args<Rt>&, hipStream_t);                          \
-  template int launch_p2<Rt>(int, int, const P2Args<Rt>&, hipStream_t);                          \
-  template int launch_p3<Rt>(int, int, const P3Args<Rt>&, hipStream_t);                          \
-  template int launch_p5<Rt>(int, int, int, const P5Args<Rt>&, hipStream_t, int*);               \
   template int launch_strided<Rt>(int, int, int, int, const StridedArgs<Rt>&, hipStream_t);      \
   template int launch_z<Rt>(int, int, int, int, const ZArgs<Rt>&, hipStream_t);                  \
+  }
+#define SDNS_PART_POINTS(Rt)                                                                     \
+  namespace sdns {                                                                               \
   template int launch_elementwise<Rt>(int, const EwArgs<Rt>&, hipStream_t);                      \
   template int launch_energy<Rt>(const EwArgs<Rt>&, double*, int, hipStream_t);                  \
   template int launch_force_reduce<Rt>(const EwArgs<Rt>&, Rt, double*, int, hipStream_t);        \
