@@ -98,7 +98,7 @@ struct sdns_plan {
   void* ws = nullptr;
   size_t ws_bytes = 0;
   bool ws_owned = false;
-  char *bufA = nullptr, *bufB = nullptr, *stB = nullptr, *stC = nullptr, *stClo = nullptr;
+  char *bufA = nullptr, *bufB = nullptr, *st[3] = {nullptr, nullptr, nullptr};  // RK stage states or right-hand sides (see P5Args)
   double* part = nullptr;
   int max_blocks = 0;
   // per-pass event timing
@@ -123,6 +123,7 @@ struct sdns_closure {
   float *y = nullptr, *gy = nullptr, *t = nullptr, *wpart = nullptr, *bpart = nullptr;
   float *phys = nullptr, *tauphys = nullptr;
   char *tauhat = nullptr, *src = nullptr;  // 6 and 3 complex64 spectral fields
+  char* stage = nullptr;                   // 3 fields: the stage state of per-stage evaluations (in tauhat)
   double *lpart = nullptr, *loss = nullptr;
   sdns::ClosureWeights w{};
   bool have_params = false;
@@ -225,9 +226,7 @@ int assign_workspace(sdns_plan* p, void* base, size_t bytes) {
   char* c = (char*)base;
   p->bufA = c; c += p->szA;
   p->bufB = c; c += p->szB;
-  p->stB = c; c += p->szS;
-  p->stC = c; c += p->szS;
-  p->stClo = c; c += p->szS;
+  for (auto& b : p->st) { b = c; c += p->szS; }
   p->part = (double*)c;
   p->ws = base;
   p->ws_bytes = bytes;
@@ -432,13 +431,12 @@ template <typename Rt> StridedArgs<Rt> p2_given_args(const sdns_plan* p) {
   return a;
 }
 
-// P1..P4 of one convection evaluation from the state u into W4 (= bufB).  w:
+// P1..P4 of one convection evaluation from the state of a1 into W4 (= bufB).  a1.w:
 // the vorticity of u when given (the velocity-vorticity solver), otherwise
 // null and the passes form curl(u).
-template <typename Rt> int conv_passes(sdns_plan* p, const void* u, const void* w = nullptr) {
+template <typename Rt> int conv_passes(sdns_plan* p, const P1Args<Rt>& a1) {
   const int M0 = p->M[0], M1 = p->M[1];
-  P1Args<Rt> a1 = p1_args<Rt>(p, u);
-  a1.w = w;
+  const void* w = a1.w;
   tstart(p, 0);
   if (launch_p1<Rt>(M0, p->var[0], a1, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", M0);
   tstop(p);
@@ -475,11 +473,39 @@ template <typename Rt> P5Args<Rt> p5_args(const sdns_plan* p, double nu) {
   return a;
 }
 
+// One classical RK4 step (integrators.py:149-159, a and b of 183-191 in the
+// working precision): argument blocks of its stages from the start value u and
+// the stage arrays st[0..2].
+template <typename Rt> struct RkStage {
+  static Rt a(int rk) { return rk == 0 || rk == 3 ? Rt(1. / 6.) : Rt(1. / 3.); }
+  static Rt b(int rk) { return rk < 2 ? Rt(0.5) : Rt(1); }
+  static int mode(int rk) { return rk == 0 ? P5_RK0 : (rk < 3 ? P5_RK12 : P5_RK3); }
+  static void p5(P5Args<Rt>& x, int keep, int rk, Rt dt, void* u, char* const st[3]) {
+    const int n = keep == KEEP_SUM ? 1 : 3;  // KEEP_SUM: one stage state, st[0], and the sum, st[1]
+    x.u = u;
+    x.s = rk > 0 ? st[(rk - 1) % n] : nullptr;
+    x.out = rk < 3 ? st[rk % n] : nullptr;
+    x.b1 = keep == KEEP_SUM ? st[1] : st[0];
+    x.b2 = st[1];
+    x.adt = a(rk) * dt;
+    x.bdt = b(rk) * dt;
+    x.sdt = rk > 0 ? b(rk - 1) * dt : Rt(0);
+    x.a12 = a(1) * dt;
+  }
+  // the state that stage rk's RHS reads
+  static void p1(P1Args<Rt>& x, int keep, int rk, Rt dt, const void* u, char* const st[3]) {
+    const void* s = rk > 0 ? st[keep == KEEP_SUM ? 0 : rk - 1] : nullptr;
+    x.u = s && keep != KEEP_RHS ? s : u;
+    x.d = keep == KEEP_RHS ? s : nullptr;
+    x.ds = rk > 0 ? b(rk - 1) * dt : Rt(0);
+  }
+};
+
 template <typename Rt> int compute_rhs(sdns_plan* p, const void* u, void* rhs, double nu, const void* src, void* ph) {
   int rc;
-  if ((rc = conv_passes<Rt>(p, u))) return rc;
+  if ((rc = conv_passes<Rt>(p, p1_args<Rt>(p, u)))) return rc;
   P5Args<Rt> a = p5_args<Rt>(p, nu);
-  a.A = const_cast<void*>(u); a.rhs = rhs; a.phat = ph; a.source = src;
+  a.u = const_cast<void*>(u); a.rhs = rhs; a.phat = ph; a.source = src;
   tstart(p, 4);
   if (launch_p5<Rt>(p->M[0], p->var[4], P5_RHS, a, p->stream, nullptr))
     return fail(SDNS_ERR_UNSUPPORTED, "x length %d", p->M[0]);
@@ -489,15 +515,29 @@ template <typename Rt> int compute_rhs(sdns_plan* p, const void* u, void* rhs, d
 
 template <typename Rt> int convection(sdns_plan* p, const void* u, void* rhs, const void* w = nullptr) {
   int rc;
-  if ((rc = conv_passes<Rt>(p, u, w))) return rc;
+  P1Args<Rt> a1 = p1_args<Rt>(p, u);
+  a1.w = w;
+  if ((rc = conv_passes<Rt>(p, a1))) return rc;
   P5Args<Rt> a = p5_args<Rt>(p, 0.0);
-  a.A = const_cast<void*>(u); a.rhs = rhs; a.conv_only = 1;
+  a.u = const_cast<void*>(u); a.rhs = rhs; a.conv_only = 1;
   if (launch_p5<Rt>(p->M[0], p->var[4], P5_RHS, a, p->stream, nullptr))
     return fail(SDNS_ERR_UNSUPPORTED, "x length %d", p->M[0]);
   return 0;
 }
 
 template <typename Rt> EwArgs<Rt> ew_args(sdns_plan* p);
+
+// out = a.u + a.ds a.d, a whole state.
+template <typename Rt> int form_state(sdns_plan* p, void* out, const P1Args<Rt>& a) {
+  LinArgs<Rt> l{};
+  l.out = out;
+  l.n = 3L * p->N[0] * p->N[1] * p->Nh;
+  l.nterms = 2;
+  l.x[0] = a.u; l.c[0] = Rt(1);
+  l.x[1] = a.d; l.c[1] = a.ds;
+  if (launch_lincomb<Rt>(l, p->stream)) return fail(SDNS_ERR_HIP, "stage state");
+  return 0;
+}
 
 // Network forward on the closure's packed input x0 -> y (FP32, 6 of 8 channels).
 // keep_pre: store the pre-activations z1, z2 (the backward pass reads them;
@@ -537,24 +577,29 @@ int closure_source(sdns_closure* c, sdns_plan* p, const void* u, float in_scale,
 template <typename Rt> int rk4_steps(sdns_plan* p, void* u, void* ulo, const double* dts, int nsteps, double nu,
                                       double* diag, void* ph, const void* src = nullptr, sdns_closure* cl = nullptr,
                                       float in_scale = 1.f, float out_scale = 1.f, int per_stage = 0) {
-  // a, b and dt in the working precision (integrators.py:185-186, config.py:123-127)
-  const Rt a[4] = {Rt(1. / 6.), Rt(1. / 3.), Rt(1. / 3.), Rt(1. / 6.)};
-  const Rt b[3] = {Rt(0.5), Rt(0.5), Rt(1.)};
+  using RK = RkStage<Rt>;
+  const int keep = rk_keep<Rt>(p->M[0] != p->N[0], ulo != nullptr);
   const Rt nur = (Rt)nu;
   for (int s = 0; s < nsteps; ++s) {
     const Rt dt = (Rt)dts[s];
     for (int rk = 0; rk < 4; ++rk) {
       int rc;
-      const void* stage_in = rk == 0 ? u : (const void*)p->stB;
-      if (cl && (per_stage || rk == 0) && (rc = closure_source(cl, p, stage_in, in_scale, out_scale))) return rc;
-      if ((rc = conv_passes<Rt>(p, stage_in))) return rc;
+      P1Args<Rt> a1 = p1_args<Rt>(p, u);
+      RK::p1(a1, keep, rk, dt, u, p->st);
+      if (cl && (per_stage || rk == 0)) {
+        const void* state = a1.u;
+        if (a1.d) {  // the closure's transform reads the stage state as an array
+          if ((rc = form_state<Rt>(p, cl->stage, a1))) return rc;
+          state = cl->stage;
+        }
+        if ((rc = closure_source(cl, p, state, in_scale, out_scale))) return rc;
+      }
+      if ((rc = conv_passes<Rt>(p, a1))) return rc;
       P5Args<Rt> pa = p5_args<Rt>(p, nu);
-      pa.A = u; pa.B = p->stB; pa.Cacc = p->stC;
-      if (ulo) { pa.Alo = ulo; pa.Clo = p->stClo; }
+      RK::p5(pa, keep, rk, dt, u, p->st);
+      pa.lo = ulo;
       pa.source = cl ? (const void*)cl->src : src;
-      pa.adt = a[rk] * dt;
-      pa.bdt = rk < 3 ? b[rk] * dt : Rt(0);
-      const int mode = rk == 0 ? P5_RK0 : (rk < 3 ? P5_RK12 : P5_RK3);
+      const int mode = RK::mode(rk);
       pa.partials = (rk == 3 && diag) ? p->part : nullptr;
       pa.phat = (rk == 3 && s == nsteps - 1) ? ph : nullptr;
       int nblk = 0;
@@ -738,7 +783,7 @@ struct sdns_batch {
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
   char* dmem = nullptr;
   // device arrays inside dmem
-  void* d_p1[2] = {nullptr, nullptr};  // P1 args: stage 0 reads u_hat, stages 1-3 the stage buffer
+  void* d_p1[4] = {nullptr, nullptr, nullptr, nullptr};  // P1 args of RK stages 0..3
   void *d_p2 = nullptr, *d_p3 = nullptr, *d_p4 = nullptr;
   void* d_p5[4] = {nullptr, nullptr, nullptr, nullptr};  // P5 args of RK stages 0..3
   int* d_len[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -825,17 +870,17 @@ template <typename Rt> int batch_layout(sdns_batch* b) {
   b->pcnt = nt[4];
   int part_total = 0;
   for (int i = 0; i < nb; ++i) { b->poff[i] = part_total; part_total += 2 * nt[4][i]; }
-  // one allocation: 9 argument arrays, lengths, work lists, partials, diag, nu, offsets
+  // one allocation: 11 argument arrays, lengths, work lists, partials, diag, nu, offsets
   size_t argsz = std::max(std::max(sizeof(P1Args<Rt>), sizeof(P2Args<Rt>)),
                           std::max(std::max(sizeof(P3Args<Rt>), sizeof(StridedArgs<Rt>)), sizeof(P5Args<Rt>)));
   b->args_bytes = align256(argsz * nb);
-  const size_t bytes = 9 * b->args_bytes + align256(5 * nb * sizeof(int)) + align256(nitems * sizeof(BatchWork)) +
+  const size_t bytes = 11 * b->args_bytes + align256(5 * nb * sizeof(int)) + align256(nitems * sizeof(BatchWork)) +
                        align256(part_total * sizeof(double)) + 2 * align256(2 * nb * sizeof(double)) +
                        2 * align256(nb * sizeof(int));
   if (hipMalloc((void**)&b->dmem, bytes) != hipSuccess) return fail(SDNS_ERR_NOMEM, "hipMalloc of %zu bytes failed", bytes);
   char* c = b->dmem;
-  void** slots[9] = {&b->d_p1[0], &b->d_p1[1], &b->d_p2, &b->d_p3, &b->d_p4,
-                     &b->d_p5[0], &b->d_p5[1], &b->d_p5[2], &b->d_p5[3]};
+  void** slots[11] = {&b->d_p1[0], &b->d_p1[1], &b->d_p1[2], &b->d_p1[3], &b->d_p2, &b->d_p3, &b->d_p4,
+                      &b->d_p5[0], &b->d_p5[1], &b->d_p5[2], &b->d_p5[3]};
   for (auto sl : slots) { *sl = c; c += b->args_bytes; }
   int* lens = (int*)c;
   c += align256(5 * nb * sizeof(int));
@@ -866,17 +911,19 @@ template <typename Rt> int batch_layout(sdns_batch* b) {
 // Per-box argument arrays for the current state pointers, nu and dt.
 template <typename Rt> int batch_upload(sdns_batch* b) {
   const int nb = b->nbox;
-  const Rt a[4] = {Rt(1. / 6.), Rt(1. / 3.), Rt(1. / 3.), Rt(1. / 6.)};
-  const Rt bb[3] = {Rt(0.5), Rt(0.5), Rt(1.)};
-  std::vector<P1Args<Rt>> h1[2];
+  std::vector<P1Args<Rt>> h1[4];
   std::vector<P2Args<Rt>> h2;
   std::vector<P3Args<Rt>> h3;
   std::vector<StridedArgs<Rt>> h4;
   std::vector<P5Args<Rt>> h5[4];
   for (int i = 0; i < nb; ++i) {
     const sdns_plan* p = b->box[i];
-    h1[0].push_back(p1_args<Rt>(p, b->u[i]));
-    h1[1].push_back(p1_args<Rt>(p, p->stB));
+    const Rt dt = (Rt)b->dt[i];
+    const int keep = rk_keep<Rt>(p->M[0] != p->N[0], false);
+    for (int rk = 0; rk < 4; ++rk) {
+      h1[rk].push_back(p1_args<Rt>(p, b->u[i]));
+      RkStage<Rt>::p1(h1[rk].back(), keep, rk, dt, b->u[i], p->st);
+    }
     h2.push_back(p2_args<Rt>(p));
     h3.push_back(p3_args<Rt>(p));
     h4.push_back(p4_args<Rt>(p));
@@ -886,12 +933,9 @@ template <typename Rt> int batch_upload(sdns_batch* b) {
       q.stream_in = tiles_whole_lines<Rt>(q.in, T, q.cdiv, q.in_hi, q.in_row, q.in_field);
       q.stream_out = tiles_whole_lines<Rt>(q.out, T, q.cdiv, q.out_hi, q.out_row, q.out_field);
     }
-    const Rt dt = (Rt)b->dt[i];
-    for (int rk = 0; rk < 4; ++rk) {  // stages 1 and 2 share a but not b
+    for (int rk = 0; rk < 4; ++rk) {
       P5Args<Rt> pa = p5_args<Rt>(p, b->nu[i]);
-      pa.A = b->u[i]; pa.B = p->stB; pa.Cacc = p->stC;
-      pa.adt = a[rk] * dt;
-      pa.bdt = rk < 3 ? bb[rk] * dt : Rt(0);
+      RkStage<Rt>::p5(pa, keep, rk, dt, b->u[i], p->st);
       pa.partials = rk == 3 ? b->d_part + b->poff[i] : nullptr;
       h5[rk].push_back(pa);
     }
@@ -899,8 +943,8 @@ template <typename Rt> int batch_upload(sdns_batch* b) {
   // copies on the batch stream, which is then drained: the host vectors stay
   // alive until the data are on the device and no replay can see a partial update
   hipStream_t s = b->own;
-  HIP_TRY(hipMemcpyAsync(b->d_p1[0], h1[0].data(), nb * sizeof(P1Args<Rt>), hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(b->d_p1[1], h1[1].data(), nb * sizeof(P1Args<Rt>), hipMemcpyHostToDevice, s));
+  for (int rk = 0; rk < 4; ++rk)
+    HIP_TRY(hipMemcpyAsync(b->d_p1[rk], h1[rk].data(), nb * sizeof(P1Args<Rt>), hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(b->d_p2, h2.data(), nb * sizeof(P2Args<Rt>), hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(b->d_p3, h3.data(), nb * sizeof(P3Args<Rt>), hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(b->d_p4, h4.data(), nb * sizeof(StridedArgs<Rt>), hipMemcpyHostToDevice, s));
@@ -914,12 +958,12 @@ template <typename Rt> int batch_upload(sdns_batch* b) {
 // One RK4 step of every box on stream s.
 template <typename Rt> int batch_step(sdns_batch* b, hipStream_t s) {
   for (int rk = 0; rk < 4; ++rk) {
-    launch_batch_p1<Rt>(b->lmax[0], (const P1Args<Rt>*)b->d_p1[rk == 0 ? 0 : 1], b->d_len[0], b->d_work[0],
+    launch_batch_p1<Rt>(b->lmax[0], (const P1Args<Rt>*)b->d_p1[rk], b->d_len[0], b->d_work[0],
                         b->nwork[0], s);
     launch_batch_p2<Rt>(b->lmax[1], (const P2Args<Rt>*)b->d_p2, b->d_len[1], b->d_work[1], b->nwork[1], s);
     launch_batch_p3<Rt>(b->lmax[2], (const P3Args<Rt>*)b->d_p3, b->d_len[2], b->d_work[2], b->nwork[2], s);
     launch_batch_fwd<Rt>(b->lmax[3], (const StridedArgs<Rt>*)b->d_p4, b->d_len[3], b->d_work[3], b->nwork[3], 3, s);
-    const int mode = rk == 0 ? P5_RK0 : (rk < 3 ? P5_RK12 : P5_RK3);
+    const int mode = RkStage<Rt>::mode(rk);
     launch_batch_p5<Rt>(b->lmax[4], mode, (const P5Args<Rt>*)b->d_p5[rk], b->d_len[4], b->d_work[4], b->nwork[4], s);
   }
   hipLaunchKernelGGL(k_batch_sum, dim3(b->nbox), dim3(256), 0, s, (const double*)b->d_part, (const int*)b->d_poff,
@@ -1519,6 +1563,7 @@ int sdns_closure_create(sdns_closure** out, const int32_t N[3], void* hip_stream
   c->y = (float*)(m + o_y); c->gy = (float*)(m + o_gy); c->t = (float*)(m + o_t);
   c->wpart = (float*)(m + o_wp); c->bpart = (float*)(m + o_bp); c->phys = (float*)(m + o_ph);
   c->tauphys = (float*)(m + o_tp); c->tauhat = m + o_th; c->src = m + o_src;
+  c->stage = c->tauhat;  // read by the transform before tau's is written
   c->lpart = (double*)(m + o_lp); c->loss = (double*)(m + o_l);
   c->w.w1f = (__bf16*)(m + o_w1); c->w.w2f = (__bf16*)(m + o_w2); c->w.w3f = (__bf16*)(m + o_w3);
   c->w.w3b = (__bf16*)(m + o_w3b); c->w.w2b = (__bf16*)(m + o_w2b);

@@ -26,6 +26,23 @@ namespace sdns {
     break;
 #define SDNS_BATCH_CASE(m, ...) SDNS_BATCH_CASE_V(m, 0, __VA_ARGS__) SDNS_BATCH_CASE_V(m, 1, __VA_ARGS__)
 
+template <typename Rt, int M, int E, int T>
+__device__ __forceinline__ void batch_p1(const P1Args<Rt>& a, int tile, int yb, cx<Rt>* lds, const cx<Rt>* tw) {
+  if constexpr (rk_keep<Rt>(false, false) == KEEP_RHS) {
+    if (a.d) return p1_body<Rt, M, E, T, true>(a, tile, yb, lds, tw);
+  }
+  p1_body<Rt, M, E, T, false>(a, tile, yb, lds, tw);
+}
+// (a batched box's arrays are within a buffer descriptor's reach: its sides
+// are at most 128)
+template <typename Rt, int M, int E, int MODE, int T>
+__device__ __forceinline__ void batch_p5(const P5Args<Rt>& a, int tile, cx<Rt>* lds, const cx<Rt>* tw) {
+  if constexpr (M % 3 == 0 && E % 3 == 0) {
+    if (a.N0 != M) return p5b_body<Rt, M, E, MODE, true, false, T>(a, tile, lds, tw);
+  }
+  p5b_body<Rt, M, E, MODE, false, false, T>(a, tile, lds, tw);
+}
+
 template <typename Rt, int LMAX>
 __global__ void __launch_bounds__(batch_threads<Rt>())
     k_batch_p1(const P1Args<Rt>* __restrict__ args, const int* __restrict__ len, const BatchWork* __restrict__ work) {
@@ -35,7 +52,7 @@ __global__ void __launch_bounds__(batch_threads<Rt>())
   if (w.box < 0) return;
   const P1Args<Rt> a = args[w.box];
   switch (len[w.box]) {
-#define SDNS_X(m) SDNS_BATCH_CASE(m, p1_body<Rt, m, E, T>(a, w.tile, blockIdx.y, smem, tw))
+#define SDNS_X(m) SDNS_BATCH_CASE(m, batch_p1<Rt, m, E, T>(a, w.tile, blockIdx.y, smem, tw))
     SDNS_BATCH_STRIDED(SDNS_X)
 #undef SDNS_X
     default: break;
@@ -84,7 +101,7 @@ __global__ void __launch_bounds__(batch_threads<Rt>())
   if (w.box < 0) return;
   const P5Args<Rt> a = args[w.box];
   switch (len[w.box]) {
-#define SDNS_X(m) SDNS_BATCH_CASE(m, p5_body<Rt, m, E, MODE, false, T>(a, w.tile, smem, tw))
+#define SDNS_X(m) SDNS_BATCH_CASE(m, batch_p5<Rt, m, E, MODE, T>(a, w.tile, smem, tw))
     SDNS_BATCH_STRIDED(SDNS_X)
 #undef SDNS_X
     default: break;

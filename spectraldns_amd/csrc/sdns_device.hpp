@@ -69,6 +69,10 @@ template <typename C> __device__ __forceinline__ C cmul(C a, C b) {
 template <typename C> __device__ __forceinline__ C cmulc(C a, C b) {
   return mk<C>(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
 }
+// a + s b
+template <typename C> __device__ __forceinline__ C caxpy(C a, decltype(C::x) s, C b) {
+  return mk<C>(a.x + s * b.x, a.y + s * b.y);
+}
 template <typename C> __device__ __forceinline__ C cconj(C a) { return mk<C>(a.x, -a.y); }
 template <typename C> __device__ __forceinline__ C cscale(C a, decltype(C::x) s) { return mk<C>(a.x * s, a.y * s); }
 // multiply by +i (S=+1) or -i (S=-1)

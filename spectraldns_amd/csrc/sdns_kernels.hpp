@@ -104,7 +104,8 @@ __device__ __forceinline__ void table_to_lds(C* dst, const C* __restrict__ src, 
 // y = 1 -> v (fields 1 and 4 = X(kx v)), y = 2 -> u (field 0).  With a given
 // vorticity (a.w) there are six blocks rows y = 0..5, each the plain
 // x-inverse of one field: u, v, w from a.u, then wx, wy, wz from a.w.
-template <typename Rt, int M, int E, int T>
+// INC: the state is u + ds d, formed on reading (the RK stages of KEEP_RHS).
+template <typename Rt, int M, int E, int T, bool INC>
 __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, cx<Rt>* lds, const cx<Rt>* tw) {
   using C = cx<Rt>;
   constexpr int P = M / E;
@@ -121,10 +122,23 @@ __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, c
   const C* __restrict__ U = (const C*)(given && yb >= 3 ? a.w : a.u) + (long)comp * a.N0 * plane +
                             (valid ? (long)iy * a.Nh + kzi : 0);
   C v[E];
+  if constexpr (INC) {
+    const C* __restrict__ D = (const C*)a.d + (U - (const C*)a.u);
+    C d[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int r = bin_row(t + P * e, M, a.x);
-    v[e] = (valid && r >= 0) ? U[r * plane] : czero<C>();
+    for (int e = 0; e < E; ++e) {
+      const int r = bin_row(t + P * e, M, a.x);
+      v[e] = (valid && r >= 0) ? U[r * plane] : czero<C>();
+      d[e] = (valid && r >= 0) ? D[r * plane] : czero<C>();
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = caxpy(v[e], a.ds, d[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int r = bin_row(t + P * e, M, a.x);
+      v[e] = (valid && r >= 0) ? U[r * plane] : czero<C>();
+    }
   }
   __syncthreads();
   C* __restrict__ out = (C*)a.w1 + q;
@@ -165,7 +179,7 @@ template <typename Rt, int M, int E> constexpr int p1_occ() {
   return sizeof(Rt) == 4 && o < 3 && 163840 / lds >= 3 && 3 * SCfg<Rt, M, E>::THREADS <= 4 * 64 * 3 ? 3 : o;
 }
 // D: the launcher's tile divisor for small grids (T / D columns per block).
-template <typename Rt, int M, int E, int D = 1>
+template <typename Rt, int M, int E, int D = 1, bool INC = false>
 __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p1_occ<Rt, M, E>())) k_p1(P1Args<Rt> a) {
   using C = cx<Rt>;
   constexpr int T = SCfg<Rt, M, E>::T / D;
@@ -174,7 +188,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p1_occ<Rt, M, 
   const int tile = xcd_tile((a.Q + T - 1) / T);
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
-  p1_body<Rt, M, E, T>(a, tile, blockIdx.y, lds, tw);
+  p1_body<Rt, M, E, T, INC>(a, tile, blockIdx.y, lds, tw);
 }
 
 // ------------------------------------------------------------------ P2
@@ -871,10 +885,61 @@ template <int TH> __device__ __forceinline__ void p5_partials(double esum, doubl
   }
 }
 
-// COMP: compensated accumulation of the RK4 sum u2 = u1 + sum a dt rhs in a
-// (hi, lo) pair of single-precision fields; the state is u = hi + lo with hi
-// the caller's u_hat and lo the caller's u_lo.  Stage values stay plain.
-template <typename Rt, int M, int E, int MODE, bool COMP, int T>
+// The new state of the last RK4 stage from u, the kept stage arrays x1, x2, x3
+// and the stage's right-hand side r (see P5Args).  COMP: the state is the pair
+// u + lo, summed term by term with TwoSum and renormalised (hi = fl(h + l), lo
+// the exact remainder).
+template <int KEEP, bool COMP, typename Rt>
+__device__ __forceinline__ cx<Rt> rk_last(const P5Args<Rt>& a, cx<Rt> u, cx<Rt> x1, cx<Rt> x2, cx<Rt> x3, cx<Rt> r,
+                                          cx<Rt>& lo) {
+  using C = cx<Rt>;
+  if constexpr (KEEP == KEEP_SUM) {
+    return caxpy(x1, a.adt, r);
+  } else if constexpr (KEEP == KEEP_STATES) {
+    constexpr Rt third = Rt(1) / Rt(3);
+    const C d = mk<C>(third * (((x1.x - u.x) + (x3.x - u.x)) + Rt(2) * (x2.x - u.x)),
+                      third * (((x1.y - u.y) + (x3.y - u.y)) + Rt(2) * (x2.y - u.y)));
+    return cadd(u, caxpy(d, a.adt, r));
+  } else if constexpr (!COMP) {
+    return caxpy(caxpy(caxpy(caxpy(u, a.adt, x1), a.a12, x2), a.a12, x3), a.adt, r);
+  } else {
+    const C k[4] = {x1, x2, x3, r};
+    C h = u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const Rt w = i == 0 || i == 3 ? a.adt : a.a12;
+      const Rt yx = w * k[i].x, yy = w * k[i].y;
+      Rt ex, ey;
+      h = mk<C>(two_sum(h.x, yx, ex), two_sum(h.y, yy, ey));
+      lo = mk<C>(lo.x + ex, lo.y + ey);
+    }
+    C rest;
+    h = mk<C>(two_sum(h.x, lo.x, rest.x), two_sum(h.y, lo.y, rest.y));
+    lo = rest;
+    return h;
+  }
+}
+
+// State arrays read per element by a stage, and elements per chunk of the
+// update loop: all loads of a chunk are issued before any of its stores, so
+// that a chunk's state is in flight at once instead of one round trip per
+// array and element.  The chunk holds about six complex triples at most and
+// shrinks where the line itself fills the registers.  Stage 0 reads u; stages
+// 1 and 2 read u and s, with KEEP_SUM also b1; stage 3 reads u, s, b1, b2 and,
+// compensated, lo, with KEEP_SUM s and b1 (u is only written).
+constexpr int p5_arrays(int mode, bool comp, int keep) {
+  if (mode == P5_RK12) return keep == KEEP_SUM ? 3 : 2;
+  if (mode == P5_RK3) return keep == KEEP_SUM ? 2 : (comp ? 5 : 4);
+  return 1;
+}
+constexpr int p5_chunk(int mode, bool comp, int keep, int E, int threads) {
+  if (E >= 24 || threads >= 1024 || mode == P5_RHS) return 1;
+  return p5_arrays(mode, comp, keep) > 2 ? 1 : 2;
+}
+
+// COMP: the state is the pair u = hi + lo (hi the caller's u_hat, lo the
+// caller's u_lo), which only the last stage reads.
+template <typename Rt, int M, int E, int MODE, bool COMP, int T, int KEEP>
 __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* lds, const cx<Rt>* tw) {
   using C = cx<Rt>;
   constexpr bool STREAM = T * (int)sizeof(C) >= 128;  // tiles of whole 128-byte lines
@@ -909,25 +974,27 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
   const Rt K1 = a.ky[iy], K2c = a.kz[kz];
   const bool nyq_col = a.mask_nyquist && (iy == a.N1 / 2 || kz == a.N2 / 2);
   double esum = 0.0, osum = 0.0;
-  // Elements go in chunks of G: all loads of a chunk are issued before any of
-  // its stores, so G elements' state is in flight at once instead of one
-  // round trip per array and element.  An element's rows are written only by
+  // Chunks of G elements (see p5_chunk); an element's rows are written only by
   // that element, so no load of a chunk can see a store of the same chunk.
-  constexpr int G = (E >= 24 || TH >= 1024 || MODE == P5_RHS) ? 1 : 2;
+  constexpr int G = p5_chunk(MODE, COMP, KEEP, E, TH);
   static_assert(E % G == 0, "chunk must divide the points per thread");
-  const C* ust = (const C*)(MODE == P5_RK0 || MODE == P5_RHS ? a.A : a.B);
   const C* src = (const C*)a.source;
-  const C* Ain = (const C*)a.A;
-  const C* Cin = (const C*)a.Cacc;
-  const C* Lin = (const C*)(MODE == P5_RK0 ? a.Alo : a.Clo);
-  constexpr bool LOAD_A = MODE == P5_RK12;
-  constexpr bool LOAD_C = MODE == P5_RK12 || MODE == P5_RK3;
-  constexpr bool LOAD_L = COMP && MODE != P5_RHS;
+  const C* Uin = (const C*)a.u;
+  const C* Sin = (const C*)a.s;
+  const C* B1in = (const C*)a.b1;
+  const C* B2in = (const C*)a.b2;
+  const C* Lin = (const C*)a.lo;
+  constexpr bool SUM = KEEP == KEEP_SUM;
+  constexpr bool LOAD_U = !(SUM && MODE == P5_RK3);
+  constexpr bool LOAD_S = MODE == P5_RK12 || MODE == P5_RK3;
+  constexpr bool LOAD_B1 = MODE == P5_RK3 || (SUM && MODE == P5_RK12);
+  constexpr bool LOAD_B2 = MODE == P5_RK3 && !SUM;
+  constexpr bool LOAD_L = COMP && MODE == P5_RK3;
 #pragma unroll
   for (int e0 = 0; e0 < E; e0 += G) {
     int ixs[G];
     bool keeps[G];
-    C su[G][3], sr[G][3], xa[G][3], xc[G][3], xl[G][3];
+    C su[G][3], sr[G][3], ss[G][3], x1[G][3], x2[G][3], xl[G][3];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       const int p = t + P * (e0 + g);
@@ -950,10 +1017,11 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
       const long off = (long)ix * plane + q;
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        su[g][i] = ust[i * fs + off];
+        if constexpr (LOAD_U) su[g][i] = Uin[i * fs + off];
         if (src) sr[g][i] = src[i * fs + off];
-        if constexpr (LOAD_A) xa[g][i] = Ain[i * fs + off];
-        if constexpr (LOAD_C) xc[g][i] = Cin[i * fs + off];
+        if constexpr (LOAD_S) ss[g][i] = Sin[i * fs + off];
+        if constexpr (LOAD_B1) x1[g][i] = B1in[i * fs + off];
+        if constexpr (LOAD_B2) x2[g][i] = B2in[i * fs + off];
         if constexpr (LOAD_L) xl[g][i] = Lin[i * fs + off];
       }
     }
@@ -975,9 +1043,8 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
         }
       }
       const bool conv = colconv && kept && !(nyq_col || (a.mask_nyquist && ix == a.N0 / 2));
-      C r0 = conv ? cscale(X0[e], a.scale) : czero<C>();
-      C r1 = conv ? cscale(X1[e], a.scale) : czero<C>();
-      C r2 = conv ? cscale(X2[e], a.scale) : czero<C>();
+      C r[3] = {conv ? cscale(X0[e], a.scale) : czero<C>(), conv ? cscale(X1[e], a.scale) : czero<C>(),
+                conv ? cscale(X2[e], a.scale) : czero<C>()};
       const Rt K0 = a.kx[ix];
       Rt k2 = K0 * K0;
       k2 += K1 * K1;
@@ -985,98 +1052,48 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
       const Rt den = k2 == Rt(0) ? Rt(1) : k2;
       const Rt o0 = K0 / den, o1 = K1 / den, o2 = K2c / den;
       // P_hat = sum_i rhs_i K_i/K^2 ; rhs_i -= P_hat K_i ; rhs -= (nu K^2) u_hat  (NS.py:208-215)
-      C ph = mk<C>(r0.x * o0 + r1.x * o1, r0.y * o0 + r1.y * o1);
-      ph = mk<C>(ph.x + r2.x * o2, ph.y + r2.y * o2);
-      r0 = mk<C>(r0.x - ph.x * K0, r0.y - ph.y * K0);
-      r1 = mk<C>(r1.x - ph.x * K1, r1.y - ph.y * K1);
-      r2 = mk<C>(r2.x - ph.x * K2c, r2.y - ph.y * K2c);
+      C ph = mk<C>(r[0].x * o0 + r[1].x * o1, r[0].y * o0 + r[1].y * o1);
+      ph = mk<C>(ph.x + r[2].x * o2, ph.y + r[2].y * o2);
+      const Rt Kv[3] = {K0, K1, K2c};
       const Rt z = a.nu * k2;
-      const C s0 = su[g][0], s1 = su[g][1], s2 = su[g][2];
-      r0 = mk<C>(r0.x - z * s0.x, r0.y - z * s0.y);
-      r1 = mk<C>(r1.x - z * s1.x, r1.y - z * s1.y);
-      r2 = mk<C>(r2.x - z * s2.x, r2.y - z * s2.y);
-      if (src) {  // rhs += Source (NS.py:256-258), every mode
-        r0 = cadd(r0, sr[g][0]); r1 = cadd(r1, sr[g][1]); r2 = cadd(r2, sr[g][2]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        r[i] = mk<C>(r[i].x - ph.x * Kv[i], r[i].y - ph.y * Kv[i]);
+        const C st = !LOAD_S ? su[g][i] : (KEEP == KEEP_RHS ? caxpy(su[g][i], a.sdt, ss[g][i]) : ss[g][i]);
+        r[i] = mk<C>(r[i].x - z * st.x, r[i].y - z * st.y);
+        if (src) r[i] = cadd(r[i], sr[g][i]);  // rhs += Source (NS.py:256-258), every mode
       }
       if constexpr (MODE == P5_RHS) {
         C* rhs = (C*)a.rhs;
-        st_pass<STREAM>(rhs + off, r0); st_pass<STREAM>(rhs + fs + off, r1); st_pass<STREAM>(rhs + 2 * fs + off, r2);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) st_pass<STREAM>(rhs + (i * fs + off), r[i]);
         if (a.phat) ((C*)a.phat)[off] = ph;
+      } else if constexpr (MODE != P5_RK3) {
+        C* out = (C*)a.out;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          st_pass<STREAM>(out + (i * fs + off), KEEP == KEEP_RHS ? r[i] : caxpy(su[g][i], a.bdt, r[i]));
+          if constexpr (SUM) st_pass<STREAM>((C*)a.b1 + (i * fs + off), caxpy(MODE == P5_RK0 ? su[g][i] : x1[g][i], a.adt, r[i]));
+        }
       } else {
-        C* A = (C*)a.A;
-        C* B = (C*)a.B;
-        C* Cc = (C*)a.Cacc;
-        const Rt bdt = a.bdt, adt = a.adt;
-        auto upd = [](C base, C r, Rt s) { return mk<C>(base.x + s * r.x, base.y + s * r.y); };
-        if constexpr (!COMP) {
-          if constexpr (MODE == P5_RK0) {
-            // u0 = u1 + b dt rhs ; u2 = u1 + a dt rhs  (u1 = u2 = u0 at stage 0)
-            st_pass<STREAM>(B + (off), upd(s0, r0, bdt)); st_pass<STREAM>(B + (fs + off), upd(s1, r1, bdt)); st_pass<STREAM>(B + (2 * fs + off), upd(s2, r2, bdt));
-            st_pass<STREAM>(Cc + (off), upd(s0, r0, adt)); st_pass<STREAM>(Cc + (fs + off), upd(s1, r1, adt)); st_pass<STREAM>(Cc + (2 * fs + off), upd(s2, r2, adt));
-          } else if constexpr (MODE == P5_RK12) {
-            st_pass<STREAM>(B + (off), upd(xa[g][0], r0, bdt)); st_pass<STREAM>(B + (fs + off), upd(xa[g][1], r1, bdt)); st_pass<STREAM>(B + (2 * fs + off), upd(xa[g][2], r2, bdt));
-            st_pass<STREAM>(Cc + (off), upd(xc[g][0], r0, adt)); st_pass<STREAM>(Cc + (fs + off), upd(xc[g][1], r1, adt));
-            st_pass<STREAM>(Cc + (2 * fs + off), upd(xc[g][2], r2, adt));
-          } else {
-            const C n0 = upd(xc[g][0], r0, adt), n1 = upd(xc[g][1], r1, adt), n2 = upd(xc[g][2], r2, adt);
-            st_pass<STREAM>(A + (off), n0); st_pass<STREAM>(A + (fs + off), n1); st_pass<STREAM>(A + (2 * fs + off), n2);
-            if (a.phat) ((C*)a.phat)[off] = ph;
-            if (a.partials) {
-              const double w = (kz == 0 || kz == a.N2 / 2) ? 1.0 : 2.0;
-              const double v[6] = {n0.x, n0.y, n1.x, n1.y, n2.x, n2.y};
-              energy_terms(v, K0, K1, K2c, w, esum, osum);
-            }
-          }
-        } else {
-          C* Alo = (C*)a.Alo;
-          C* Clo = (C*)a.Clo;
-          const C rr[3] = {r0, r1, r2};
-          if constexpr (MODE == P5_RK0) {
-            const C ss[3] = {s0, s1, s2};
+        C* un = (C*)a.u;
+        double v[6];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              const long o = i * fs + off;
-              st_pass<STREAM>(B + (o), upd(ss[i], rr[i], bdt));
-              const Rt yx = adt * rr[i].x, yy = adt * rr[i].y;
-              Rt ex, ey;
-              const Rt hx = two_sum(ss[i].x, yx, ex), hy = two_sum(ss[i].y, yy, ey);
-              const C l = xl[g][i];
-              st_pass<STREAM>(Cc + (o), mk<C>(hx, hy));
-              Clo[o] = mk<C>(l.x + ex, l.y + ey);
-            }
-          } else if constexpr (MODE == P5_RK12) {
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              const long o = i * fs + off;
-              st_pass<STREAM>(B + (o), upd(xa[g][i], rr[i], bdt));
-              const C c = xc[g][i], l = xl[g][i];
-              const Rt yx = adt * rr[i].x, yy = adt * rr[i].y;
-              Rt ex, ey;
-              const Rt hx = two_sum(c.x, yx, ex), hy = two_sum(c.y, yy, ey);
-              st_pass<STREAM>(Cc + (o), mk<C>(hx, hy));
-              Clo[o] = mk<C>(l.x + ex, l.y + ey);
-            }
-          } else {
-            double v[6];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-              const long o = i * fs + off;
-              const C c = xc[g][i], l = xl[g][i];
-              const Rt yx = adt * rr[i].x, yy = adt * rr[i].y;
-              Rt ex, ey;
-              const Rt hx = two_sum(c.x, yx, ex), hy = two_sum(c.y, yy, ey);
-              const Rt lx = l.x + ex, ly = l.y + ey;
-              Rt rx, ry;  // renormalise: hi = fl(h + l), lo = exact remainder
-              const Rt nx = two_sum(hx, lx, rx), ny = two_sum(hy, ly, ry);
-              st_pass<STREAM>(A + (o), mk<C>(nx, ny));
-              Alo[o] = mk<C>(rx, ry);
-              v[2 * i] = (double)nx + (double)rx;
-              v[2 * i + 1] = (double)ny + (double)ry;
-            }
-            if (a.phat) ((C*)a.phat)[off] = ph;
-            if (a.partials) energy_terms(v, K0, K1, K2c, (kz == 0 || kz == a.N2 / 2) ? 1.0 : 2.0, esum, osum);
+        for (int i = 0; i < 3; ++i) {
+          const long o = i * fs + off;
+          C l = LOAD_L ? xl[g][i] : czero<C>();
+          const C n = rk_last<KEEP, COMP>(a, su[g][i], x1[g][i], x2[g][i], ss[g][i], r[i], l);
+          st_pass<STREAM>(un + o, n);
+          v[2 * i] = n.x;
+          v[2 * i + 1] = n.y;
+          if constexpr (COMP) {
+            ((C*)a.lo)[o] = l;
+            v[2 * i] += (double)l.x;
+            v[2 * i + 1] += (double)l.y;
           }
         }
+        if (a.phat) ((C*)a.phat)[off] = ph;
+        if (a.partials) energy_terms(v, K0, K1, K2c, (kz == 0 || kz == a.N2 / 2) ? 1.0 : 2.0, esum, osum);
       }
     }
   }
@@ -1085,33 +1102,36 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
   }
 }
 
-// P5 stages under the 3/2 rule (M = 3 N0 / 2 bins, kept output modes
-// -N0/2..N0/2-1).  The kept bins are p < M/3 (row p) and p >= 2M/3 (row
-// p - M/3); with p = t + P e that is e < E/3 and e >= 2E/3 on every lane, and
-// kept element j (e = j, or j + E/3 past the first third) lands in row
-// t + P j.  Known at compile time, these leave the update loop without
-// branches, and it is software-pipelined: the state rows of the next chunk of
-// G elements are loaded before the current chunk is computed and stored (an
-// element's rows are written only by that element, so in program order every
-// load precedes the stores it could meet).  Every access is a buffer access:
-// one descriptor per array, the lane's byte offset (the same for every
-// element) and a uniform offset of component and element in a scalar
-// register, so no access needs a 64-bit address of its own.  W4 entries of
-// columns that carry no kept mode get an offset past the descriptor and read
-// as zero.  Plain RK stages with no source and no pressure output; the
-// per-mode arithmetic is p5_body's.  The host checks that the three
-// components of a state array and of W4 span at most BUF_OOB bytes
-// (p5k_fits).
-template <typename Rt, int M, int E, int MODE, int T>
-__device__ __forceinline__ void p5k_body(const P5Args<Rt>& a, int tile, cx<Rt>* lds, const cx<Rt>* tw) {
+// P5 with every access through a buffer descriptor: one per array, the lane's
+// byte offset (the same for every element) and a uniform offset of component
+// and element in a scalar register, so no access needs a 64-bit address of
+// its own (p5_body keeps E of them per array and spills).  That needs the
+// state row of an element to be t + P j:
+//   PAD = false: no padding along x (M = N0), element j is row t + P j;
+//   PAD = true: 3/2 rule (M = 3 N0 / 2, kept output modes -N0/2..N0/2-1).  The
+//     kept bins are p < M/3 (row p) and p >= 2M/3 (row p - M/3); with p = t + P e
+//     that is e < E/3 and e >= 2E/3 on every lane, and kept element j (e = j,
+//     or j + E/3 past the first third) lands in row t + P j.
+// The update loop then has no branches and is software-pipelined: the state
+// rows of the next chunk of G elements are loaded before the current chunk is
+// computed and stored (an element's rows are written only by that element, so
+// in program order every load precedes the stores it could meet).  W4 entries
+// of columns that carry no kept mode get an offset past the descriptor and
+// read as zero; a null source or pressure array has an empty descriptor, so
+// its loads return zeros and its stores are dropped without memory traffic.
+// The host checks that the three components of a state array and of W4 span
+// at most BUF_OOB bytes (p5b_fits); larger boxes run p5_body.  The per-mode
+// arithmetic is p5_body's.
+template <typename Rt, int M, int E, int MODE, bool PAD, bool COMP, int T>
+__device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* lds, const cx<Rt>* tw) {
   using C = cx<Rt>;
-  static_assert(M % 3 == 0 && E % 3 == 0 && MODE != P5_RHS, "3/2-rule RK stages");
-  constexpr int P = M / E, TH = T * P, E3 = E / 3, NK = 2 * E3;
+  static_assert(!PAD || (M % 3 == 0 && E % 3 == 0), "3/2-rule rows");
+  constexpr int P = M / E, TH = T * P, E3 = E / 3, NK = PAD ? 2 * E3 : E;
   constexpr int CS = (int)sizeof(C);
-  // state arrays read per element: RK0 u1; RK1-2 u0, u1, u2; RK3 u0, u2
-  constexpr int NL = MODE == P5_RK12 ? 3 : (MODE == P5_RK3 ? 2 : 1);
-  constexpr int G = MODE == P5_RK12 ? 1 : 2;  // spill-free at E = 24 (256 VGPRs)
-  static_assert(NK % G == 0, "chunk must divide the kept elements");
+  constexpr int KEEP = rk_keep<Rt>(PAD, COMP);
+  constexpr bool SUM = KEEP == KEEP_SUM;
+  constexpr int NL = p5_arrays(MODE, COMP, KEEP);  // u; s; b1; b2; lo (KEEP_SUM, stage 3: s, b1)
+  constexpr int G = (NL > 2 || E * CS >= 128 || NK % 2) ? 1 : 2;
   using F = LineFFT<Rt, M, E, -1>;
   const int c = threadIdx.x % T, t = threadIdx.x / T;
   const int q = tile * T + c;
@@ -1139,33 +1159,58 @@ __device__ __forceinline__ void p5k_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
   F::run(X2, t, line, T, tw);
 
   const int plane = a.N1 * a.Nh, fs = a.N0 * plane;
+  const long span = 3L * fs * CS;
+  const int so = (t * plane + q) * CS;  // row t of the column
+  // rows whose convection term is kept (every row with PAD)
+  auto kept = [&](int ix) { return PAD || ix <= a.x.pos || ix >= a.N0 - a.x.neg; };
+  if constexpr (MODE == P5_RHS) {
+    if (a.conv_only) {
+      const auto ro = buf_rsrc(a.rhs, span);
+      if (valid) {
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+          const int e = (!PAD || j < E3) ? j : j + E3;
+          const int eo = P * j * plane;
+          const Rt sc = kept(t + P * j) ? a.scale : Rt(0);
+          buf_store_so_nt<C>(cscale(X0[e], sc), ro, so, eo * CS);
+          buf_store_so_nt<C>(cscale(X1[e], sc), ro, so, (fs + eo) * CS);
+          buf_store_so_nt<C>(cscale(X2[e], sc), ro, so, (2 * fs + eo) * CS);
+        }
+      }
+      return;
+    }
+  }
   const Rt K1 = a.ky[iy], K2c = a.kz[kz];
+  const Rt Kyz[2] = {K1, K2c};
   const bool colok = colconv && !(a.mask_nyquist && (iy == a.N1 / 2 || kz == a.N2 / 2));
   const int nyq_ix = a.mask_nyquist ? a.N0 / 2 : -1;
   const double wz = (kz == 0 || kz == a.N2 / 2) ? 1.0 : 2.0;
   double esum = 0.0, osum = 0.0;
-  const long span = 3L * fs * CS;
-  const auto r0p = buf_rsrc(MODE == P5_RK0 ? a.A : a.B, span);
-  const auto r1p = buf_rsrc(MODE == P5_RK12 ? a.A : a.Cacc, span);
-  const auto r2p = buf_rsrc(a.Cacc, span);
-  const auto rA = buf_rsrc(a.A, span);
-  const auto rB = buf_rsrc(a.B, span);
-  const auto rC = buf_rsrc(a.Cacc, span);
-  const Rt bdt = a.bdt, adt = a.adt;
-  const int so = (t * plane + q) * CS;  // row t of the column
+  const auto ru = buf_rsrc(SUM && MODE == P5_RK3 ? a.s : a.u, span);
+  const auto rs = buf_rsrc(SUM && MODE == P5_RK3 ? a.b1 : a.s, span);
+  const auto rb1 = buf_rsrc(a.b1, span);
+  const auto rb2 = buf_rsrc(a.b2, span);
+  const auto rlo = buf_rsrc(a.lo, span);
+  const auto rsrc = buf_rsrc(a.source, a.source ? span : 0L);
+  const auto rph = buf_rsrc(a.phat, a.phat ? (long)fs * CS : 0L);
+  const auto ro = buf_rsrc(MODE == P5_RHS ? a.rhs : (MODE == P5_RK3 ? a.u : a.out), span);
   if (valid) {
-    C cur[G][NL][3], nxt[G][NL][3];
+    C cur[G][NL + 1][3], nxt[G][NL + 1][3];  // state arrays, then the source
     Rt kcur[G], knxt[G];
-    auto load = [&](C(&d)[G][NL][3], Rt(&kd)[G], int j0) {
+    auto load = [&](C(&d)[G][NL + 1][3], Rt(&kd)[G], int j0) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         const int eo = P * (j0 + g) * plane;
         kd[g] = a.kx[t + P * (j0 + g)];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-          d[g][0][i] = buf_load_so<C>(r0p, so, (i * fs + eo) * CS);
-          if constexpr (NL > 1) d[g][1][i] = buf_load_so<C>(r1p, so, (i * fs + eo) * CS);
-          if constexpr (NL > 2) d[g][2][i] = buf_load_so<C>(r2p, so, (i * fs + eo) * CS);
+          const int o = (i * fs + eo) * CS;
+          d[g][0][i] = buf_load_so<C>(ru, so, o);
+          if constexpr (NL > 1) d[g][1][i] = buf_load_so<C>(rs, so, o);
+          if constexpr (NL > 2) d[g][2][i] = buf_load_so<C>(rb1, so, o);
+          if constexpr (NL > 3) d[g][3][i] = buf_load_so<C>(rb2, so, o);
+          if constexpr (NL > 4) d[g][4][i] = buf_load_so<C>(rlo, so, o);
+          d[g][NL][i] = buf_load_so<C>(rsrc, so, o);
         }
       }
     };
@@ -1175,62 +1220,59 @@ __device__ __forceinline__ void p5k_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
       if (j0 + G < NK) load(nxt, knxt, j0 + G);
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const int j = j0 + g, e = j < E3 ? j : j + E3;
+        const int j = j0 + g, e = (!PAD || j < E3) ? j : j + E3;
         const int ix = t + P * j;
         const int eo = P * j * plane;
-        const bool conv = colok & (ix != nyq_ix);
-        C r0 = conv ? cscale(X0[e], a.scale) : czero<C>();
-        C r1 = conv ? cscale(X1[e], a.scale) : czero<C>();
-        C r2 = conv ? cscale(X2[e], a.scale) : czero<C>();
-        const Rt K0 = kcur[g];
-        Rt k2 = K0 * K0;
+        const bool conv = colok & (ix != nyq_ix) & kept(ix);
+        C r[3] = {conv ? cscale(X0[e], a.scale) : czero<C>(), conv ? cscale(X1[e], a.scale) : czero<C>(),
+                  conv ? cscale(X2[e], a.scale) : czero<C>()};
+        const Rt Kv[3] = {kcur[g], Kyz[0], Kyz[1]};
+        Rt k2 = Kv[0] * Kv[0];
         k2 += K1 * K1;
         k2 += K2c * K2c;
         const Rt den = k2 == Rt(0) ? Rt(1) : k2;
-        const Rt o0 = K0 / den, o1 = K1 / den, o2 = K2c / den;
+        const Rt o0 = Kv[0] / den, o1 = K1 / den, o2 = K2c / den;
         // P_hat = sum_i rhs_i K_i/K^2 ; rhs_i -= P_hat K_i ; rhs -= (nu K^2) u_hat  (NS.py:208-215)
-        C ph = mk<C>(r0.x * o0 + r1.x * o1, r0.y * o0 + r1.y * o1);
-        ph = mk<C>(ph.x + r2.x * o2, ph.y + r2.y * o2);
-        r0 = mk<C>(r0.x - ph.x * K0, r0.y - ph.y * K0);
-        r1 = mk<C>(r1.x - ph.x * K1, r1.y - ph.y * K1);
-        r2 = mk<C>(r2.x - ph.x * K2c, r2.y - ph.y * K2c);
+        C ph = mk<C>(r[0].x * o0 + r[1].x * o1, r[0].y * o0 + r[1].y * o1);
+        ph = mk<C>(ph.x + r[2].x * o2, ph.y + r[2].y * o2);
         const Rt z = a.nu * k2;
-        const C s0 = cur[g][0][0], s1 = cur[g][0][1], s2 = cur[g][0][2];
-        r0 = mk<C>(r0.x - z * s0.x, r0.y - z * s0.y);
-        r1 = mk<C>(r1.x - z * s1.x, r1.y - z * s1.y);
-        r2 = mk<C>(r2.x - z * s2.x, r2.y - z * s2.y);
-        auto upd = [](C base, C r, Rt s) { return mk<C>(base.x + s * r.x, base.y + s * r.y); };
-        const int o0s = eo * CS, o1s = (fs + eo) * CS, o2s = (2 * fs + eo) * CS;
-        if constexpr (MODE == P5_RK0) {
-          // u0 = u1 + b dt rhs ; u2 = u1 + a dt rhs  (u1 = u2 = u0 at stage 0)
-          buf_store_so_nt<C>(upd(s0, r0, bdt), rB, so, o0s);
-          buf_store_so_nt<C>(upd(s1, r1, bdt), rB, so, o1s);
-          buf_store_so_nt<C>(upd(s2, r2, bdt), rB, so, o2s);
-          buf_store_so_nt<C>(upd(s0, r0, adt), rC, so, o0s);
-          buf_store_so_nt<C>(upd(s1, r1, adt), rC, so, o1s);
-          buf_store_so_nt<C>(upd(s2, r2, adt), rC, so, o2s);
-        } else if constexpr (MODE == P5_RK12) {
-          buf_store_so_nt<C>(upd(cur[g][1][0], r0, bdt), rB, so, o0s);
-          buf_store_so_nt<C>(upd(cur[g][1][1], r1, bdt), rB, so, o1s);
-          buf_store_so_nt<C>(upd(cur[g][1][2], r2, bdt), rB, so, o2s);
-          buf_store_so_nt<C>(upd(cur[g][2][0], r0, adt), rC, so, o0s);
-          buf_store_so_nt<C>(upd(cur[g][2][1], r1, adt), rC, so, o1s);
-          buf_store_so_nt<C>(upd(cur[g][2][2], r2, adt), rC, so, o2s);
-        } else {
-          const C n0 = upd(cur[g][1][0], r0, adt), n1 = upd(cur[g][1][1], r1, adt), n2 = upd(cur[g][1][2], r2, adt);
-          buf_store_so_nt<C>(n0, rA, so, o0s);
-          buf_store_so_nt<C>(n1, rA, so, o1s);
-          buf_store_so_nt<C>(n2, rA, so, o2s);
-          const double v[6] = {n0.x, n0.y, n1.x, n1.y, n2.x, n2.y};
-          energy_terms(v, K0, K1, K2c, wz, esum, osum);
+        double v[6];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const C(&d)[NL + 1][3] = cur[g];
+          const C u = d[0][i];
+          const C s = d[NL > 1 ? 1 : 0][i];
+          const C st = NL == 1 || (SUM && MODE == P5_RK3) ? u : (KEEP == KEEP_RHS ? caxpy(u, a.sdt, s) : s);
+          C x = mk<C>(r[i].x - ph.x * Kv[i], r[i].y - ph.y * Kv[i]);
+          x = mk<C>(x.x - z * st.x, x.y - z * st.y);
+          x = cadd(x, d[NL][i]);  // rhs += Source (NS.py:256-258), every mode
+          const int o = (i * fs + eo) * CS;
+          if constexpr (MODE == P5_RK3) {
+            C l = d[NL > 4 ? 4 : 0][i];
+            x = rk_last<KEEP, COMP>(a, u, SUM ? s : d[NL > 2 ? 2 : 0][i], d[NL > 3 ? 3 : 0][i], s, x, l);
+            v[2 * i] = x.x;
+            v[2 * i + 1] = x.y;
+            if constexpr (COMP) {
+              buf_store_so_nt<C>(l, rlo, so, o);
+              v[2 * i] += (double)l.x;
+              v[2 * i + 1] += (double)l.y;
+            }
+          } else if constexpr (MODE != P5_RHS && KEEP != KEEP_RHS) {
+            if constexpr (SUM)
+              buf_store_so_nt<C>(caxpy(d[MODE == P5_RK0 ? 0 : (NL > 2 ? 2 : 0)][i], a.adt, x), rb1, so, o);
+            x = caxpy(u, a.bdt, x);
+          }
+          buf_store_so_nt<C>(x, ro, so, o);
         }
+        if constexpr (MODE == P5_RHS || MODE == P5_RK3) buf_store_so_nt<C>(ph, rph, so, eo * CS);
+        if constexpr (MODE == P5_RK3) energy_terms(v, Kv[0], K1, K2c, wz, esum, osum);
       }
       if (j0 + G < NK) {
 #pragma unroll
         for (int g = 0; g < G; ++g) {
           kcur[g] = knxt[g];
 #pragma unroll
-          for (int l = 0; l < NL; ++l)
+          for (int l = 0; l < NL + 1; ++l)
 #pragma unroll
             for (int i = 0; i < 3; ++i) cur[g][l][i] = nxt[g][l][i];
         }
@@ -1250,27 +1292,16 @@ constexpr int occ_blocks(int occ, int threads) {
   const int w = (4 * occ) / bw * bw / 4;
   return w < 1 ? 1 : w;
 }
-// FP32 kernels are held to at least 2 waves per SIMD (256 registers): past
-// that the compiler would move into the AGPR half of the register file and
-// halve the occupancy.
-template <typename Rt, int M, int E> constexpr int p5_occ() {
+// Kernels are held to at least 2 waves per SIMD (256 registers) where they fit
+// them (FP64: lines of 8 points per thread, or 12 with the padded rows): past that the compiler would move into the
+// AGPR half of the register file and halve the occupancy.
+template <typename Rt, int M, int E, bool PAD = false> constexpr int p5_occ() {
   const int o = occ_blocks(occ_for(3 * E, esz_of<Rt>()), SCfg<Rt, M, E>::THREADS);
-  return sizeof(Rt) == 4 && o < 2 ? 2 : o;
+  return (sizeof(Rt) == 4 || (PAD && E <= 12) || E <= 8) && o < 2 ? 2 : o;
 }
-template <typename Rt, int M, int E, int MODE, bool COMP = false, int D = 1>
-__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, E>())) k_p5(P5Args<Rt> a) {
-  using C = cx<Rt>;
-  constexpr int T = SCfg<Rt, M, E>::T / D;
-  __shared__ C lds[M * T];
-  __shared__ C tw[M];
-  const int tile = xcd_tile((a.Q + T - 1) / T);
-  if (tile < 0) return;
-  table_to_lds(tw, (const C*)a.tw, M);
-  p5_body<Rt, M, E, MODE, COMP, T>(a, tile, lds, tw);
-}
-// The 3/2-rule RK stages (p5k_body).
-template <typename Rt, int M, int E, int MODE>
-__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (p5_occ<Rt, M, E>())) k_p5k(P5Args<Rt> a) {
+// Boxes beyond a buffer descriptor's reach (p5_body).
+template <typename Rt, int M, int E, int MODE, int KEEP, bool COMP>
+__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (p5_occ<Rt, M, E>())) k_p5(P5Args<Rt> a) {
   using C = cx<Rt>;
   constexpr int T = SCfg<Rt, M, E>::T;
   __shared__ C lds[M * T];
@@ -1278,7 +1309,18 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (p5_occ<Rt, M, E>()
   const int tile = xcd_tile((a.Q + T - 1) / T);
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
-  p5k_body<Rt, M, E, MODE, T>(a, tile, lds, tw);
+  p5_body<Rt, M, E, MODE, COMP, T, KEEP>(a, tile, lds, tw);
+}
+template <typename Rt, int M, int E, int MODE, bool PAD, bool COMP = false, int D = 1>
+__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, E, PAD>())) k_p5b(P5Args<Rt> a) {
+  using C = cx<Rt>;
+  constexpr int T = SCfg<Rt, M, E>::T / D;
+  __shared__ C lds[M * T];
+  __shared__ C tw[M];
+  const int tile = xcd_tile((a.Q + T - 1) / T);
+  if (tile < 0) return;
+  table_to_lds(tw, (const C*)a.tw, M);
+  p5b_body<Rt, M, E, MODE, PAD, COMP, T>(a, tile, lds, tw);
 }
 
 }  // namespace sdns

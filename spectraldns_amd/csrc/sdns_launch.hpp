@@ -24,8 +24,16 @@ template <typename Rt> int launch_p1(int M, int var, const P1Args<Rt>& a, hipStr
 template <typename Rt> int launch_p2(int M, int var, const P2Args<Rt>& a, hipStream_t s);
 template <typename Rt> int launch_p3(int n, int var, const P3Args<Rt>& a, hipStream_t s);
 // P5: returns the number of column tiles in *nblk (entries of the partial sums);
-// var 2 and 3 run schedules 0 and 1 with the 3/2-rule stage kernels where they apply
-template <typename Rt> int launch_p5(int M, int var, int mode, const P5Args<Rt>& a, hipStream_t s, int* nblk);
+// var & 1 is the schedule (2 and 3 are accepted for stored schedules and mean 0 and 1)
+template <typename Rt, int MODE> int launch_p5(int M, int var, const P5Args<Rt>& a, hipStream_t s, int* nblk);
+template <typename Rt> int launch_p5(int M, int var, int mode, const P5Args<Rt>& a, hipStream_t s, int* nblk) {
+  switch (mode) {
+    case P5_RHS: return launch_p5<Rt, P5_RHS>(M, var, a, s, nblk);
+    case P5_RK0: return launch_p5<Rt, P5_RK0>(M, var, a, s, nblk);
+    case P5_RK12: return launch_p5<Rt, P5_RK12>(M, var, a, s, nblk);
+    default: return launch_p5<Rt, P5_RK3>(M, var, a, s, nblk);
+  }
+}
 // dir = -1 forward, +1 inverse
 template <typename Rt> int launch_strided(int M, int var, int dir, int nfields, const StridedArgs<Rt>& a,
                                           hipStream_t s);

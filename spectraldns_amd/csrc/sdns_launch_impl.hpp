@@ -41,7 +41,14 @@ template <typename Rt, int M, int E> void p1_go(const P1Args<Rt>& a, hipStream_t
   const int ny = a.w ? 6 : 3;
   with_div<MD>(tile_div((long)ny * ((a.Q + Cfg::T - 1) / Cfg::T), MD), [&](auto dd) {
     constexpr int D = decltype(dd)::value, T = Cfg::T / D;
-    hipLaunchKernelGGL((k_p1<Rt, M, E, D>), dim3(xcd_grid((a.Q + T - 1) / T), ny), dim3(Cfg::THREADS / D), 0, s, a);
+    const dim3 g(xcd_grid((a.Q + T - 1) / T), ny), b(Cfg::THREADS / D);
+    if constexpr (sizeof(Rt) == 4) {  // FP64 keeps stage states (rk_keep)
+      if (a.d) {
+        hipLaunchKernelGGL((k_p1<Rt, M, E, D, true>), g, b, 0, s, a);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((k_p1<Rt, M, E, D>), g, b, 0, s, a);
   });
 }
 template <typename Rt, int M, int E> void p2_go(const P2Args<Rt>& a, hipStream_t s) {
@@ -97,57 +104,71 @@ template <typename Rt, int n, int E> void p3c_go(const P3Args<Rt>& a, hipStream_
   if (p3c_try<Rt, n, E, 4>(a, s)) return;
   p3b_go<Rt, n, E>(a, s);  // rows too long for the LDS budget: LDS-assisted scheme
 }
-// The 3/2-rule P5 stages (k_p5k) are compiled for the line lengths of the
-// padded grids from 96 to 768 points; schedule variants 2 and 3 run them when
-// the stage is a plain RK stage of the 3/2 rule whose arrays a buffer
-// descriptor reaches (otherwise, and for variants 0 and 1, p5_body runs).
-constexpr bool p5k_built(int M, int E) { return M % 3 == 0 && E % 3 == 0 && M >= 96 && M <= 768; }
-template <typename Rt> bool p5k_fits(int M, int mode, const P5Args<Rt>& a) {
-  if (mode == P5_RHS || a.Alo || a.source || a.phat || a.conv_only) return false;
-  if (3 * a.N0 != 2 * M || a.x.neg != a.N0 / 2 || a.x.pos != a.N0 / 2 - 1 || a.x.base != a.N0) return false;
+// P5 through buffer descriptors (k_p5b) wherever they reach: byte offsets are
+// 31 bits, so the three components of a state array and of W4 have to span at
+// most BUF_OOB bytes (boxes up to about 640^3 in FP32).  Larger boxes run k_p5.
+template <typename Rt> bool p5b_fits(int M, const P5Args<Rt>& a) {
   const long esz = 2 * (long)sizeof(Rt);
   const long state = 3L * a.N0 * a.N1 * a.Nh * esz;
   const long w4 = 3L * M * (a.y_neg + a.y_pos + 1) * a.nkzop * esz;
   return state <= BUF_OOB && w4 <= BUF_OOB;
 }
-template <typename Rt, int M, int E> void p5_go(int mode, const P5Args<Rt>& a, hipStream_t s, int* nblk, bool fixed_rows) {
+// Padded rows of the 3/2 rule (see p5b_body).
+template <typename Rt> bool p5b_padded(int M, const P5Args<Rt>& a) {
+  return 3 * a.N0 == 2 * M && a.x.neg == a.N0 / 2 && a.x.pos == a.N0 / 2 - 1 && a.x.base == a.N0;
+}
+template <typename Rt, int M, int E, int MODE, bool PAD> void p5b_go(const P5Args<Rt>& a, hipStream_t s, int* nblk) {
   using Cfg = SCfg<Rt, M, E>;
-  const int nt = (a.Q + Cfg::T - 1) / Cfg::T;
-  if (nblk) *nblk = nt;
-  const dim3 g(xcd_grid(nt)), b(Cfg::THREADS);
-  if constexpr (p5k_built(M, E)) {
-    if (fixed_rows && p5k_fits(M, mode, a)) {
-      switch (mode) {
-        case P5_RK0: hipLaunchKernelGGL((k_p5k<Rt, M, E, P5_RK0>), g, b, 0, s, a); break;
-        case P5_RK12: hipLaunchKernelGGL((k_p5k<Rt, M, E, P5_RK12>), g, b, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_p5k<Rt, M, E, P5_RK3>), g, b, 0, s, a); break;
-      }
-      return;
-    }
-  }
-  if constexpr (sizeof(Rt) == 4) {
-    if (a.Alo && mode != P5_RHS) {
-      switch (mode) {
-        case P5_RK0: hipLaunchKernelGGL((k_p5<Rt, M, E, P5_RK0, true>), g, b, 0, s, a); break;
-        case P5_RK12: hipLaunchKernelGGL((k_p5<Rt, M, E, P5_RK12, true>), g, b, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_p5<Rt, M, E, P5_RK3, true>), g, b, 0, s, a); break;
-      }
+  if constexpr (sizeof(Rt) == 4 && !PAD && MODE != P5_RHS) {
+    if (a.lo) {
+      const int nt = (a.Q + Cfg::T - 1) / Cfg::T;
+      if (nblk) *nblk = nt;
+      hipLaunchKernelGGL((k_p5b<Rt, M, E, MODE, PAD, true>), dim3(xcd_grid(nt)), dim3(Cfg::THREADS), 0, s, a);
       return;
     }
   }
   constexpr int MD = max_div(M, 128, Cfg::T, Cfg::THREADS);
-  with_div<MD>(tile_div(nt, MD), [&](auto dd) {
+  with_div<MD>(tile_div((a.Q + Cfg::T - 1) / Cfg::T, MD), [&](auto dd) {
     constexpr int D = decltype(dd)::value, T = Cfg::T / D;
-    const int ntd = (a.Q + T - 1) / T;
-    if (nblk) *nblk = ntd;
-    const dim3 gd(xcd_grid(ntd)), bd(Cfg::THREADS / D);
-    switch (mode) {
-      case P5_RHS: hipLaunchKernelGGL((k_p5<Rt, M, E, P5_RHS, false, D>), gd, bd, 0, s, a); break;
-      case P5_RK0: hipLaunchKernelGGL((k_p5<Rt, M, E, P5_RK0, false, D>), gd, bd, 0, s, a); break;
-      case P5_RK12: hipLaunchKernelGGL((k_p5<Rt, M, E, P5_RK12, false, D>), gd, bd, 0, s, a); break;
-      default: hipLaunchKernelGGL((k_p5<Rt, M, E, P5_RK3, false, D>), gd, bd, 0, s, a); break;
-    }
+    const int nt = (a.Q + T - 1) / T;
+    if (nblk) *nblk = nt;
+    hipLaunchKernelGGL((k_p5b<Rt, M, E, MODE, PAD, false, D>), dim3(xcd_grid(nt)), dim3(Cfg::THREADS / D), 0, s, a);
   });
+}
+// Stages 1 and 2 with the accumulator (FP32, 3/2 rule: ten mixed read and write
+// streams) run p5_body: 0.313 ms at 256^3 against 0.336 ms of p5b_body, whose
+// prefetch only adds streams there; stages 0 and 3 take 0.246 against 0.248 and
+// 0.241 against 0.247 ms.
+template <typename Rt, int M, int V, int MODE> void p5_go(const P5Args<Rt>& a, hipStream_t s, int* nblk) {
+  constexpr int EV = strided_E(M, V);
+  constexpr bool PADB = M % 3 == 0 && EV % 3 == 0;
+  constexpr bool PAD_SUM = PADB && MODE == P5_RK12 && rk_keep<Rt>(true, false) == KEEP_SUM;
+  const bool fits = p5b_fits(M, a);
+  if (fits && M == a.N0) return p5b_go<Rt, M, EV, MODE, false>(a, s, nblk);
+  if constexpr (PADB && !PAD_SUM) {
+    // (the compensated stages of the 3/2 rule run p5_body)
+    if (fits && p5b_padded(M, a) && (!a.lo || MODE == P5_RHS)) return p5b_go<Rt, M, EV, MODE, true>(a, s, nblk);
+  }
+  // one schedule for the boxes beyond a descriptor's reach
+  constexpr int E0 = PAD_SUM ? EV : strided_E(M, 0);
+  using Cfg = SCfg<Rt, M, E0>;
+  const int nt = (a.Q + Cfg::T - 1) / Cfg::T;
+  if (nblk) *nblk = nt;
+  const dim3 g(xcd_grid(nt)), b(Cfg::THREADS);
+  constexpr bool RK = MODE != P5_RHS;
+  if constexpr (sizeof(Rt) == 4 && RK) {
+    if (a.lo) {
+      hipLaunchKernelGGL((k_p5<Rt, M, E0, MODE, rk_keep<Rt>(false, true), true>), g, b, 0, s, a);
+      return;
+    }
+  }
+  if constexpr (RK && rk_keep<Rt>(true, false) != rk_keep<Rt>(false, false)) {
+    if (M != a.N0) {
+      hipLaunchKernelGGL((k_p5<Rt, M, E0, MODE, rk_keep<Rt>(true, false), false>), g, b, 0, s, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_p5<Rt, M, E0, MODE, rk_keep<Rt>(false, false), false>), g, b, 0, s, a);
 }
 template <typename Rt, int M, int E> void strided_go(int dir, int nfields, const StridedArgs<Rt>& a0, hipStream_t s) {
   using Cfg = SCfg<Rt, M, E>;
@@ -221,12 +242,12 @@ template <typename Rt> int launch_p3(int n, int var, const P3Args<Rt>& a, hipStr
   }
 }
 
-template <typename Rt> int launch_p5(int M, int var, int mode, const P5Args<Rt>& a, hipStream_t s, int* nblk) {
+template <typename Rt, int MODE> int launch_p5(int M, int var, const P5Args<Rt>& a, hipStream_t s, int* nblk) {
   switch (M) {
 #define SDNS_X(m)                                                        \
   case m:                                                                \
-    if (var & 1) p5_go<Rt, m, strided_E(m, 1)>(mode, a, s, nblk, var >= 2); \
-    else p5_go<Rt, m, strided_E(m, 0)>(mode, a, s, nblk, var >= 2);      \
+    if (var & 1) p5_go<Rt, m, 1, MODE>(a, s, nblk);                      \
+    else p5_go<Rt, m, 0, MODE>(a, s, nblk);                              \
     return 0;
     SDNS_STRIDED_SIZES(SDNS_X)
 #undef SDNS_X
@@ -748,8 +769,12 @@ template <typename Rt> int launch_errnorm(const void* err, const void* u0, const
   namespace sdns { template int launch_p2<Rt>(int, int, const P2Args<Rt>&, hipStream_t); }
 #define SDNS_PART_P3(Rt) \
   namespace sdns { template int launch_p3<Rt>(int, int, const P3Args<Rt>&, hipStream_t); }
-#define SDNS_PART_P5(Rt) \
-  namespace sdns { template int launch_p5<Rt>(int, int, int, const P5Args<Rt>&, hipStream_t, int*); }
+#define SDNS_P5_MODE(Rt, MODE) \
+  namespace sdns { template int launch_p5<Rt, MODE>(int, int, const P5Args<Rt>&, hipStream_t, int*); }
+#define SDNS_PART_P5RHS(Rt) SDNS_P5_MODE(Rt, P5_RHS)
+#define SDNS_PART_P5RK0(Rt) SDNS_P5_MODE(Rt, P5_RK0)
+#define SDNS_PART_P5RK12(Rt) SDNS_P5_MODE(Rt, P5_RK12)
+#define SDNS_PART_P5RK3(Rt) SDNS_P5_MODE(Rt, P5_RK3)
 #define SDNS_PART_LINES(Rt)                                                                      \
   namespace sdns {                                                                               \
   template int launch_strided<Rt>(int, int, int, int, const StridedArgs<Rt>&, hipStream_t);      \

@@ -29,6 +29,7 @@ struct RowMap {
 
 template <typename Rt> struct P1Args {  // x-inverse of u_hat + kx products
   const void* u;      // state [3][N0][N1][Nh]
+  const void* d;      // the state is u + ds d (RK stages with KEEP_RHS), or null: u
   const void* w;      // given vorticity [3][N0][N1][Nh], or null: then W1 holds
                       // the six plain x-inverses u, v, w, wx, wy, wz (no kx products)
   void* w1;           // [5][M0][Q] ([6][M0][Q] with a given vorticity)
@@ -39,6 +40,7 @@ template <typename Rt> struct P1Args {  // x-inverse of u_hat + kx products
   int y_neg, y_pos;   // kept input modes of axis 1
   int nkz, nkzp;      // kept input kz count, padded kz stride of W1
   int Q;              // nky * nkzp columns (= W1 row stride)
+  Rt ds;
 };
 
 template <typename Rt> struct P2Args {  // y-inverse + curl assembly
@@ -93,13 +95,34 @@ template <typename Rt> struct ZArgs {
 
 enum P5Mode { P5_RHS = 0, P5_RK0 = 1, P5_RK12 = 2, P5_RK3 = 3 };
 
+// RK4 in the P5 stages: start value u, stage right-hand sides k1..k4, stage
+// states B_i = u + b_i dt k_i, sum u + sum a_i dt k_i (integrators.py:155-157).
+// What the stages keep for the sum decides their traffic (F: one spectral
+// field; the passes before P5 read the stage state):
+//   KEEP_SUM: an accumulator that every stage reads and writes: 48 F per step,
+//     21 F of it written.
+//   KEEP_STATES: only the B_i; the last stage adds
+//     ((B1 - u) + 2 (B2 - u) + (B3 - u)) / 3 + dt/6 k4: 39 F, 12 F written.
+//   KEEP_RHS: only the k_i; whoever reads a stage state forms u + b_i dt k_i,
+//     and the last stage adds the terms with the accumulator's roundings, plain
+//     or compensated: 39 F, 12 F written, and 9 F more in the x-inverse pass times
+//     the share of the modes that it reads (0.3 with the 2/3 rule).
+// FP64 keeps the states.  FP32 keeps the accumulator's roundings: right-hand
+// sides, except with the 3/2 rule, whose x-inverse reads every mode (256^3:
+// 4.95 ms per step with the sum, 5.12 ms with right-hand sides).
+enum RkKeep { KEEP_SUM = 0, KEEP_STATES = 1, KEEP_RHS = 2 };
+template <typename Rt> constexpr int rk_keep(bool padded, bool comp) {
+  return sizeof(Rt) == 8 ? KEEP_STATES : (padded && !comp ? KEEP_SUM : KEEP_RHS);
+}
+
 template <typename Rt> struct P5Args {  // x-forward + mask + pressure + diffusion + RK4 stage
   const void* w4;     // [3][M0][nkyo][nkzo]
-  void* A;            // step base u1 (and final result)
-  void* B;            // stage value u0
-  void* Cacc;         // accumulator u2
-  void* Alo;          // compensated mode: low part of u1 / of the result (caller's u_lo)
-  void* Clo;          // compensated mode: low part of u2
+  void* u;            // state: step base, and the result of stage 3 (P5_RHS: the input state)
+  const void* s;      // stages 1..3: the stage state whose RHS this is, or the last k (KEEP_RHS)
+  void* out;          // stages 0..2: the next stage state, or this stage's k (KEEP_RHS)
+  void* b1;           // stage 3: B1, B2 or k1, k2; KEEP_SUM: b1 is the accumulator of all stages
+  const void* b2;
+  void* lo;           // compensated mode: low part of u (caller's u_lo)
   void* rhs;          // P5_RHS: rhs output
   void* phat;         // P5_RHS: pressure output (may be null)
   const void* source; // P5_RHS: added source (may be null)
@@ -112,7 +135,10 @@ template <typename Rt> struct P5Args {  // x-forward + mask + pressure + diffusi
   int nkzo, nkzop;    // kept output kz count, padded kz stride of W4
   int mask_nyquist;
   int conv_only;      // P5_RHS: write the scaled convection term only
-  Rt nu, scale, adt, bdt;
+  Rt nu, scale;
+  Rt adt, bdt;        // a dt and b dt of this stage
+  Rt sdt;             // KEEP_RHS: the stage state is u + sdt s
+  Rt a12;             // KEEP_RHS, stage 3: a dt of stages 1 and 2 (stage 0's is adt)
   int Q;              // N1 * Nh state columns
 };
 
