@@ -120,11 +120,11 @@ struct sdns_closure {
   char* mem = nullptr;
   __bf16 *x0 = nullptr, *z1 = nullptr, *a1 = nullptr, *z2 = nullptr, *a2 = nullptr;
   __bf16 *gyb = nullptr, *gz2 = nullptr, *gz1 = nullptr;
-  float *y = nullptr, *gy = nullptr, *t = nullptr, *wpart = nullptr, *bpart = nullptr;
+  float *y = nullptr, *wpart = nullptr, *gsum = nullptr;
   float *phys = nullptr, *tauphys = nullptr;
   char *tauhat = nullptr, *src = nullptr;  // 6 and 3 complex64 spectral fields
   char* stage = nullptr;                   // 3 fields: the stage state of per-stage evaluations (in tauhat)
-  double *lpart = nullptr, *loss = nullptr;
+  double* lpart = nullptr;
   sdns::ClosureWeights w{};
   bool have_params = false;
 };
@@ -539,18 +539,19 @@ template <typename Rt> int form_state(sdns_plan* p, void* out, const P1Args<Rt>&
   return 0;
 }
 
-// Network forward on the closure's packed input x0 -> y (FP32, 6 of 8 channels).
-// keep_pre: store the pre-activations z1, z2 (the backward pass reads them;
-// inference does not).
-int closure_net_forward(sdns_closure* c, hipStream_t st, bool keep_pre) {
+// Network forward on the closure's packed input x0.  Training (tau = null):
+// y = output, FP32 [P][8], 6 real, and the pre-activations z1, z2 that the
+// backward pass reads; inference: tau = out_scale * output, planar.
+int closure_net_forward(sdns_closure* c, hipStream_t st, float* tau, float out_scale) {
   ConvArgs a{};
   a.n0 = c->n[0]; a.n1 = c->n[1]; a.n2 = c->n[2];
-  a.x = c->x0; a.w = c->w.w1f; a.bias = c->w.b1; a.z = keep_pre ? c->z1 : nullptr; a.a = c->a1;
+  a.x = c->x0; a.w = c->w.w1f; a.bias = c->w.b1; a.z = tau ? nullptr : c->z1; a.a = c->a1;
   if (launch_conv(8, 32, CONV_EPI_SILU, a, st)) return fail(SDNS_ERR_UNSUPPORTED, "closure grid");
-  a.x = c->a1; a.w = c->w.w2f; a.bias = c->w.b2; a.z = keep_pre ? c->z2 : nullptr; a.a = c->a2;
+  a.x = c->a1; a.w = c->w.w2f; a.bias = c->w.b2; a.z = tau ? nullptr : c->z2; a.a = c->a2;
   if (launch_conv(32, 32, CONV_EPI_SILU, a, st)) return fail(SDNS_ERR_HIP, "closure layer 2");
-  a.x = c->a2; a.w = c->w.w3f; a.bias = c->w.b3; a.z = nullptr; a.a = nullptr; a.y = c->y; a.ystride = 8; a.ncout = 6;
-  if (launch_conv(32, 16, CONV_EPI_LINEAR, a, st)) return fail(SDNS_ERR_HIP, "closure layer 3");
+  a.x = c->a2; a.w = c->w.w3f; a.bias = c->w.b3; a.z = nullptr; a.a = nullptr; a.ncout = 6;
+  a.y = tau ? tau : c->y; a.ystride = 8; a.scale = out_scale;
+  if (launch_conv(32, 16, tau ? CONV_EPI_PLANAR : CONV_EPI_LINEAR, a, st)) return fail(SDNS_ERR_HIP, "closure layer 3");
   return 0;
 }
 
@@ -560,8 +561,7 @@ int closure_source(sdns_closure* c, sdns_plan* p, const void* u, float in_scale,
   int rc;
   if ((rc = plain_backward<float>(p, u, c->phys, 3))) return rc;
   launch_pack_input(c->phys, in_scale, c->x0, c->P, p->stream);
-  if ((rc = closure_net_forward(c, p->stream, false))) return rc;
-  launch_unpack_output(c->y, out_scale, c->tauphys, c->P, p->stream);
+  if ((rc = closure_net_forward(c, p->stream, c->tauphys, out_scale))) return rc;
   const size_t fbytes = (size_t)p->N[0] * p->N[1] * p->Nh * p->esz;
   if ((rc = plain_forward<float>(p, c->tauphys, c->tauhat, 3))) return rc;
   if ((rc = plain_forward<float>(p, c->tauphys + 3 * c->P, c->tauhat + 3 * fbytes, 3))) return rc;
@@ -1540,16 +1540,14 @@ int sdns_closure_create(sdns_closure** out, const int32_t N[3], void* hip_stream
   for (int i = 0; i < 3; ++i) c->n[i] = N[i];
   c->P = P;
   c->stream = (hipStream_t)hip_stream;
-  const long nchunk = P / 4096;
   const size_t fbytes = (size_t)N[0] * N[1] * (N[2] / 2 + 1) * 8;  // complex64 spectral field
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t o = off; off += align256(bytes); return o; };
   const size_t o_x0 = take(P * 8 * 2), o_z1 = take(P * 64), o_a1 = take(P * 64), o_z2 = take(P * 64),
                o_a2 = take(P * 64), o_gyb = take(P * 16), o_gz2 = take(P * 64), o_gz1 = take(P * 64),
-               o_y = take(P * 32), o_gy = take(P * 32), o_t = take(P * 32),
-               o_wp = take(nchunk * 27 * 32 * 32 * 4), o_bp = take(256 * 32 * 4), o_ph = take(3 * P * 4),
-               o_tp = take(6 * P * 4), o_th = take(6 * fbytes), o_src = take(3 * fbytes), o_lp = take(256 * 8),
-               o_l = take(8), o_w1 = take(27 * 32 * 8 * 2), o_w2 = take(27 * 32 * 32 * 2),
+               o_y = take(P * 32), o_wp = take(wgrad_part_floats(N[0], N[1], N[2]) * 4), o_gs = take(256 * 8 * 4),
+               o_ph = take(3 * P * 4), o_tp = take(6 * P * 4), o_th = take(6 * fbytes), o_src = take(3 * fbytes),
+               o_lp = take(256 * 8), o_w1 = take(27 * 32 * 8 * 2), o_w2 = take(27 * 32 * 32 * 2),
                o_w3 = take(27 * 16 * 32 * 2), o_w3b = take(27 * 32 * 8 * 2), o_w2b = take(27 * 32 * 32 * 2),
                o_b = take(80 * 4);
   if (hipMalloc((void**)&c->mem, off) != hipSuccess) {
@@ -1560,11 +1558,10 @@ int sdns_closure_create(sdns_closure** out, const int32_t N[3], void* hip_stream
   c->x0 = (__bf16*)(m + o_x0); c->z1 = (__bf16*)(m + o_z1); c->a1 = (__bf16*)(m + o_a1);
   c->z2 = (__bf16*)(m + o_z2); c->a2 = (__bf16*)(m + o_a2); c->gyb = (__bf16*)(m + o_gyb);
   c->gz2 = (__bf16*)(m + o_gz2); c->gz1 = (__bf16*)(m + o_gz1);
-  c->y = (float*)(m + o_y); c->gy = (float*)(m + o_gy); c->t = (float*)(m + o_t);
-  c->wpart = (float*)(m + o_wp); c->bpart = (float*)(m + o_bp); c->phys = (float*)(m + o_ph);
+  c->y = (float*)(m + o_y); c->wpart = (float*)(m + o_wp); c->gsum = (float*)(m + o_gs); c->phys = (float*)(m + o_ph);
   c->tauphys = (float*)(m + o_tp); c->tauhat = m + o_th; c->src = m + o_src;
   c->stage = c->tauhat;  // read by the transform before tau's is written
-  c->lpart = (double*)(m + o_lp); c->loss = (double*)(m + o_l);
+  c->lpart = (double*)(m + o_lp);
   c->w.w1f = (__bf16*)(m + o_w1); c->w.w2f = (__bf16*)(m + o_w2); c->w.w3f = (__bf16*)(m + o_w3);
   c->w.w3b = (__bf16*)(m + o_w3b); c->w.w2b = (__bf16*)(m + o_w2b);
   c->w.b1 = (float*)(m + o_b); c->w.b2 = c->w.b1 + 32; c->w.b3 = c->w.b2 + 32;
@@ -1589,10 +1586,8 @@ int sdns_closure_forward(sdns_closure* c, const float* u_phys, float in_scale, f
   if (!c || !u_phys || !tau_phys) return fail(SDNS_ERR_INVALID, "bad argument");
   if (!c->have_params) return fail(SDNS_ERR_INVALID, "closure parameters not set");
   launch_pack_input(u_phys, in_scale, c->x0, c->P, c->stream);
-  int rc = closure_net_forward(c, c->stream, false);
-  if (rc) return rc;
-  launch_unpack_output(c->y, out_scale, tau_phys, c->P, c->stream);
-  return check_launch();
+  const int rc = closure_net_forward(c, c->stream, tau_phys, out_scale);
+  return rc ? rc : check_launch();
 }
 
 int sdns_closure_train_step(sdns_closure* c, const float* u_phys, const float* tau_phys, float in_scale,
@@ -1603,30 +1598,22 @@ int sdns_closure_train_step(sdns_closure* c, const float* u_phys, const float* t
   const long P = c->P;
   const int n0 = c->n[0], n1 = c->n[1], n2 = c->n[2];
   launch_pack_input(u_phys, in_scale, c->x0, P, st);
-  int rc = closure_net_forward(c, st, true);
+  const int rc = closure_net_forward(c, st, nullptr, 1.f);
   if (rc) return rc;
-  launch_pack_target(tau_phys, 1.0f / out_scale, c->t, P, st);
-  launch_loss(c->y, c->t, c->gy, c->gyb, P, c->lpart, c->loss, st);
+  launch_loss(c->y, tau_phys, 1.0f / out_scale, c->gyb, P, c->lpart, c->gsum, st);
   // layer 3
-  int nch = launch_wgrad(8, 32, c->gyb, c->a2, c->wpart, n0, n1, n2, st);
-  if (nch < 0) return fail(SDNS_ERR_UNSUPPORTED, "closure grid");
-  launch_wgrad_reduce(c->wpart, nch, 8, 32, 6, 32, grad + CL_OW3, st);
-  launch_bgrad_f32(c->gy, 8, 6, P, c->bpart, grad + CL_OB3, st);
+  if (launch_wgrad(2, c->gyb, c->a2, c->wpart, n0, n1, n2, st)) return fail(SDNS_ERR_UNSUPPORTED, "closure grid");
   ConvArgs a{};
   a.n0 = n0; a.n1 = n1; a.n2 = n2;
   a.x = c->gyb; a.w = c->w.w3b; a.zprev = c->z2; a.a = c->gz2;
   if (launch_conv(8, 32, CONV_EPI_DSILU, a, st)) return fail(SDNS_ERR_HIP, "closure layer 3 input gradient");
   // layer 2
-  nch = launch_wgrad(32, 32, c->gz2, c->a1, c->wpart, n0, n1, n2, st);
-  launch_wgrad_reduce(c->wpart, nch, 32, 32, 32, 32, grad + CL_OW2, st);
-  launch_bgrad_bf16(c->gz2, 32, 32, P, c->bpart, grad + CL_OB2, st);
+  launch_wgrad(1, c->gz2, c->a1, c->wpart, n0, n1, n2, st);
   a.x = c->gz2; a.w = c->w.w2b; a.zprev = c->z1; a.a = c->gz1;
   if (launch_conv(32, 32, CONV_EPI_DSILU, a, st)) return fail(SDNS_ERR_HIP, "closure layer 2 input gradient");
   // layer 1
-  nch = launch_wgrad(32, 8, c->gz1, c->x0, c->wpart, n0, n1, n2, st);
-  launch_wgrad_reduce(c->wpart, nch, 32, 8, 32, 3, grad + CL_OW1, st);
-  launch_bgrad_bf16(c->gz1, 32, 32, P, c->bpart, grad + CL_OB1, st);
-  if (loss) HIP_TRY(hipMemcpyAsync(loss, c->loss, sizeof(double), hipMemcpyDeviceToDevice, st));
+  launch_wgrad(0, c->gz1, c->x0, c->wpart, n0, n1, n2, st);
+  launch_grad_reduce(c->wpart, n0, n1, n2, c->gsum, c->lpart, grad, loss, st);
   return check_launch();
 }
 

@@ -35,7 +35,7 @@ struct ClosureWeights {
   float* b3;     // [16] (6 real)
 };
 
-enum { CONV_EPI_SILU = 0, CONV_EPI_LINEAR = 1, CONV_EPI_DSILU = 2 };
+enum { CONV_EPI_SILU = 0, CONV_EPI_LINEAR = 1, CONV_EPI_DSILU = 2, CONV_EPI_PLANAR = 3 };
 
 struct ConvArgs {
   const __bf16* x;      // input [P][cin]
@@ -43,37 +43,32 @@ struct ConvArgs {
   const float* bias;    // [cout] or null
   __bf16* z;            // SILU: pre-activation out [P][cout] (null: not stored)
   __bf16* a;            // SILU: activation out; DSILU: gradient out [P][cout]
-  float* y;             // LINEAR: FP32 out [P][ystride], channels < ncout written
+  float* y;             // LINEAR: FP32 out [P][ystride]; PLANAR: [ncout][P], times scale; channels < ncout written
   const __bf16* zprev;  // DSILU: stored pre-activation [P][cout] whose SiLU' multiplies the result
   int n0, n1, n2;
   int ystride, ncout;
+  float scale;
 };
 
-// cin in {8, 32}, cout in {16, 32}; N2 % 16 == 0 and N0*N1*N2 % 64 == 0.
-// 32-channel inputs are LDS-tiled (weights and a rolling window of input
-// planes staged per block) when N0 % 4 == 0, N1 % 4 == 0 and N2 <= 64 or
-// N2 % 64 == 0.  Returns nonzero if the shape or the launch set-up
-// is not supported.
+// cin in {8, 32}, cout in {16, 32}; N2 % 32 == 0, N0 and N1 at least 4.  Returns
+// nonzero if the shape or the launch set-up is not supported.
 int launch_conv(int cin, int cout, int epi, const ConvArgs& a, hipStream_t s);
-// Weight-gradient partials: part[chunk][27][gc][xc] = sum over the chunk's
-// points p of g[p][co] x[p + d(tap)][ci]; gc, xc in {8, 32}; chunk = 4096
-// points (N0*N1*N2 % 4096 == 0, N2 % 32 == 0).  Returns the number of chunks.
-int launch_wgrad(int gc, int xc, const __bf16* g, const __bf16* x, float* part, int n0, int n1, int n2,
-                 hipStream_t s);
-// Sum the partials over chunks into the canonical gradient W[tap][co < cout_real][ci < cin_real].
-int launch_wgrad_reduce(const float* part, int nchunk, int gc, int xc, int cout_real, int cin_real, float* grad,
-                        hipStream_t s);
-// Bias gradient: grad[c] = sum_p g[p][c] for c < creal (g bf16 or FP32 with row stride gc).
-int launch_bgrad_bf16(const __bf16* g, int gc, int creal, long npts, float* part, float* grad, hipStream_t s);
-int launch_bgrad_f32(const float* g, int gc, int creal, long npts, float* part, float* grad, hipStream_t s);
-// Loss and its gradient: y, t FP32 [P][8] (6 real); gy = 2 (y - t) / (6 P) as FP32
-// and bf16 [P][8] (pad 0); loss (device double) = mean (y - t)^2.
-int launch_loss(const float* y, const float* t, float* gy, __bf16* gyb, long npts, double* part, double* loss,
+// Weight- and bias-gradient partials of layer 0..2 (g: gradient of the layer's
+// pre-activation, x: its input; channels 32/8, 32/32, 8/32) into its part of
+// `part`, wgrad_part_floats floats in all; the same shapes as launch_conv.
+size_t wgrad_part_floats(int n0, int n1, int n2);
+int launch_wgrad(int layer, const __bf16* g, const __bf16* x, float* part, int n0, int n1, int n2, hipStream_t s);
+// Loss partials, gyb = 2 (y - scale tau) / (6 P) in bf16 [P][8] (pad 0) and its
+// FP32 channel sums; y FP32 [P][8] (6 real), tau planar [6][P]; part: 256
+// doubles, gsum: 256 x 8 floats.
+int launch_loss(const float* y, const float* tau, float scale, __bf16* gyb, long npts, double* part, float* gsum,
                 hipStream_t s);
-// Planar FP32 fields [c][P] * scale <-> channels-last.
+// The canonical gradient from the partials of the three layers and of the
+// loss, and loss (device double, may be null) = mean (y - scale tau)^2.
+int launch_grad_reduce(const float* part, int n0, int n1, int n2, const float* gsum, const double* lpart, float* grad,
+                       double* loss, hipStream_t s);
+// Planar FP32 fields [c][P] * scale -> channels-last.
 int launch_pack_input(const float* u, float scale, __bf16* x, long npts, hipStream_t s);        // [3][P] -> bf16 [P][8]
-int launch_pack_target(const float* tau, float scale, float* t, long npts, hipStream_t s);      // [6][P] -> f32 [P][8]
-int launch_unpack_output(const float* y, float scale, float* tau, long npts, hipStream_t s);    // f32 [P][8] -> [6][P]
 // Canonical FP32 parameters -> bf16 device layouts.
 int launch_pack_weights(const float* params, const ClosureWeights& w, hipStream_t s);
 // Adam (Kingma & Ba 2015) on n FP32 parameters, step t >= 1.
