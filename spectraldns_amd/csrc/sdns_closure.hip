@@ -77,54 +77,68 @@ template <int EPI> __device__ __forceinline__ f32x4 conv_bias(const ConvArgs& a,
 }
 
 // 8-channel inputs: K = 32 is 4 taps x 8 channels, seven K-steps (k-group g of
-// step s is tap 4 s + g; the 28th tap is zeros).  A wave owns one z-row segment
-// of 16 MT points and keeps the layer's weights in registers; the input
-// fragments come straight from global memory (each input row is read by 9
-// rows' waves through L1 and L2), their row offsets computed once per wave.
+// step s is tap 4 s + g; the 28th tap is zeros).  A block owns 4 y-rows x 16 MT z
+// points of two x-planes and stages their halo (4 planes x 6 rows x (16 MT + 2)
+// points of 16 bytes, 25 KB) in LDS; wave w computes row w of both planes with
+// the layer's weights in registers.  (Fragments straight from global memory,
+// 7 KB per 16 points through L1, took 19 us at 64^3.)
+constexpr int CONV8_XP = 2, CONV_ROWS = 4;
 template <int COUT, int EPI, int MT>
 __global__ void __launch_bounds__(256) k_conv8(ConvArgs a) {
-  constexpr int NB = COUT / 16, KS = 7;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int NB = COUT / 16, KS = 7, npt = 16 * MT + 2;
+  constexpr int PC = (CONV_ROWS + 2) * npt, NC = (CONV8_XP + 2) * PC, NR = (NC + 255) / 256;
+  __shared__ bf16x8 hl[NC];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int nseg = a.n2 / (16 * MT);
-  const int seg = blockIdx.x * 4 + wave;
-  if (seg >= a.n0 * a.n1 * nseg) return;
-  const int z0 = seg % nseg * (16 * MT), r = seg / nseg;
-  const int i1 = r % a.n1, i0 = r / a.n1;
+  const int n0 = a.n0, n1 = a.n1, n2 = a.n2;
+  const int nzb = n2 / (16 * MT), nrb = (n1 + CONV_ROWS - 1) / CONV_ROWS;
+  int blk = blockIdx.x;
+  const int z0 = blk % nzb * (16 * MT);
+  blk /= nzb;
+  const int i1b = blk % nrb * CONV_ROWS, x0 = blk / nrb * CONV8_XP;
   const bf16x8* __restrict__ X = (const bf16x8*)a.x;
   const bf16x8* __restrict__ W = (const bf16x8*)a.w;
+  bf16x8 r[NR];
+#pragma unroll
+  for (int e = 0; e < NR; ++e) {
+    const int c = min((int)threadIdx.x + 256 * e, NC - 1);
+    const int pt = c % npt, row = c / npt % (CONV_ROWS + 2), j = c / PC;
+    r[e] = X[((long)wrap(x0 + j - 1, n0) * n1 + wrap(i1b + row - 1, n1)) * n2 + wrap(z0 + pt - 1, n2)];
+  }
   bf16x8 wv[KS][NB];
-  long row[KS];
-  int dx[KS];
+  int off[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
     const int tap = 4 * s + g < 27 ? 4 * s + g : 26;
 #pragma unroll
     for (int b = 0; b < NB; ++b) wv[s][b] = 4 * s + g < 27 ? W[tap * COUT + b * 16 + m] : bf16x8{};
-    const int tz = tap / 9, ty = (tap / 3) % 3;
-    dx[s] = tap % 3 - 1;
-    row[s] = ((long)wrap(i0 + tz - 1, a.n0) * a.n1 + wrap(i1 + ty - 1, a.n1)) * a.n2;
+    off[s] = (tap / 9) * PC + (w + tap / 3 % 3) * npt + tap % 3 + m;
   }
   f32x4 bias[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) bias[b] = conv_bias<EPI>(a, 16 * b + 4 * g);
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int i2 = z0 + 16 * t + m;
-    f32x4 acc[NB];
+  for (int e = 0; e < NR; ++e)
+    if (threadIdx.x + 256 * e < NC) hl[threadIdx.x + 256 * e] = r[e];
+  __syncthreads();
+  if (i1b + w >= n1) return;
+  for (int k = 0; k < CONV8_XP && x0 + k < n0; ++k) {
+    const long prow = ((long)(x0 + k) * n1 + i1b + w) * n2 + z0;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 pv[KS];
+    for (int t = 0; t < MT; ++t) {
+      f32x4 acc[NB];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) pv[s] = X[row[s] + wrap(i2 + dx[s], a.n2)];
-    if (4 * (KS - 1) + g >= 27) pv[KS - 1] = bf16x8{};
+      for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
+      for (int s = 0; s < KS; ++s) {
+        bf16x8 pv = hl[k * PC + off[s] + 16 * t];
+        if (s == KS - 1 && 4 * s + g >= 27) pv = bf16x8{};
 #pragma unroll
-      for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[s][b], pv[s], acc[b], 0, 0, 0);
-    const long pt = (long)r * a.n2 + i2;
+        for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[s][b], pv, acc[b], 0, 0, 0);
+      }
 #pragma unroll
-    for (int b = 0; b < NB; ++b) conv_epilogue<EPI, COUT>(a, acc[b], bias[b], pt, 16 * b + 4 * g);
+      for (int b = 0; b < NB; ++b) conv_epilogue<EPI, COUT>(a, acc[b], bias[b], prow + 16 * t + m, 16 * b + 4 * g);
+    }
   }
 }
 
@@ -135,11 +149,12 @@ __global__ void __launch_bounds__(256) k_conv8(ConvArgs a) {
 // LDS slots, the plane after next loaded into registers while the current
 // output plane is computed and stored into its free slot afterwards.  One
 // block fills a CU's LDS (157 KB at 32 -> 32 channels and 64 points), so it has
-// 8 waves: waves w and w + 4 compute the two halves of row w, and on each SIMD
-// one wave's products overlap the other's epilogue (with 4 waves, one per SIMD,
-// the matrix cores waited for it).  Rows and planes past the grid are computed
+// 8 waves: waves w and w + 4 compute the two halves of row w, and each wave
+// finishes a plane (SiLU is about 40 VALU instructions a value, more time than
+// the products) between the next plane's products, the two waves of a SIMD at
+// different taps.  Rows and planes past the grid are computed
 // from wrapped input and not stored.
-constexpr int CONV_ROWS = 4, CONV_XP = 4, CONV_SLOTS = 4;
+constexpr int CONV_XP = 4, CONV_SLOTS = 4;
 template <int COUT> constexpr int conv_w_bytes() { return 27 * COUT * 32 * 2; }
 constexpr int conv_plane_chunks(int tzn) { return (CONV_ROWS + 2) * (tzn + 2) * 4; }
 
@@ -185,23 +200,35 @@ __global__ void __launch_bounds__(512, 2) k_conv_lds(ConvArgs a) {
   load_plane(-1, p0);  // planes x0 - 1, x0, x0 + 1
   load_plane(0, p1);
   load_plane(1, pre);
-  for (int c = threadIdx.x; c < 27 * COUT * 4; c += 512) wl[c] = W[c];
+  constexpr int WC = 27 * COUT * 4, WR = (WC + 511) / 512;
+  bf16x8 wr[WR];
+#pragma unroll
+  for (int e = 0; e < WR; ++e) wr[e] = W[min((int)threadIdx.x + 512 * e, WC - 1)];
+#pragma unroll
+  for (int e = 0; e < WR; ++e)
+    if (threadIdx.x + 512 * e < WC) wl[threadIdx.x + 512 * e] = wr[e];
   store_plane(-1, p0);
   store_plane(0, p1);
   store_plane(1, pre);
   __syncthreads();
-  const int lane = threadIdx.x & 63, w = (threadIdx.x >> 6) & 3, half = threadIdx.x >> 8;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int w = wave & 3, half = wave >> 2;
   const int m = lane & 15, g = lane >> 4;
   const bool row_ok = i1b + w < n1;
   f32x4 bias[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) bias[b] = conv_bias<EPI>(a, 16 * b + 4 * g);
+  f32x4 acc[MW][NB], done[MW][NB];  // this plane's sums, the last plane's
+  auto finish = [&](int k, int i) {
+    const long prow = ((long)(x0 + k) * n1 + i1b + w) * n2 + z0;
+    const int t = i / NB, b = i % NB;
+    conv_epilogue<EPI, COUT>(a, done[t][b], bias[b], prow + 16 * (half * MW + t) + m, 16 * b + 4 * g);
+  };
   for (int k = 0; k < nx; ++k) {
-    const bool more = k + 1 < nx;
+    const bool more = k + 1 < nx, pending = k > 0 && row_ok;
     if (more) load_plane(k + 2, pre);  // in flight during this plane's products
     const bf16x8* const pl[3] = {hl + (k % CONV_SLOTS) * PC, hl + ((k + 1) % CONV_SLOTS) * PC,
                                  hl + ((k + 2) % CONV_SLOTS) * PC};
-    f32x4 acc[MW][NB];
 #pragma unroll
     for (int t = 0; t < MW; ++t)
 #pragma unroll
@@ -220,18 +247,28 @@ __global__ void __launch_bounds__(512, 2) k_conv_lds(ConvArgs a) {
 #pragma unroll
         for (int b = 0; b < NB; ++b)
           acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[b], pv[t], acc[t][b], 0, 0, 0);
+      // the last plane's epilogue, a fragment every third tap: waves 0..3 in the
+      // first half of the taps, waves 4..7 in the second
+      if (tap % 3 == 2 && tap / 3 < MW * NB) {
+        if (pending && half == 0) finish(k - 1, tap / 3);
+      }
+      if (tap % 3 == 2 && tap / 3 >= 4 && tap / 3 - 4 < MW * NB) {
+        if (pending && half == 1) finish(k - 1, tap / 3 - 4);
+      }
     }
-    if (row_ok) {
-      const long prow = ((long)(x0 + k) * n1 + i1b + w) * n2 + z0;
 #pragma unroll
-      for (int t = 0; t < MW; ++t)
+    for (int t = 0; t < MW; ++t)
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-          conv_epilogue<EPI, COUT>(a, acc[t][b], bias[b], prow + 16 * (half * MW + t) + m, 16 * b + 4 * g);
-    }
+      for (int b = 0; b < NB; ++b) done[t][b] = acc[t][b];
     // the slot of plane k + 2 held plane k - 2, which no wave reads any more
-    if (more) store_plane(k + 2, pre);
-    __syncthreads();
+    if (more) {
+      store_plane(k + 2, pre);
+      __syncthreads();
+    }
+  }
+  if (row_ok) {
+#pragma unroll
+    for (int i = 0; i < MW * NB; ++i) finish(nx - 1, i);
   }
 }
 
@@ -249,8 +286,9 @@ template <int CIN, int COUT, int EPI, int MT> int conv_go(const ConvArgs& a, hip
   if constexpr (CIN == 32) {
     return conv_lds_go<COUT, EPI, MT>(a, s);
   } else {
-    const long segs = (long)a.n0 * a.n1 * (a.n2 / (16 * MT));
-    hipLaunchKernelGGL((k_conv8<COUT, EPI, MT>), dim3((unsigned)((segs + 3) / 4)), dim3(256), 0, s, a);
+    const long nblk =
+        (long)((a.n0 + CONV8_XP - 1) / CONV8_XP) * ((a.n1 + CONV_ROWS - 1) / CONV_ROWS) * (a.n2 / (16 * MT));
+    hipLaunchKernelGGL((k_conv8<COUT, EPI, MT>), dim3((unsigned)nblk), dim3(256), 0, s, a);
     return 0;
   }
 }
