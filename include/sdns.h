@@ -93,6 +93,18 @@ int sdns_mul_minus_i(sdns_plan* plan, void* out, const void* a, size_t n);
  *    (add_linear, VV.py:108-113), in place on rhs */
 int sdns_cross2_k_over_k2(sdns_plan* plan, void* u_hat, const void* w_hat);
 int sdns_add_linear(sdns_plan* plan, void* rhs, const void* w_hat, double nu, const void* source);
+/* Whether the fused stages below (and of MHD) reach this box: 1, or 0 where an
+ * array of three components spans more than 2^31 bytes; the step-by-step
+ * entries serve those. */
+int sdns_fused_stages(const sdns_plan* plan);
+/* The whole VV right-hand side (ComputeRHS, VV.py:117-146) in the five dealiased
+ * passes: velocity 1j*((K/K^2) x w_hat) formed where the first pass reads w_hat,
+ * u x w, cross2, Nyquist mask, -nu*K2*w_hat and + source (NULL: none) in the
+ * last.  rhs may not alias w_hat. */
+int sdns_vv_rhs(sdns_plan* plan, const void* w_hat, void* rhs, double nu, const void* source);
+/* nsteps classical RK4 steps (integrators.py:149-159) of w_hat in place, the
+ * stage updates in the last pass of each stage. */
+int sdns_vv_rk4_steps(sdns_plan* plan, void* w_hat, const double* dts, int nsteps, double nu, const void* source);
 /* The VV right-hand side after the convection passes, in one launch:
  * rhs = 1j*(K x v_hat) (Conv, VV.py:104-106), Nyquist planes zeroed when the
  * plan masks them (VV.py:143-144), then rhs -= nu*K2*w_hat and rhs += source
@@ -132,6 +144,19 @@ int sdns_backward_dealiased(sdns_plan* plan, const void* u_hat, void* u, int nco
 int sdns_forward_dealiased(sdns_plan* plan, const void* u, void* u_hat, int ncomp);
 int sdns_elsasser_products(sdns_plan* plan, void* zz, const void* ub, size_t npoints);
 int sdns_set_elsasser(sdns_plan* plan, void* c_hat, const void* zz_hat);
+/* The whole MHD right-hand side (ComputeRHS, MHD.py:150-176) of ub_hat[6] in the
+ * dealiased passes: the nine products are formed in the z pass, and the last
+ * pass adds up set_Elsasser, the Nyquist mask, pressure and nu on U and eta on
+ * B.  p_hat may be NULL.  workspace: sdns_mhd_workspace_bytes bytes (0: the box
+ * is beyond the fused stages), 256-byte aligned, on the plan's stream like the
+ * plan's own.  rhs may not alias ub_hat. */
+size_t sdns_mhd_workspace_bytes(const sdns_plan* plan);
+int sdns_mhd_rhs(sdns_plan* plan, const void* ub_hat, void* rhs, double nu, double eta, void* p_hat, void* workspace,
+                 size_t bytes);
+/* nsteps classical RK4 steps of ub_hat in place; p_hat (NULL: none) receives the
+ * last stage's pressure. */
+int sdns_mhd_rk4_steps(sdns_plan* plan, void* ub_hat, const double* dts, int nsteps, double nu, double eta, void* p_hat,
+                       void* workspace, size_t bytes);
 /* The Standard, Divergence and Skewed convection forms of the NS solver
  * (spectralDNS/solvers/NS.py:138-199), any dealiasing (physical arrays on the
  * plan's grid, or on the padded grid for the 3/2 rule):

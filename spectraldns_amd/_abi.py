@@ -35,6 +35,13 @@ _SIGS = {
     "sdns_cross2_k_over_k2": (ctypes.c_int, [_P, _P, _P]),
     "sdns_add_linear": (ctypes.c_int, [_P, _P, _P, ctypes.c_double, _P]),
     "sdns_vv_rhs_tail": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_double, _P]),
+    "sdns_fused_stages": (ctypes.c_int, [_P]),
+    "sdns_vv_rhs": (ctypes.c_int, [_P, _P, _P, ctypes.c_double, _P]),
+    "sdns_vv_rk4_steps": (ctypes.c_int, [_P, _P, ctypes.POINTER(ctypes.c_double), ctypes.c_int, ctypes.c_double, _P]),
+    "sdns_mhd_workspace_bytes": (ctypes.c_size_t, [_P]),
+    "sdns_mhd_rhs": (ctypes.c_int, [_P, _P, _P, ctypes.c_double, ctypes.c_double, _P, _P, ctypes.c_size_t]),
+    "sdns_mhd_rk4_steps": (ctypes.c_int, [_P, _P, ctypes.POINTER(ctypes.c_double), ctypes.c_int, ctypes.c_double,
+                                          ctypes.c_double, _P, _P, ctypes.c_size_t]),
     "sdns_dealias_truncate": (ctypes.c_int, [_P, _P, _P]),
     "sdns_backward_dealiased": (ctypes.c_int, [_P, _P, _P, ctypes.c_int]),
     "sdns_forward_dealiased": (ctypes.c_int, [_P, _P, _P, ctypes.c_int]),
@@ -440,6 +447,65 @@ class Plan:
                                                _ptr(diag) if diag is not None else None,
                                                _ptr(p_hat) if p_hat is not None else None))
         return u_hat
+
+    # VV and MHD with fused stages (sdns_fused_stages)
+    @property
+    def fused_stages(self):
+        return bool(self._lib.sdns_fused_stages(self._h))
+
+    def vv_rhs(self, w_hat, rhs, nu, source=None):
+        self._spec(w_hat, 3, "w_hat")
+        self._spec(rhs, 3, "rhs")
+        if source is not None:
+            self._spec(source, 3, "Source")
+        self._sync_stream()
+        _check(self._lib.sdns_vv_rhs(self._h, _ptr(w_hat), _ptr(rhs), float(nu),
+                                     _ptr(source) if source is not None else None))
+        return rhs
+
+    def vv_rk4_steps(self, w_hat, dts, nu, source=None):
+        self._spec(w_hat, 3, "w_hat")
+        if source is not None:
+            self._spec(source, 3, "Source")
+        n = len(dts)
+        arr = (ctypes.c_double * max(n, 1))(*[float(d) for d in dts])
+        self._sync_stream()
+        _check(self._lib.sdns_vv_rk4_steps(self._h, _ptr(w_hat), arr, n, float(nu),
+                                           _ptr(source) if source is not None else None))
+        return w_hat
+
+    def _mhd_workspace(self):
+        """(pointer, bytes) of the fused MHD stages' workspace, allocated on first use."""
+        import torch
+        if getattr(self, "_mhd_ws", None) is None:
+            n = self._lib.sdns_mhd_workspace_bytes(self._h)
+            self._mhd_ws = torch.empty(n + 256, dtype=torch.uint8, device=self.device)
+        base = self._mhd_ws.data_ptr()
+        off = (-base) % 256
+        return _P(base + off), self._mhd_ws.numel() - 256
+
+    def mhd_rhs(self, ub_hat, rhs, nu, eta, p_hat=None):
+        self._spec(ub_hat, 6, "ub_hat")
+        self._spec(rhs, 6, "rhs")
+        if p_hat is not None:
+            self._spec(p_hat, 1, "P_hat")
+        self._sync_stream()
+        ws, nbytes = self._mhd_workspace()
+        _check(self._lib.sdns_mhd_rhs(self._h, _ptr(ub_hat), _ptr(rhs), float(nu), float(eta),
+                                      _ptr(p_hat) if p_hat is not None else None, ws, nbytes))
+        return rhs
+
+    def mhd_rk4_steps(self, ub_hat, dts, nu, eta, p_hat=None):
+        self._spec(ub_hat, 6, "ub_hat")
+        if p_hat is not None:
+            self._spec(p_hat, 1, "P_hat")
+        n = len(dts)
+        arr = (ctypes.c_double * max(n, 1))(*[float(d) for d in dts])
+        self._sync_stream()
+        ws, nbytes = self._mhd_workspace()
+        _check(self._lib.sdns_mhd_rk4_steps(self._h, _ptr(ub_hat), arr, n, float(nu), float(eta),
+                                            _ptr(p_hat) if p_hat is not None else None, ws, nbytes))
+        return ub_hat
 
     def lincomb(self, out, xs, cs):
         """out = cs[0]*xs[0] + cs[1]*xs[1] + ... over state-shaped arrays (in place

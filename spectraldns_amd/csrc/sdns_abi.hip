@@ -525,6 +525,133 @@ template <typename Rt> int convection(sdns_plan* p, const void* u, void* rhs, co
   return 0;
 }
 
+// ---------------------------------------------------------------- VV and MHD, fused stages
+// Whether the stage kernels of the VV and MHD solvers reach this box's arrays.
+bool fused_stages(const sdns_plan* p) {
+  return p->precision == SDNS_DOUBLE ? p5b_fits<double>(p->M[0], p->N[0], p->N[1], p->Nh, p->nkyo, p->nkzop)
+                                     : p5b_fits<float>(p->M[0], p->N[0], p->N[1], p->Nh, p->nkyo, p->nkzop);
+}
+
+// One right-hand side of the vorticity w and its stage (mode) into a's arrays.
+template <typename Rt> int vv_stage(sdns_plan* p, const void* w, int mode, const P5Args<Rt>& a) {
+  P1Args<Rt> a1 = p1_args<Rt>(p, w);
+  a1.w = w;
+  a1.ky = (const Rt*)p->ktab[1];
+  a1.kz = (const Rt*)p->ktab[2];
+  a1.curl_inv = 1;
+  int rc;
+  if ((rc = conv_passes<Rt>(p, a1))) return rc;
+  if (launch_p5vv<Rt>(p->M[0], mode, a, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", p->M[0]);
+  return 0;
+}
+template <typename Rt> int vv_rhs(sdns_plan* p, const void* w, void* rhs, double nu, const void* src) {
+  P5Args<Rt> a = p5_args<Rt>(p, nu);
+  a.u = const_cast<void*>(w); a.rhs = rhs; a.source = src;
+  return vv_stage<Rt>(p, w, P5_RHS, a);
+}
+template <typename Rt> int vv_rk4_steps(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* src) {
+  using RK = RkStage<Rt>;
+  for (int s = 0; s < nsteps; ++s)
+    for (int rk = 0; rk < 4; ++rk) {
+      P5Args<Rt> a = p5_args<Rt>(p, nu);
+      RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], w, p->st);
+      a.source = src;
+      const int rc = vv_stage<Rt>(p, rk == 0 ? w : p->st[rk - 1], RK::mode(rk), a);
+      if (rc) return rc;
+    }
+  return 0;
+}
+
+// Workspace of the fused MHD stages: W1/W3, W2/W4, and the B halves of the
+// three stage states (the U halves are the plan's).
+struct MhdWs {
+  size_t a, b, total;
+  explicit MhdWs(const sdns_plan* p) {
+    const size_t e = p->esz, M0 = p->M[0], M1 = p->M[1];
+    a = align256(std::max(6 * M0 * p->nky * p->nkzp, 9 * M0 * M1 * p->nkzop) * e);
+    b = align256(std::max(6 * M0 * M1 * p->nkzp, 9 * M0 * p->nkyo * p->nkzop) * e);
+    total = a + b + 3 * p->szS;
+  }
+};
+// One right-hand side of the state (u, b) and its stage (mode) into x's arrays.
+template <typename Rt> int mhd_stage(sdns_plan* p, const void* u, const void* b, int mode, MhdXArgs<Rt> x, char* ws) {
+  const MhdWs L(p);
+  const int M0 = p->M[0], M1 = p->M[1];
+  char *A = ws, *B = ws + L.a;
+  P1Args<Rt> a1 = p1_args<Rt>(p, u);
+  a1.w = b; a1.w1 = A;
+  tstart(p, 0);
+  if (launch_p1<Rt>(M0, p->var[0], a1, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", M0);
+  tstop(p);
+  StridedArgs<Rt> a2 = p2_given_args<Rt>(p);
+  a2.in = A; a2.out = B;
+  tstart(p, 1);
+  if (launch_strided<Rt>(M1, p->var[1], +1, 6, a2, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "y length %d", M1);
+  tstop(p);
+  const P3Args<Rt> n = p3_args<Rt>(p);
+  const MhdZArgs<Rt> z{B, A, n.tw, n.rtw, n.nkz, n.nkzp, n.nkzo, n.nkzop, n.L};
+  tstart(p, 2);
+  if (launch_mhd_z<Rt>(p->n2h, z, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "z length %d", p->M[2]);
+  tstop(p);
+  StridedArgs<Rt> a4 = p4_args<Rt>(p);
+  a4.in = A; a4.out = B;
+  tstart(p, 3);
+  if (launch_strided<Rt>(M1, p->var[3], -1, 9, a4, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "y length %d", M1);
+  tstop(p);
+  x.w4 = B;
+  tstart(p, 4);
+  if (launch_mhd_x<Rt>(M0, mode, x, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", M0);
+  tstop(p);
+  return 0;
+}
+template <typename Rt> MhdXArgs<Rt> mhd_x_args(const sdns_plan* p, double nu, double eta) {
+  const P5Args<Rt> a = p5_args<Rt>(p, nu);
+  MhdXArgs<Rt> x{};
+  x.tw = a.tw; x.kx = a.kx; x.ky = a.ky; x.kz = a.kz;
+  x.N0 = a.N0; x.N1 = a.N1; x.Nh = a.Nh; x.N2 = a.N2; x.x = a.x;
+  x.y_neg = a.y_neg; x.y_pos = a.y_pos; x.nkzo = a.nkzo; x.nkzop = a.nkzop; x.mask_nyquist = a.mask_nyquist;
+  x.visc[0] = (Rt)nu; x.visc[1] = (Rt)eta; x.scale = a.scale; x.Q = a.Q;
+  return x;
+}
+size_t mhd_half(const sdns_plan* p) { return 3ull * p->N[0] * p->N[1] * p->Nh * p->esz; }
+template <typename Rt> int mhd_rhs(sdns_plan* p, const void* ub, void* rhs, double nu, double eta, void* ph, char* ws) {
+  MhdXArgs<Rt> x = mhd_x_args<Rt>(p, nu, eta);
+  const size_t half = mhd_half(p);
+  for (int h = 0; h < 2; ++h) {
+    x.u[h] = (char*)const_cast<void*>(ub) + h * half;
+    x.out[h] = (char*)rhs + h * half;
+  }
+  x.phat = ph;
+  return mhd_stage<Rt>(p, x.u[0], x.u[1], P5_RHS, x, ws);
+}
+template <typename Rt> int mhd_rk4_steps(sdns_plan* p, void* ub, const double* dts, int nsteps, double nu, double eta,
+                                         void* ph, char* ws) {
+  using RK = RkStage<Rt>;
+  const size_t half = mhd_half(p);
+  const MhdWs L(p);
+  char* st[2][3];
+  for (int k = 0; k < 3; ++k) {
+    st[0][k] = p->st[k];
+    st[1][k] = ws + L.a + L.b + k * p->szS;
+  }
+  for (int s = 0; s < nsteps; ++s)
+    for (int rk = 0; rk < 4; ++rk) {
+      MhdXArgs<Rt> x = mhd_x_args<Rt>(p, nu, eta);
+      const void* in[2];
+      for (int h = 0; h < 2; ++h) {
+        P5Args<Rt> a{};
+        RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], (char*)ub + h * half, st[h]);
+        x.u[h] = a.u; x.s[h] = a.s; x.out[h] = a.out; x.b1[h] = a.b1; x.b2[h] = a.b2;
+        x.adt = a.adt; x.bdt = a.bdt;
+        in[h] = rk == 0 ? a.u : a.s;
+      }
+      x.phat = rk == 3 && s == nsteps - 1 ? ph : nullptr;
+      const int rc = mhd_stage<Rt>(p, in[0], in[1], RK::mode(rk), x, ws);
+      if (rc) return rc;
+    }
+  return 0;
+}
+
 template <typename Rt> EwArgs<Rt> ew_args(sdns_plan* p);
 
 // out = a.u + a.ds a.d, a whole state.
@@ -1286,6 +1413,57 @@ int sdns_rk4_steps_source(sdns_plan* p, void* u, void* u_lo, const double* dts, 
   if (rc) return rc;
   rc = p->precision == SDNS_DOUBLE ? rk4_steps<double>(p, u, nullptr, dts, nsteps, nu, diag, ph, source)
                                    : rk4_steps<float>(p, u, u_lo, dts, nsteps, nu, diag, ph, source);
+  return rc ? rc : check_launch();
+}
+
+// ---------------------------------------------------------------- VV and MHD, fused
+int sdns_fused_stages(const sdns_plan* p) { return p && fused_stages(p) ? 1 : 0; }
+
+int sdns_vv_rhs(sdns_plan* p, const void* w, void* rhs, double nu, const void* source) {
+  if (!p || !w || !rhs || rhs == w) return fail(SDNS_ERR_INVALID, "bad argument");
+  if (!fused_stages(p)) return fail(SDNS_ERR_UNSUPPORTED, "box beyond the fused stages");
+  int rc = ensure_workspace(p);
+  if (rc) return rc;
+  rc = p->precision == SDNS_DOUBLE ? vv_rhs<double>(p, w, rhs, nu, source) : vv_rhs<float>(p, w, rhs, nu, source);
+  return rc ? rc : check_launch();
+}
+
+int sdns_vv_rk4_steps(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* source) {
+  if (!p || !w || (!dts && nsteps > 0) || nsteps < 0) return fail(SDNS_ERR_INVALID, "bad argument");
+  if (source && source == w) return fail(SDNS_ERR_INVALID, "the source may not alias the state");
+  if (!fused_stages(p)) return fail(SDNS_ERR_UNSUPPORTED, "box beyond the fused stages");
+  int rc = ensure_workspace(p);
+  if (rc) return rc;
+  rc = p->precision == SDNS_DOUBLE ? vv_rk4_steps<double>(p, w, dts, nsteps, nu, source)
+                                   : vv_rk4_steps<float>(p, w, dts, nsteps, nu, source);
+  return rc ? rc : check_launch();
+}
+
+size_t sdns_mhd_workspace_bytes(const sdns_plan* p) { return p && fused_stages(p) ? MhdWs(p).total : 0; }
+
+static int mhd_check(sdns_plan* p, void* ws, size_t bytes) {
+  if (!fused_stages(p)) return fail(SDNS_ERR_UNSUPPORTED, "box beyond the fused stages");
+  if (!ws || bytes < MhdWs(p).total || ((uintptr_t)ws & 255))
+    return fail(SDNS_ERR_INVALID, "MHD workspace: %zu bytes, 256-byte aligned", MhdWs(p).total);
+  return ensure_workspace(p);
+}
+
+int sdns_mhd_rhs(sdns_plan* p, const void* ub, void* rhs, double nu, double eta, void* phat, void* ws, size_t bytes) {
+  if (!p || !ub || !rhs || rhs == ub) return fail(SDNS_ERR_INVALID, "bad argument");
+  int rc = mhd_check(p, ws, bytes);
+  if (rc) return rc;
+  rc = p->precision == SDNS_DOUBLE ? mhd_rhs<double>(p, ub, rhs, nu, eta, phat, (char*)ws)
+                                   : mhd_rhs<float>(p, ub, rhs, nu, eta, phat, (char*)ws);
+  return rc ? rc : check_launch();
+}
+
+int sdns_mhd_rk4_steps(sdns_plan* p, void* ub, const double* dts, int nsteps, double nu, double eta, void* phat,
+                       void* ws, size_t bytes) {
+  if (!p || !ub || (!dts && nsteps > 0) || nsteps < 0) return fail(SDNS_ERR_INVALID, "bad argument");
+  int rc = mhd_check(p, ws, bytes);
+  if (rc) return rc;
+  rc = p->precision == SDNS_DOUBLE ? mhd_rk4_steps<double>(p, ub, dts, nsteps, nu, eta, phat, (char*)ws)
+                                   : mhd_rk4_steps<float>(p, ub, dts, nsteps, nu, eta, phat, (char*)ws);
   return rc ? rc : check_launch();
 }
 

@@ -133,6 +133,31 @@ __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, c
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = caxpy(v[e], a.ds, d[e]);
+  } else if (a.curl_inv && yb < 3) {
+    // velocity component `comp` of the vorticity: i (o_j w_k - o_k w_j), o = K / K^2,
+    // K^2 = 0 taken as 1 (solvers/VV.py:71-72)
+    const int cj = (comp + 1) % 3, ck = (comp + 2) % 3;
+    const C* __restrict__ B = (const C*)a.w + (valid ? (long)iy * a.Nh + kzi : 0);
+    const C *Wj = B + (long)cj * a.N0 * plane, *Wk = B + (long)ck * a.N0 * plane;
+    const Rt K1 = a.ky[valid ? iy : 0], K2 = a.kz[valid ? kzi : 0];
+    C d[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int r = bin_row(t + P * e, M, a.x);
+      v[e] = (valid && r >= 0) ? Wk[r * plane] : czero<C>();
+      d[e] = (valid && r >= 0) ? Wj[r * plane] : czero<C>();
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int r = bin_row(t + P * e, M, a.x);
+      const Rt K0 = a.kx[r >= 0 ? r : 0];
+      Rt k2 = K0 * K0;
+      k2 += K1 * K1;
+      k2 += K2 * K2;
+      const Rt den = k2 == Rt(0) ? Rt(1) : k2;
+      const Rt oj = (cj == 0 ? K0 : (cj == 1 ? K1 : K2)) / den, ok = (ck == 0 ? K0 : (ck == 1 ? K1 : K2)) / den;
+      v[e] = cmuli<1>(mk<C>(oj * v[e].x - ok * d[e].x, oj * v[e].y - ok * d[e].y));
+    }
   } else {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -885,6 +910,14 @@ template <int TH> __device__ __forceinline__ void p5_partials(double esum, doubl
   }
 }
 
+// u + ((x1 - u) + 2 (x2 - u) + (x3 - u)) / 3 + adt r (KEEP_STATES).
+template <typename C, typename Rt = decltype(C::x)>
+__device__ __forceinline__ C rk_add_states(C u, C x1, C x2, C x3, Rt adt, C r) {
+  constexpr Rt third = Rt(1) / Rt(3);
+  const C d = mk<C>(third * (((x1.x - u.x) + (x3.x - u.x)) + Rt(2) * (x2.x - u.x)),
+                    third * (((x1.y - u.y) + (x3.y - u.y)) + Rt(2) * (x2.y - u.y)));
+  return cadd(u, caxpy(d, adt, r));
+}
 // The new state of the last RK4 stage from u, the kept stage arrays x1, x2, x3
 // and the stage's right-hand side r (see P5Args).  COMP: the state is the pair
 // u + lo, summed term by term with TwoSum and renormalised (hi = fl(h + l), lo
@@ -896,10 +929,7 @@ __device__ __forceinline__ cx<Rt> rk_last(const P5Args<Rt>& a, cx<Rt> u, cx<Rt> 
   if constexpr (KEEP == KEEP_SUM) {
     return caxpy(x1, a.adt, r);
   } else if constexpr (KEEP == KEEP_STATES) {
-    constexpr Rt third = Rt(1) / Rt(3);
-    const C d = mk<C>(third * (((x1.x - u.x) + (x3.x - u.x)) + Rt(2) * (x2.x - u.x)),
-                      third * (((x1.y - u.y) + (x3.y - u.y)) + Rt(2) * (x2.y - u.y)));
-    return cadd(u, caxpy(d, a.adt, r));
+    return rk_add_states(u, x1, x2, x3, a.adt, r);
   } else if constexpr (!COMP) {
     return caxpy(caxpy(caxpy(caxpy(u, a.adt, x1), a.a12, x2), a.a12, x3), a.adt, r);
   } else {
@@ -1122,13 +1152,16 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
 // The host checks that the three components of a state array and of W4 span
 // at most BUF_OOB bytes (p5b_fits); larger boxes run p5_body.  The per-mode
 // arithmetic is p5_body's.
-template <typename Rt, int M, int E, int MODE, bool PAD, bool COMP, int T>
+// VV: the velocity-vorticity right-hand side instead (solvers/VV.py:104-146): the
+// state is the vorticity, the convection term is i K x F(u x w) and there is no
+// pressure.
+template <typename Rt, int M, int E, int MODE, bool PAD, bool COMP, int T, int KEEP = rk_keep<Rt>(PAD, COMP),
+          bool VV = false>
 __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* lds, const cx<Rt>* tw) {
   using C = cx<Rt>;
   static_assert(!PAD || (M % 3 == 0 && E % 3 == 0), "3/2-rule rows");
   constexpr int P = M / E, TH = T * P, E3 = E / 3, NK = PAD ? 2 * E3 : E;
   constexpr int CS = (int)sizeof(C);
-  constexpr int KEEP = rk_keep<Rt>(PAD, COMP);
   constexpr bool SUM = KEEP == KEEP_SUM;
   constexpr int NL = p5_arrays(MODE, COMP, KEEP);  // u; s; b1; b2; lo (KEEP_SUM, stage 3: s, b1)
   constexpr int G = (NL > 2 || E * CS >= 128 || NK % 2) ? 1 : 2;
@@ -1235,6 +1268,12 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
         // P_hat = sum_i rhs_i K_i/K^2 ; rhs_i -= P_hat K_i ; rhs -= (nu K^2) u_hat  (NS.py:208-215)
         C ph = mk<C>(r[0].x * o0 + r[1].x * o1, r[0].y * o0 + r[1].y * o1);
         ph = mk<C>(ph.x + r[2].x * o2, ph.y + r[2].y * o2);
+        if constexpr (VV) {
+          const C v0 = r[0], v1 = r[1], v2 = r[2];
+          r[0] = cmuli<1>(mk<C>(K1 * v2.x - K2c * v1.x, K1 * v2.y - K2c * v1.y));
+          r[1] = cmuli<1>(mk<C>(K2c * v0.x - Kv[0] * v2.x, K2c * v0.y - Kv[0] * v2.y));
+          r[2] = cmuli<1>(mk<C>(Kv[0] * v1.x - K1 * v0.x, Kv[0] * v1.y - K1 * v0.y));
+        }
         const Rt z = a.nu * k2;
         double v[6];
 #pragma unroll
@@ -1243,7 +1282,8 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
           const C u = d[0][i];
           const C s = d[NL > 1 ? 1 : 0][i];
           const C st = NL == 1 || (SUM && MODE == P5_RK3) ? u : (KEEP == KEEP_RHS ? caxpy(u, a.sdt, s) : s);
-          C x = mk<C>(r[i].x - ph.x * Kv[i], r[i].y - ph.y * Kv[i]);
+          C x = r[i];
+          if constexpr (!VV) x = mk<C>(x.x - ph.x * Kv[i], x.y - ph.y * Kv[i]);
           x = mk<C>(x.x - z * st.x, x.y - z * st.y);
           x = cadd(x, d[NL][i]);  // rhs += Source (NS.py:256-258), every mode
           const int o = (i * fs + eo) * CS;
@@ -1264,7 +1304,7 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
           }
           buf_store_so_nt<C>(x, ro, so, o);
         }
-        if constexpr (MODE == P5_RHS || MODE == P5_RK3) buf_store_so_nt<C>(ph, rph, so, eo * CS);
+        if constexpr (!VV && (MODE == P5_RHS || MODE == P5_RK3)) buf_store_so_nt<C>(ph, rph, so, eo * CS);
         if constexpr (MODE == P5_RK3) energy_terms(v, Kv[0], K1, K2c, wz, esum, osum);
       }
       if (j0 + G < NK) {
@@ -1321,6 +1361,222 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, 
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
   p5b_body<Rt, M, E, MODE, PAD, COMP, T>(a, tile, lds, tw);
+}
+
+// The VV stages (p5b_body).
+template <typename Rt, int M, int E, int MODE, bool PAD, int D = 1>
+__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, E, PAD>())) k_p5vv(P5Args<Rt> a) {
+  using C = cx<Rt>;
+  constexpr int T = SCfg<Rt, M, E>::T / D;
+  __shared__ C lds[M * T];
+  __shared__ C tw[M];
+  const int tile = xcd_tile((a.Q + T - 1) / T);
+  if (tile < 0) return;
+  table_to_lds(tw, (const C*)a.tw, M);
+  p5b_body<Rt, M, E, MODE, PAD, false, T, KEEP_STATES, true>(a, tile, lds, tw);
+}
+
+// ------------------------------------------------------------------ MHD
+// The right-hand sides of the Elsasser form (solvers/MHD.py:91-133) are
+//   U_i = -i sum_j K_j F(S_ij),  S_ij = u_i u_j - b_i b_j  (symmetric)
+//   B_i = +i sum_j K_j F(A_ij),  A_ij = u_i b_j - u_j b_i  (antisymmetric):
+// with z0 = u + b and z1 = u - b, z0_i z1_j + z0_j z1_i = 2 S_ij and
+// z0_j z1_i - z0_i z1_j = 2 A_ij.  Six fields of S feed U alone and three of A
+// feed B alone, so the x pass handles the two halves in separate blocks.
+//
+// z pass: the six real lines of u and b stay in registers, and each of the
+// nine products is formed, transformed and written from there.  Physical space
+// never touches HBM: as separate launches the same step wrote and read 6 + 9
+// physical fields.
+__device__ constexpr int mhd_i(int f) { return f < 3 ? 0 : (f < 5 ? 1 : (f == 5 ? 2 : (f < 8 ? 0 : 1))); }
+__device__ constexpr int mhd_j(int f) { return f < 3 ? f : (f < 5 ? f - 2 : (f == 5 ? 2 : (f < 8 ? f - 5 : 2))); }
+template <typename Rt, int n, int E>
+__global__ void __launch_bounds__((ZCfg<Rt, n, E>::THREADS), (occ_for(7 * E + stage_k(n, n / E), esz_of<Rt>()))) k_mhd_z(MhdZArgs<Rt> a) {
+  using C = cx<Rt>;
+  using Cfg = ZCfg<Rt, n, E>;
+  constexpr int P = Cfg::P, LPB = Cfg::LPB;
+  constexpr bool WL = 64 % P == 0;  // a line's threads share one wave
+  using Fi = LineFFT<Rt, n, E, +1, WL>;
+  using Ff = LineFFT<Rt, n, E, -1, WL>;
+  __shared__ C lds[LPB * zslot(n, P)];
+  __shared__ C tw[n], rtw[n];
+  table_to_lds(tw, (const C*)a.tw, n);
+  table_to_lds(rtw, (const C*)a.rtw, n);
+  __syncthreads();
+  const int t = threadIdx.x % P, l = threadIdx.x / P;
+  const int line0 = blockIdx.x * LPB;
+  C* my = lds + l * zslot(n, P);
+  const int nl = min(LPB, a.L - line0);
+  const long ifield = (long)a.L * a.nkzp;
+  const C* inb = (const C*)a.w2 + (long)line0 * a.nkzp;
+  const long ibytes = (long)nl * a.nkzp * (long)sizeof(C);
+  const int ibase = l * a.nkzp * (int)sizeof(C);
+  LineStage<Rt, n, P> st;
+  st.load_buf(buf_rsrc(inb, ibytes), ibase, a.nkz, t);
+  C z[6][E];
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    st.store(my, t);
+    lds_barrier<WL>();
+    c2r_pre_lds<Rt, n, E>(z[f], my, rtw, t);
+    lds_barrier<WL>();
+    if (f < 5) st.load_buf(buf_rsrc(inb + (f + 1) * ifield, ibytes), ibase, a.nkz, t);  // in flight during the FFT
+    Fi::run(z[f], t, my, 1, tw);
+  }
+  const long ofield = (long)a.L * a.nkzop;
+  C* outb = (C*)a.w3 + (long)line0 * a.nkzop;
+  const long obytes = (long)nl * a.nkzop * (long)sizeof(C);
+  const int obase = l * a.nkzop * (int)sizeof(C);
+#pragma unroll
+  for (int f = 0; f < 9; ++f) {
+    const int i = mhd_i(f), j = mhd_j(f);
+    C w[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const C ui = z[i][e], uj = z[j][e], bi = z[3 + i][e], bj = z[3 + j][e];
+      w[e] = f < 6 ? mk<C>(ui.x * uj.x - bi.x * bj.x, ui.y * uj.y - bi.y * bj.y)
+                   : mk<C>(ui.x * bj.x - uj.x * bi.x, ui.y * bj.y - uj.y * bi.y);
+    }
+    Ff::run(w, t, my, 1, tw);
+    r2c_post_buf<Rt, n, E, WL>(w, my, buf_rsrc(outb + f * ofield, obytes), obase, a.nkzo, rtw, t);
+  }
+}
+
+// x-forward pass of U (blockIdx.y = 0, six fields) or B (1, three fields): each
+// transformed product is added into the three sums as soon as its lines are
+// done, so that three lines of sums, one line in work and the next one's loads
+// are live; then mask, pressure (U) and diffusion (MHD.py:135-176) and the RK4
+// stage as in p5b_body with KEEP_STATES.  Buffer descriptors span three fields
+// or components each.
+template <typename Rt, int M, int E, int MODE, bool PAD>
+__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz_of<Rt>()))) k_mhd_x(MhdXArgs<Rt> a) {
+  using C = cx<Rt>;
+  static_assert(!PAD || (M % 3 == 0 && E % 3 == 0), "3/2-rule rows");
+  constexpr int T = SCfg<Rt, M, E>::T;
+  constexpr int P = M / E, E3 = E / 3, NK = PAD ? 2 * E3 : E;
+  constexpr int CS = (int)sizeof(C);
+  using F = LineFFT<Rt, M, E, -1>;
+  __shared__ C lds[M * T];
+  __shared__ C tw[M];
+  const int tile = xcd_tile((a.Q + T - 1) / T);
+  if (tile < 0) return;
+  table_to_lds(tw, (const C*)a.tw, M);
+  const int c = threadIdx.x % T, t = threadIdx.x / T;
+  const int q = tile * T + c;
+  const bool valid = q < a.Q;
+  const int qq = valid ? q : 0;
+  const int iy = qq / a.Nh, kz = qq - iy * a.Nh;
+  const int ky = iy < a.N1 / 2 ? iy : iy - a.N1;
+  const int nkyo = a.y_neg + a.y_pos + 1;
+  const bool colconv = valid && ky >= -a.y_neg && ky <= a.y_pos && kz < a.nkzo;
+  const int kyc = ky >= 0 ? ky : nkyo + ky;
+  const int wrow = nkyo * a.nkzop, wfield = M * wrow;
+  const int wo = colconv ? (t * wrow + kyc * a.nkzop + kz) * CS : BUF_OOB;
+  const int h = blockIdx.y;  // U or B
+  const int f0 = h ? 6 : 0, nf = h ? 3 : 6;
+  auto load_field = [&](C(&d)[E], int f) {
+    const auto rw = buf_rsrc((const C*)a.w4 + (long)(f / 3) * 3 * wfield, 3L * wfield * CS);
+#pragma unroll
+    for (int e = 0; e < E; ++e) d[e] = buf_load_so<C>(rw, wo, ((f % 3) * wfield + P * e * wrow) * CS);
+  };
+  const Rt K1 = a.ky[iy], K2c = a.kz[kz];
+  Rt k0[NK];
+#pragma unroll
+  for (int j = 0; j < NK; ++j) k0[j] = a.kx[t + P * j];
+  C S[3][NK];
+#pragma unroll
+  for (int f = 0; f < 3; ++f)
+#pragma unroll
+    for (int r = 0; r < NK; ++r) S[f][r] = czero<C>();
+  C X[E], Y[E];
+  load_field(X, f0);
+  __syncthreads();
+  C* line = lds + c;
+  // S[i] += +-K_j v, S[j] += +-K_i v of the field f
+  auto add = [&](auto fc) {
+    constexpr int f = decltype(fc)::value, i = mhd_i(f), j = mhd_j(f);
+    if (f + 1 < f0 + nf) load_field(Y, f + 1);  // in flight during the FFT
+    F::run(X, t, line, T, tw);
+#pragma unroll
+    for (int r = 0; r < NK; ++r) {
+      const int e = (!PAD || r < E3) ? r : r + E3;
+      const C v = cscale(X[e], a.scale);
+      const Rt Kv[3] = {k0[r], K1, K2c};
+      S[i][r] = caxpy(S[i][r], Kv[j], v);
+      if constexpr (i != j) S[j][r] = caxpy(S[j][r], f < 6 ? Kv[i] : -Kv[i], v);
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) X[e] = Y[e];
+  };
+  if (h == 0) sfor<6>([&](auto fc) { add(fc); });
+  else sfor<3>([&](auto fc) { add(std::integral_constant<int, decltype(fc)::value + 6>{}); });
+  if (!valid) return;
+  const int plane = a.N1 * a.Nh, fs = a.N0 * plane;
+  const long span = 3L * fs * CS;
+  const int so = (t * plane + q) * CS;  // row t of the column
+  const bool colok = colconv && !(a.mask_nyquist && (iy == a.N1 / 2 || kz == a.N2 / 2));
+  const int nyq_ix = a.mask_nyquist ? a.N0 / 2 : -1;
+  const auto rph = buf_rsrc(a.phat, a.phat && h == 0 ? (long)fs * CS : 0L);
+  const auto ru = buf_rsrc(a.u[h], span);
+  const auto rs = buf_rsrc(a.s[h], span);
+  const auto r1 = buf_rsrc(a.b1[h], span);
+  const auto r2 = buf_rsrc(a.b2[h], span);
+  const auto ro = buf_rsrc(MODE == P5_RK3 ? a.u[h] : a.out[h], span);
+  const Rt visc = a.visc[h], press = h == 0 ? Rt(1) : Rt(0);
+  constexpr int NL = p5_arrays(MODE, false, KEEP_STATES);
+  C cur[NL][3], nxt[NL][3];
+  auto load = [&](C(&d)[NL][3], int r) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int o = (i * fs + P * r * plane) * CS;
+      d[0][i] = buf_load_so<C>(ru, so, o);
+      if constexpr (NL > 1) d[1][i] = buf_load_so<C>(rs, so, o);
+      if constexpr (NL > 2) {
+        d[2][i] = buf_load_so<C>(r1, so, o);
+        d[3][i] = buf_load_so<C>(r2, so, o);
+      }
+    }
+  };
+  load(cur, 0);
+#pragma unroll
+  for (int r = 0; r < NK; ++r) {
+    if (r + 1 < NK) load(nxt, r + 1);
+    const int ix = t + P * r;
+    const int eo = P * r * plane;
+    const bool conv = colok & (ix != nyq_ix) & (PAD || ix <= a.x.pos || ix >= a.N0 - a.x.neg);
+    const Rt Kv[3] = {k0[r], K1, K2c};
+    Rt k2 = Kv[0] * Kv[0];
+    k2 += K1 * K1;
+    k2 += K2c * K2c;
+    const Rt den = k2 == Rt(0) ? Rt(1) : k2;
+    // U: -i S, B: +i S
+    C g[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const C v = h ? cmuli<1>(S[i][r]) : cmuli<-1>(S[i][r]);
+      g[i] = conv ? v : czero<C>();
+    }
+    C ph = mk<C>(g[0].x * (Kv[0] / den) + g[1].x * (K1 / den), g[0].y * (Kv[0] / den) + g[1].y * (K1 / den));
+    ph = mk<C>(ph.x + g[2].x * (K2c / den), ph.y + g[2].y * (K2c / den));
+    if constexpr (MODE == P5_RHS || MODE == P5_RK3) buf_store_so_nt<C>(ph, rph, so, eo * CS);
+    const Rt z = visc * k2;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const C u = cur[0][i], st = cur[NL > 1 ? 1 : 0][i];
+      const Rt pk = press * Kv[i];
+      C x = mk<C>(g[i].x - ph.x * pk, g[i].y - ph.y * pk);
+      x = mk<C>(x.x - z * st.x, x.y - z * st.y);
+      if constexpr (MODE == P5_RK0 || MODE == P5_RK12) x = caxpy(u, a.bdt, x);
+      if constexpr (MODE == P5_RK3) x = rk_add_states(u, cur[NL > 2 ? 2 : 0][i], cur[NL > 2 ? 3 : 0][i], st, a.adt, x);
+      buf_store_so_nt<C>(x, ro, so, (i * fs + eo) * CS);
+    }
+    if (r + 1 < NK) {
+#pragma unroll
+      for (int l = 0; l < NL; ++l)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) cur[l][i] = nxt[l][i];
+    }
+  }
 }
 
 }  // namespace sdns

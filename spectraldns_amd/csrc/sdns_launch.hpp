@@ -34,6 +34,13 @@ template <typename Rt> int launch_p5(int M, int var, int mode, const P5Args<Rt>&
     default: return launch_p5<Rt, P5_RK3>(M, var, a, s, nblk);
   }
 }
+// The x-forward stage of the velocity-vorticity solver (KEEP_STATES), and the z
+// and x-forward passes of MHD; boxes within a buffer descriptor's reach
+// (p5b_fits), one schedule per length.
+template <typename Rt> bool p5b_fits(int M, int N0, int N1, int Nh, int nkyo, int nkzop);
+template <typename Rt> int launch_p5vv(int M, int mode, const P5Args<Rt>& a, hipStream_t s);
+template <typename Rt> int launch_mhd_z(int n, const MhdZArgs<Rt>& a, hipStream_t s);
+template <typename Rt> int launch_mhd_x(int M, int mode, const MhdXArgs<Rt>& a, hipStream_t s);
 // dir = -1 forward, +1 inverse
 template <typename Rt> int launch_strided(int M, int var, int dir, int nfields, const StridedArgs<Rt>& a,
                                           hipStream_t s);

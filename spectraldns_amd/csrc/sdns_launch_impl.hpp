@@ -107,11 +107,12 @@ template <typename Rt, int n, int E> void p3c_go(const P3Args<Rt>& a, hipStream_
 // P5 through buffer descriptors (k_p5b) wherever they reach: byte offsets are
 // 31 bits, so the three components of a state array and of W4 have to span at
 // most BUF_OOB bytes (boxes up to about 640^3 in FP32).  Larger boxes run k_p5.
-template <typename Rt> bool p5b_fits(int M, const P5Args<Rt>& a) {
+template <typename Rt> bool p5b_fits(int M, int N0, int N1, int Nh, int nkyo, int nkzop) {
   const long esz = 2 * (long)sizeof(Rt);
-  const long state = 3L * a.N0 * a.N1 * a.Nh * esz;
-  const long w4 = 3L * M * (a.y_neg + a.y_pos + 1) * a.nkzop * esz;
-  return state <= BUF_OOB && w4 <= BUF_OOB;
+  return 3L * N0 * N1 * Nh * esz <= BUF_OOB && 3L * M * nkyo * nkzop * esz <= BUF_OOB;
+}
+template <typename Rt> bool p5b_fits(int M, const P5Args<Rt>& a) {
+  return p5b_fits<Rt>(M, a.N0, a.N1, a.Nh, a.y_neg + a.y_pos + 1, a.nkzop);
 }
 // Padded rows of the 3/2 rule (see p5b_body).
 template <typename Rt> bool p5b_padded(int M, const P5Args<Rt>& a) {
@@ -250,6 +251,89 @@ template <typename Rt, int MODE> int launch_p5(int M, int var, const P5Args<Rt>&
     else p5_go<Rt, m, 0, MODE>(a, s, nblk);                              \
     return 0;
     SDNS_STRIDED_SIZES(SDNS_X)
+#undef SDNS_X
+    default: return -1;
+  }
+}
+
+// Runs go(std::integral_constant<int, mode>) for the runtime mode.
+template <typename F> void with_mode(int mode, F go) {
+  switch (mode) {
+    case P5_RHS: return go(std::integral_constant<int, P5_RHS>{});
+    case P5_RK0: return go(std::integral_constant<int, P5_RK0>{});
+    case P5_RK12: return go(std::integral_constant<int, P5_RK12>{});
+    default: return go(std::integral_constant<int, P5_RK3>{});
+  }
+}
+// Schedules of the VV and MHD x passes: the one with the fewest points per
+// thread (MHD keeps eight values per point in registers).
+constexpr int min_E(int M) { return strided_E(M, 1) < strided_E(M, 0) ? strided_E(M, 1) : strided_E(M, 0); }
+template <typename Rt, int M> int p5vv_go(int mode, const P5Args<Rt>& a, hipStream_t s) {
+  constexpr int E = min_E(M);
+  using Cfg = SCfg<Rt, M, E>;
+  constexpr int MD = max_div(M, 128, Cfg::T, Cfg::THREADS);
+  const bool pad = M != a.N0;
+  if (pad && (M % 3 || E % 3)) return -1;
+  with_div<MD>(tile_div((a.Q + Cfg::T - 1) / Cfg::T, MD), [&](auto dd) {
+    constexpr int D = decltype(dd)::value, T = Cfg::T / D;
+    const dim3 g(xcd_grid((a.Q + T - 1) / T)), b(Cfg::THREADS / D);
+    with_mode(mode, [&](auto mm) {
+      constexpr int MODE = decltype(mm)::value;
+      if constexpr (M % 3 == 0 && E % 3 == 0) {
+        if (pad) {
+          hipLaunchKernelGGL((k_p5vv<Rt, M, E, MODE, true, D>), g, b, 0, s, a);
+          return;
+        }
+      }
+      hipLaunchKernelGGL((k_p5vv<Rt, M, E, MODE, false, D>), g, b, 0, s, a);
+    });
+  });
+  return 0;
+}
+template <typename Rt> int launch_p5vv(int M, int mode, const P5Args<Rt>& a, hipStream_t s) {
+  switch (M) {
+#define SDNS_X(m) case m: return p5vv_go<Rt, m>(mode, a, s);
+    SDNS_STRIDED_SIZES(SDNS_X)
+#undef SDNS_X
+    default: return -1;
+  }
+}
+template <typename Rt, int M> int mhd_x_go(int mode, const MhdXArgs<Rt>& a, hipStream_t s) {
+  constexpr int E = min_E(M);
+  using Cfg = SCfg<Rt, M, E>;
+  const bool pad = M != a.N0;
+  if (pad && (M % 3 || E % 3)) return -1;
+  const dim3 g(xcd_grid((a.Q + Cfg::T - 1) / Cfg::T), 2), b(Cfg::THREADS);  // U, B
+  with_mode(mode, [&](auto mm) {
+    constexpr int MODE = decltype(mm)::value;
+    if constexpr (M % 3 == 0 && E % 3 == 0) {
+      if (pad) {
+        hipLaunchKernelGGL((k_mhd_x<Rt, M, E, MODE, true>), g, b, 0, s, a);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((k_mhd_x<Rt, M, E, MODE, false>), g, b, 0, s, a);
+  });
+  return 0;
+}
+template <typename Rt> int launch_mhd_x(int M, int mode, const MhdXArgs<Rt>& a, hipStream_t s) {
+  switch (M) {
+#define SDNS_X(m) case m: return mhd_x_go<Rt, m>(mode, a, s);
+    SDNS_STRIDED_SIZES(SDNS_X)
+#undef SDNS_X
+    default: return -1;
+  }
+}
+template <typename Rt> int launch_mhd_z(int n, const MhdZArgs<Rt>& a, hipStream_t s) {
+  switch (n) {
+#define SDNS_X(m)                                                                                     \
+  case m: {                                                                                           \
+    constexpr int E = zline_E(m, 1) < zline_E(m, 0) && zline_E(m, 1) >= 4 ? zline_E(m, 1) : zline_E(m, 0); \
+    using Cfg = ZCfg<Rt, m, E>;                                                                       \
+    hipLaunchKernelGGL((k_mhd_z<Rt, m, E>), dim3((a.L + Cfg::LPB - 1) / Cfg::LPB), dim3(Cfg::THREADS), 0, s, a); \
+    return 0;                                                                                         \
+  }
+    SDNS_HALF_SIZES(SDNS_X)
 #undef SDNS_X
     default: return -1;
   }
@@ -775,6 +859,14 @@ template <typename Rt> int launch_errnorm(const void* err, const void* u0, const
 #define SDNS_PART_P5RK0(Rt) SDNS_P5_MODE(Rt, P5_RK0)
 #define SDNS_PART_P5RK12(Rt) SDNS_P5_MODE(Rt, P5_RK12)
 #define SDNS_PART_P5RK3(Rt) SDNS_P5_MODE(Rt, P5_RK3)
+#define SDNS_PART_P5VV(Rt) \
+  namespace sdns {         \
+  template bool p5b_fits<Rt>(int, int, int, int, int, int); \
+  template int launch_p5vv<Rt>(int, int, const P5Args<Rt>&, hipStream_t); }
+#define SDNS_PART_MHDX(Rt) \
+  namespace sdns { template int launch_mhd_x<Rt>(int, int, const MhdXArgs<Rt>&, hipStream_t); }
+#define SDNS_PART_MHDZ(Rt) \
+  namespace sdns { template int launch_mhd_z<Rt>(int, const MhdZArgs<Rt>&, hipStream_t); }
 #define SDNS_PART_LINES(Rt)                                                                      \
   namespace sdns {                                                                               \
   template int launch_strided<Rt>(int, int, int, int, const StridedArgs<Rt>&, hipStream_t);      \

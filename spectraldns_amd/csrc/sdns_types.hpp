@@ -35,6 +35,8 @@ template <typename Rt> struct P1Args {  // x-inverse of u_hat + kx products
   void* w1;           // [5][M0][Q] ([6][M0][Q] with a given vorticity)
   const void* tw;     // forward twiddles of length M0
   const Rt* kx;       // wavenumbers of axis 0 by stored index
+  const Rt *ky, *kz;  // read with curl_inv only
+  int curl_inv;       // with a given vorticity: the velocity is i (K/K^2) x w (u is not read)
   int N0, N1, Nh;
   RowMap x;           // kept input modes of axis 0 (base = N0)
   int y_neg, y_pos;   // kept input modes of axis 1
@@ -140,6 +142,38 @@ template <typename Rt> struct P5Args {  // x-forward + mask + pressure + diffusi
   Rt sdt;             // KEEP_RHS: the stage state is u + sdt s
   Rt a12;             // KEEP_RHS, stage 3: a dt of stages 1 and 2 (stage 0's is adt)
   int Q;              // N1 * Nh state columns
+};
+
+// MHD in Elsasser form (solvers/MHD.py): W1 and W2 hold the six fields u, b of a
+// given-vorticity pass, W3 and W4 the transforms of the nine products S00, S01,
+// S02, S11, S12, S22, A01, A02, A12 (see k_mhd_z).
+template <typename Rt> struct MhdZArgs {  // z C2R x6, nine products, z R2C x9
+  const void* w2;
+  void* w3;           // [9][L][nkzo]
+  const void* tw;
+  const void* rtw;
+  int nkz, nkzp, nkzo, nkzop;
+  int L;
+};
+template <typename Rt> struct MhdXArgs {  // x-forward of the products, mask, pressure, diffusion, RK4 stage
+  const void* w4;     // [9][M0][nkyo][nkzo]
+  // arrays of three components, [0] of U and [1] of B; roles as in P5Args with
+  // KEEP_STATES (P5_RHS: u the input state, out the right-hand side)
+  void* u[2];
+  const void* s[2];
+  void* out[2];
+  const void* b1[2];
+  const void* b2[2];
+  void* phat;         // P5_RHS, P5_RK3: pressure output (may be null)
+  const void* tw;
+  const Rt *kx, *ky, *kz;
+  int N0, N1, Nh, N2;
+  RowMap x;
+  int y_neg, y_pos, nkzo, nkzop;
+  int mask_nyquist;
+  Rt visc[2];         // nu, eta
+  Rt scale, adt, bdt;
+  int Q;
 };
 
 // One block of a batched pass: box index (-1 for padding blocks) and the

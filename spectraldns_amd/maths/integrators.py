@@ -156,11 +156,16 @@ def getintegrator(rhs, u0, solver, context):
             raise NotImplementedError("the compensated state is carried by the fused NS RK4 step only")
         a = np.array([1. / 6., 1. / 3., 1. / 3., 1. / 6.], dtype=context.float)
         b = np.array([0.5, 0.5, 1.], dtype=context.float)
-        u1, u2 = u0.clone(), u0.clone()
+        work = []
 
         @wraps(RK4_stages)
         def func():
-            return RK4_stages(u0, u1, u2, rhs, a, b, params.dt, solver, context)
+            fused = getattr(solver, "fused_rk4_step", None)
+            if fused is not None and fused(u0, params.dt, solver, context):
+                return u0, params.dt, params.dt
+            if not work:
+                work.extend((u0.clone(), u0.clone()))
+            return RK4_stages(u0, work[0], work[1], rhs, a, b, params.dt, solver, context)
         return func
 
     if params.integrator == "RK4":

@@ -5,13 +5,14 @@ The primary variable is UB_hat = (U_hat, B_hat), six spectral components.
 The module keeps the reference's protocol (``get_context`` with its keys,
 ``set_Elsasser``, ``divergenceConvection``, ``getConvection('Divergence')``,
 ``add_pressure_diffusion`` with nu on U and eta on B, ``ComputeRHS``,
-``get_divergence``) and RK4 runs stage by stage over ComputeRHS.  Each step
-of the RHS is a libsdns_hip launch: the inverse transforms of the six
-fields over their kept modes (the 2/3-rule truncation inside the transform
-passes), one kernel for the nine Elsasser
-products (u_i + b_i)(u_j - b_j), their forward transforms, one kernel for
-set_Elsasser, the Nyquist mask, the NS pressure/diffusion kernel on U and
-the diffusion kernel on B.
+``get_divergence``).  The right-hand side and RK4 run in fused passes
+(sdns_mhd_rhs, sdns_mhd_rk4_steps): dealiased inverse transforms of the six
+fields, the nine products formed in the z pass, and the sums of
+set_Elsasser, the Nyquist mask, pressure, diffusion and the stage update in
+the last pass; ub_dealias and ZZ_hat are not written then.  With a replaced
+step (conv, set_Elsasser, divergenceConvection, add_pressure_diffusion), or a
+box beyond the fused passes, each step is a launch of its own over those
+arrays.
 
 Built for the 2/3 rule (shenfun's dealias_direct, dealias_mode 0), the 3/2
 rule (the six fields transformed onto the padded 3N/2 grid, the nine
@@ -145,6 +146,7 @@ def getConvection(convection):
         return rhs
 
     Conv.convection = convection
+    Conv.mhd_fused = True
     return Conv
 
 
@@ -157,9 +159,20 @@ def add_pressure_diffusion(rhs, ub_hat, nu, eta, K2, K, P_hat, K_over_K2):
     return rhs
 
 
+def _fused(solver, c):
+    """Whether the right-hand side is the module's own (no step of it replaced)
+    and the fused passes reach the box."""
+    plan = c["T"].plan
+    return (getattr(solver.conv, "mhd_fused", False) and solver.add_pressure_diffusion is add_pressure_diffusion and
+            solver.divergenceConvection is _module_convection and solver.set_Elsasser is _module_elsasser and
+            plan.nyquist_masked == (c["mask"] is not None) and plan.fused_stages)
+
+
 def ComputeRHS(rhs, ub_hat, solver, **context):
     """conv, Nyquist mask, pressure and diffusion (MHD.py:150-176)."""
     c = context
+    if _fused(solver, c) and rhs.data_ptr() != ub_hat.data_ptr():
+        return c["T"].plan.mhd_rhs(ub_hat, rhs, params.nu, params.eta, c["P_hat"])
     rhs = solver.conv(rhs, ub_hat, c["Tp"], c["VMp"], c["K"], c["ub_dealias"], c["ZZ_hat"])
     if c["mask"] is not None:
         c["T"].plan.mask_nyquist(rhs[:3])
@@ -167,3 +180,18 @@ def ComputeRHS(rhs, ub_hat, solver, **context):
     rhs = solver.add_pressure_diffusion(rhs, ub_hat, params.nu, params.eta, c["K2"], c["K"], c["P_hat"],
                                         c["K_over_K2"])
     return rhs
+
+
+_module_rhs = ComputeRHS
+_module_convection = divergenceConvection
+_module_elsasser = set_Elsasser
+
+
+def fused_rk4_step(ub_hat, dt, solver, context):
+    """One RK4 step of ub_hat in place with the stage updates inside the passes
+    (P_hat of the last stage); False where the right-hand side is not the
+    module's own."""
+    if solver.ComputeRHS is not _module_rhs or not _fused(solver, context):
+        return False
+    context.T.plan.mhd_rk4_steps(ub_hat, [dt], params.nu, params.eta, context.P_hat)
+    return True

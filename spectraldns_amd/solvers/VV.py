@@ -134,12 +134,22 @@ def add_linear(rhs, w_hat, nu, K2, Source):
     """Add contributions from source and diffusion to the rhs (VV.py:110-115)."""
 
 
+def _fused(solver, c):
+    """Whether the right-hand side is the module's own (Conv, cross2, mask and
+    add_linear not replaced) and the fused passes reach the box."""
+    plan = c["VT"].plan
+    return (getattr(solver.conv, "vv_fused_tail", False) and solver.add_linear is add_linear and
+            plan.nyquist_masked == (c["mask"] is not None) and plan.fused_stages)
+
+
 def ComputeRHS(rhs, w_hat, solver, **context):
     """rhs = conv(w_hat), Nyquist mask, -nu K^2 w_hat, + Source (VV.py:117-146).
 
     The Source is always added, as the reference does."""
     c = context
     src = c["Source"]
+    if _fused(solver, c) and rhs.data_ptr() != w_hat.data_ptr():
+        return c["VT"].plan.vv_rhs(w_hat, rhs, params.nu, src)
     if getattr(solver.conv, "vv_fused_tail", False) and solver.add_linear is add_linear:
         # the module's own Conv and add_linear: cross2, mask and add_linear in one launch
         v_hat = _cross_convection(w_hat, c["work"], c["VTp"], c["K_over_K2"])
@@ -149,3 +159,15 @@ def ComputeRHS(rhs, w_hat, solver, **context):
         c["VT"].plan.mask_nyquist(rhs)
     rhs = solver.add_linear(rhs, w_hat, params.nu, c["K2"], src)
     return rhs
+
+
+_module_rhs = ComputeRHS
+
+
+def fused_rk4_step(w_hat, dt, solver, context):
+    """One RK4 step of w_hat in place with the stage updates inside the passes;
+    False where the right-hand side is not the module's own."""
+    if solver.ComputeRHS is not _module_rhs or not _fused(solver, context):
+        return False
+    context.VT.plan.vv_rk4_steps(w_hat, [dt], params.nu, context.Source)
+    return True
