@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <string>
@@ -88,6 +89,7 @@ struct sdns_plan {
   int in[3][2], out[3][2];
   int nky, nkz, nkyo, nkzo;
   int nkzp, nkzop;  // kz strides of the work buffers, padded to 16 elements
+  bool plane = false;  // P2, P3 and P4 run as one launch per evaluation (sdns_plane.hpp)
   int var[6] = {0, 0, 0, 0, 0, 0};  // schedule variant per pass (see sdns_plan_set_variant)
   // device tables
   std::map<int, void*> tw;       // forward twiddles by line length
@@ -217,6 +219,16 @@ void compute_sizes(sdns_plan* p) {
   // P5 blocks: columns N1*Nh over the smallest tile of the supported lengths
   p->max_blocks = p->N[1] * p->Nh;  // upper bound (>= 1 column per block)
   p->szPart = align256((size_t)std::max(p->max_blocks, 4096) * 2 * sizeof(double) + 4096);
+}
+
+// Work-buffer layout: kz strides padded to 16 elements for the column-tiled y
+// passes and the z pass; unpadded where one kernel handles whole planes, whose
+// accesses then are contiguous and whose W4 columns line up with the state's.
+void plan_layout(sdns_plan* p, bool plane) {
+  p->plane = plane;
+  p->nkzp = plane ? p->nkz : (p->nkz + 15) / 16 * 16;
+  p->nkzop = plane ? p->nkzo : (p->nkzo + 15) / 16 * 16;
+  compute_sizes(p);
 }
 
 int assign_workspace(sdns_plan* p, void* base, size_t bytes) {
@@ -431,6 +443,18 @@ template <typename Rt> StridedArgs<Rt> p2_given_args(const sdns_plan* p) {
   return a;
 }
 
+template <typename Rt> PlaneArgs<Rt> plane_args(const sdns_plan* p) {
+  PlaneArgs<Rt> a{};
+  a.w1 = p->bufA; a.w4 = p->bufB;
+  a.twy = p->tw.at(p->M[1]); a.twz = p->tw.at(p->n2h); a.rtw = p->rtw.at(p->M[2]);
+  a.ky = (const Rt*)p->ktab[1]; a.kz = (const Rt*)p->ktab[2];
+  a.N1 = p->N[1]; a.M0 = p->M[0];
+  a.y = rmap(p->in[1][0], p->in[1][1], p->nky);
+  a.yo = rmap(p->out[1][0], p->out[1][1], p->nkyo);
+  a.nkz = p->nkz; a.nkzp = p->nkzp; a.nkzo = p->nkzo; a.nkzop = p->nkzop;
+  return a;
+}
+
 // P1..P4 of one convection evaluation from the state of a1 into W4 (= bufB).  a1.w:
 // the vorticity of u when given (the velocity-vorticity solver), otherwise
 // null and the passes form curl(u).
@@ -440,6 +464,14 @@ template <typename Rt> int conv_passes(sdns_plan* p, const P1Args<Rt>& a1) {
   tstart(p, 0);
   if (launch_p1<Rt>(M0, p->var[0], a1, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", M0);
   tstop(p);
+  if (p->plane) {  // small boxes: P2, P3 and P4 in one
+    PlaneArgs<Rt> ap = plane_args<Rt>(p);
+    ap.given = w != nullptr;
+    tstart(p, 2);
+    if (launch_plane<Rt>(M1, p->n2h, ap, p->stream)) return fail(SDNS_ERR_HIP, "plane launch, %d rows", M1);
+    tstop(p);
+    return 0;
+  }
   tstart(p, 1);
   if (w) {
     if (launch_strided<Rt>(M1, p->var[1], +1, 6, p2_given_args<Rt>(p), p->stream))
@@ -913,6 +945,11 @@ struct sdns_batch {
   void* d_p1[4] = {nullptr, nullptr, nullptr, nullptr};  // P1 args of RK stages 0..3
   void *d_p2 = nullptr, *d_p3 = nullptr, *d_p4 = nullptr;
   void* d_p5[4] = {nullptr, nullptr, nullptr, nullptr};  // P5 args of RK stages 0..3
+  // boxes whose planes all fit in LDS run one plane launch per side instead of
+  // passes 2..4: argument blocks, and per side the work items (box, plane)
+  struct PlaneClass { int M1, nkz, nwork; BatchWork* work; };
+  void* d_plane = nullptr;
+  std::vector<PlaneClass> planes;
   int* d_len[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   BatchWork* d_work[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   int nwork[5] = {0, 0, 0, 0, 0}, lmax[5] = {0, 0, 0, 0, 0};
@@ -986,8 +1023,25 @@ template <typename Rt> int batch_layout(sdns_batch* b) {
       b->lmax[k] = std::max(b->lmax[k], l[k]);
     }
   }
+  b->planes.clear();
+  std::vector<std::vector<BatchWork>> pwork;
+  if (b->box[0]->plane) {
+    std::map<int, std::vector<int>, std::greater<int>> side;  // largest planes first: their launch fills the chip
+    for (int i = 0; i < nb; ++i) side[b->box[i]->M[1]].push_back(i);
+    for (const auto& kv : side) {
+      std::vector<int> n(nb, 0), w(nb, 1);
+      int nkz = 0;
+      for (int i : kv.second) {
+        n[i] = b->box[i]->M[0];
+        nkz = std::max(nkz, b->box[i]->nkz);
+      }
+      pwork.push_back(batch_work(n, w));
+      b->planes.push_back({kv.first, nkz, (int)pwork.back().size() / 8 * 8, nullptr});
+    }
+  }
   std::vector<BatchWork> work[5];
   size_t nitems = 0;
+  for (const auto& w : pwork) nitems += w.size();
   for (int k = 0; k < 5; ++k) {
     work[k] = batch_work(nt[k], wt[k]);
     b->nwork[k] = (int)work[k].size() / 8 * 8;
@@ -997,16 +1051,16 @@ template <typename Rt> int batch_layout(sdns_batch* b) {
   b->pcnt = nt[4];
   int part_total = 0;
   for (int i = 0; i < nb; ++i) { b->poff[i] = part_total; part_total += 2 * nt[4][i]; }
-  // one allocation: 11 argument arrays, lengths, work lists, partials, diag, nu, offsets
-  size_t argsz = std::max(std::max(sizeof(P1Args<Rt>), sizeof(P2Args<Rt>)),
+  // one allocation: 12 argument arrays, lengths, work lists, partials, diag, nu, offsets
+  size_t argsz = std::max(std::max(std::max(sizeof(P1Args<Rt>), sizeof(P2Args<Rt>)), sizeof(PlaneArgs<Rt>)),
                           std::max(std::max(sizeof(P3Args<Rt>), sizeof(StridedArgs<Rt>)), sizeof(P5Args<Rt>)));
   b->args_bytes = align256(argsz * nb);
-  const size_t bytes = 11 * b->args_bytes + align256(5 * nb * sizeof(int)) + align256(nitems * sizeof(BatchWork)) +
+  const size_t bytes = 12 * b->args_bytes + align256(5 * nb * sizeof(int)) + align256(nitems * sizeof(BatchWork)) +
                        align256(part_total * sizeof(double)) + 2 * align256(2 * nb * sizeof(double)) +
                        2 * align256(nb * sizeof(int));
   if (hipMalloc((void**)&b->dmem, bytes) != hipSuccess) return fail(SDNS_ERR_NOMEM, "hipMalloc of %zu bytes failed", bytes);
   char* c = b->dmem;
-  void** slots[11] = {&b->d_p1[0], &b->d_p1[1], &b->d_p1[2], &b->d_p1[3], &b->d_p2, &b->d_p3, &b->d_p4,
+  void** slots[12] = {&b->d_plane, &b->d_p1[0], &b->d_p1[1], &b->d_p1[2], &b->d_p1[3], &b->d_p2, &b->d_p3, &b->d_p4,
                       &b->d_p5[0], &b->d_p5[1], &b->d_p5[2], &b->d_p5[3]};
   for (auto sl : slots) { *sl = c; c += b->args_bytes; }
   int* lens = (int*)c;
@@ -1029,6 +1083,12 @@ template <typename Rt> int batch_layout(sdns_batch* b) {
                            b->own));
     o += work[k].size();
   }
+  for (size_t c = 0; c < pwork.size(); ++c) {
+    b->planes[c].work = wl + o;
+    HIP_TRY(hipMemcpyAsync(wl + o, pwork[c].data(), pwork[c].size() * sizeof(BatchWork), hipMemcpyHostToDevice,
+                           b->own));
+    o += pwork[c].size();
+  }
   HIP_TRY(hipMemcpyAsync(b->d_poff, b->poff.data(), nb * sizeof(int), hipMemcpyHostToDevice, b->own));
   HIP_TRY(hipMemcpyAsync(b->d_pcnt, b->pcnt.data(), nb * sizeof(int), hipMemcpyHostToDevice, b->own));
   HIP_TRY(hipStreamSynchronize(b->own));
@@ -1043,8 +1103,10 @@ template <typename Rt> int batch_upload(sdns_batch* b) {
   std::vector<P3Args<Rt>> h3;
   std::vector<StridedArgs<Rt>> h4;
   std::vector<P5Args<Rt>> h5[4];
+  std::vector<PlaneArgs<Rt>> hp;
   for (int i = 0; i < nb; ++i) {
     const sdns_plan* p = b->box[i];
+    hp.push_back(plane_args<Rt>(p));
     const Rt dt = (Rt)b->dt[i];
     const int keep = rk_keep<Rt>(p->M[0] != p->N[0], false);
     for (int rk = 0; rk < 4; ++rk) {
@@ -1072,6 +1134,7 @@ template <typename Rt> int batch_upload(sdns_batch* b) {
   hipStream_t s = b->own;
   for (int rk = 0; rk < 4; ++rk)
     HIP_TRY(hipMemcpyAsync(b->d_p1[rk], h1[rk].data(), nb * sizeof(P1Args<Rt>), hipMemcpyHostToDevice, s));
+  HIP_TRY(hipMemcpyAsync(b->d_plane, hp.data(), nb * sizeof(PlaneArgs<Rt>), hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(b->d_p2, h2.data(), nb * sizeof(P2Args<Rt>), hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(b->d_p3, h3.data(), nb * sizeof(P3Args<Rt>), hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(b->d_p4, h4.data(), nb * sizeof(StridedArgs<Rt>), hipMemcpyHostToDevice, s));
@@ -1087,9 +1150,15 @@ template <typename Rt> int batch_step(sdns_batch* b, hipStream_t s) {
   for (int rk = 0; rk < 4; ++rk) {
     launch_batch_p1<Rt>(b->lmax[0], (const P1Args<Rt>*)b->d_p1[rk], b->d_len[0], b->d_work[0],
                         b->nwork[0], s);
-    launch_batch_p2<Rt>(b->lmax[1], (const P2Args<Rt>*)b->d_p2, b->d_len[1], b->d_work[1], b->nwork[1], s);
-    launch_batch_p3<Rt>(b->lmax[2], (const P3Args<Rt>*)b->d_p3, b->d_len[2], b->d_work[2], b->nwork[2], s);
-    launch_batch_fwd<Rt>(b->lmax[3], (const StridedArgs<Rt>*)b->d_p4, b->d_len[3], b->d_work[3], b->nwork[3], 3, s);
+    if (!b->planes.empty()) {
+      for (const auto& c : b->planes)
+        if (launch_batch_plane<Rt>(c.M1, c.nkz, (const PlaneArgs<Rt>*)b->d_plane, c.work, c.nwork, s))
+          return fail(SDNS_ERR_HIP, "plane launch, %d rows", c.M1);
+    } else {
+      launch_batch_p2<Rt>(b->lmax[1], (const P2Args<Rt>*)b->d_p2, b->d_len[1], b->d_work[1], b->nwork[1], s);
+      launch_batch_p3<Rt>(b->lmax[2], (const P3Args<Rt>*)b->d_p3, b->d_len[2], b->d_work[2], b->nwork[2], s);
+      launch_batch_fwd<Rt>(b->lmax[3], (const StridedArgs<Rt>*)b->d_p4, b->d_len[3], b->d_work[3], b->nwork[3], 3, s);
+    }
     const int mode = RkStage<Rt>::mode(rk);
     launch_batch_p5<Rt>(b->lmax[4], mode, (const P5Args<Rt>*)b->d_p5[rk], b->d_len[4], b->d_work[4], b->nwork[4], s);
   }
@@ -1193,8 +1262,8 @@ int sdns_plan_create(sdns_plan** plan, const int32_t N[3], const double L[3], in
   p->nkz = p->in[2][1] + 1;
   p->nkyo = p->out[1][0] + p->out[1][1] + 1;
   p->nkzo = p->out[2][1] + 1;
-  p->nkzp = (p->nkz + 15) / 16 * 16;
-  p->nkzop = (p->nkzo + 15) / 16 * 16;
+  plan_layout(p, precision == SDNS_DOUBLE ? plane_fits<double>(p->M[0], p->M[1], p->n2h, p->nkz)
+                                          : plane_fits<float>(p->M[0], p->M[1], p->n2h, p->nkz));
   const int lens[] = {p->M[0], p->M[1], p->N[0], p->N[1]};
   for (int l : lens)
     if (!strided_supported(l)) { delete p; return fail(SDNS_ERR_UNSUPPORTED, "no kernel for line length %d", l); }
@@ -1206,7 +1275,6 @@ int sdns_plan_create(sdns_plan** plan, const int32_t N[3], const double L[3], in
   if (cols > 0x7fffffffLL) { delete p; return fail(SDNS_ERR_UNSUPPORTED, "grid too large"); }
   const int rc = precision == SDNS_DOUBLE ? build_tables<double>(p) : build_tables<float>(p);
   if (rc) { sdns_plan_destroy(p); return rc; }
-  compute_sizes(p);
   *plan = p;
   return 0;
 }
@@ -1601,7 +1669,16 @@ int sdns_batch_create(sdns_batch** out, int nbox, const int32_t* N, const double
     if (!batch_strided_ok(p->M[0]) || !batch_strided_ok(p->M[1]) || !batch_half_ok(p->n2h))
       return bail(fail(SDNS_ERR_UNSUPPORTED, "box %d: no batched kernel for lines %d x %d x %d (x, y in 16..128 "
                        "with a power-of-two thread count per line, z/2 in 8..64)", i, p->M[0], p->M[1], p->M[2]));
-    if ((rc = ensure_workspace(p))) return bail(rc);
+  }
+  // plane launches for all boxes or for none: the passes run over whole ensembles
+  bool planes = true;
+  for (const sdns_plan* p : b->box)
+    planes = planes && (precision == SDNS_DOUBLE ? batch_plane_fits<double>(p->M[1], p->n2h, p->nkz)
+                                                 : batch_plane_fits<float>(p->M[1], p->n2h, p->nkz));
+  for (sdns_plan* p : b->box) {
+    plan_layout(p, planes);
+    const int rc = ensure_workspace(p);
+    if (rc) return bail(rc);
   }
   const int rc = precision == SDNS_DOUBLE ? batch_layout<double>(b) : batch_layout<float>(b);
   if (rc) return bail(rc);

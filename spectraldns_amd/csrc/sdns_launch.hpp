@@ -34,6 +34,14 @@ template <typename Rt> int launch_p5(int M, int var, int mode, const P5Args<Rt>&
     default: return launch_p5<Rt, P5_RK3>(M, var, a, s, nblk);
   }
 }
+// P2, P3 and P4 of small boxes in one kernel per x-plane (sdns_plane.hpp); -1
+// where the plane does not fit in LDS or its lengths are not compiled.
+template <typename Rt> int launch_plane(int M1, int n, const PlaneArgs<Rt>& a, hipStream_t s);
+template <typename Rt> bool plane_fits(int M0, int M1, int n, int nkz);
+// Batched: boxes with cubic planes of M1 rows; nkz: the largest kept count among them.
+template <typename Rt> bool batch_plane_fits(int M1, int n, int nkz);
+template <typename Rt> int launch_batch_plane(int M1, int nkz, const PlaneArgs<Rt>* args, const BatchWork* work,
+                                              int nwork, hipStream_t s);
 // The x-forward stage of the velocity-vorticity solver (KEEP_STATES), and the z
 // and x-forward passes of MHD; boxes within a buffer descriptor's reach
 // (p5b_fits), one schedule per length.

@@ -1,0 +1,3 @@
+// Single-precision instantiation of the plane kernels.
+#include "sdns_plane.hpp"
+SDNS_PLANE_INSTANTIATE(float)

@@ -176,6 +176,18 @@ template <typename Rt> struct MhdXArgs {  // x-forward of the products, mask, pr
   int Q;
 };
 
+// One x-plane of P2, P3 and P4 in LDS (sdns_plane.hpp).
+template <typename Rt> struct PlaneArgs {
+  const void* w1;
+  void* w4;
+  const void *twy, *twz, *rtw;  // forward twiddles of lengths M1 and M2/2, real-transform table
+  const Rt *ky, *kz;
+  int N1, M0;
+  RowMap y, yo;       // kept input modes of axis 1 (base = nky), kept output modes (base = nkyo)
+  int nkz, nkzp, nkzo, nkzop;
+  int given;          // W1 holds the six fields of a given vorticity
+};
+
 // One block of a batched pass: box index (-1 for padding blocks) and the
 // block's tile within that box.
 struct BatchWork {
