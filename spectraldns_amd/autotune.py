@@ -43,7 +43,8 @@ def load_table(path=SCHEDULE_FILE):
 
 
 def apply_schedule(plan, path=SCHEDULE_FILE):
-    """Set the stored variants for this plan's box (no-op if none stored)."""
+    """Set the stored variants for this plan's box (none stored: the plan keeps
+    its default schedules, chosen by line length)."""
     entry = load_table(path).get(key_of(plan.N, plan.precision, plan.dealias, plan.dealias_mode))
     if not entry:
         return None

@@ -2,11 +2,13 @@
 // twiddle / wavenumber tables and the orchestration of the pass kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <string>
@@ -229,6 +231,33 @@ void plan_layout(sdns_plan* p, bool plane) {
   p->nkzp = plane ? p->nkz : (p->nkz + 15) / 16 * 16;
   p->nkzop = plane ? p->nkzo : (p->nkzo + 15) / 16 * 16;
   compute_sizes(p);
+}
+
+// Schedule variant of each pass for a box that the autotuner's table does not
+// hold, by line length: variant 1 (and for the z pass 2 and 3, the LDS-assisted
+// scheme) where it measured faster on cubes of 32..512 points with either
+// dealiasing rule, by more than 2%; 0 elsewhere.  What decides:
+//   z: six lines of 12 to 16 points per thread take 200 to 256 registers in FP32;
+//   parking two of them in LDS (2, 3) is 1.1 to 1.7 times faster from 36-point
+//   lines on (256^3 3/2 rule 0.63 -> 0.37 ms, 512^3 2/3 rule 1.69 -> 1.10 ms with
+//   16 -> 8 points).  In FP64 the LDS lines cost more than the registers, except
+//   at 96 and 192 points (256^3 3/2 rule 1.08 -> 1.02 ms).  Lines of 16 and 32
+//   points: more threads per line (64^3: 13.0 -> 10.1 us).
+//   x, y: the schedule with the block size that fills a CU's LDS better.
+int default_variant(int pass, int len, int precision) {
+  const bool f32 = precision == SDNS_SINGLE;
+  auto in = [len](std::initializer_list<int> l) { return std::find(l.begin(), l.end(), len) != l.end() ? 1 : 0; };
+  switch (pass) {
+    case 0: return f32 ? in({128, 192, 256, 384}) : in({128});
+    case 1: return f32 ? in({128, 256, 512}) : in({64, 128, 256});
+    case 2:
+      if (in({16, 32})) return 1;
+      if (f32) return len == 256 ? 3 : (len == 512 ? 1 : (len >= 36 ? 2 : 0));
+      return in({96, 192}) ? 2 : 0;
+    case 3: return f32 ? 0 : in({128});
+    case 4: return f32 ? in({64, 128, 384, 512}) : in({128, 384});
+    default: return 0;
+  }
 }
 
 int assign_workspace(sdns_plan* p, void* base, size_t bytes) {
@@ -1264,6 +1293,8 @@ int sdns_plan_create(sdns_plan** plan, const int32_t N[3], const double L[3], in
   p->nkzo = p->out[2][1] + 1;
   plan_layout(p, precision == SDNS_DOUBLE ? plane_fits<double>(p->M[0], p->M[1], p->n2h, p->nkz)
                                           : plane_fits<float>(p->M[0], p->M[1], p->n2h, p->nkz));
+  const int plen[5] = {p->M[0], p->M[1], p->n2h, p->M[1], p->M[0]};
+  for (int k = 0; k < 5; ++k) p->var[k] = default_variant(k, plen[k], precision);
   const int lens[] = {p->M[0], p->M[1], p->N[0], p->N[1]};
   for (int l : lens)
     if (!strided_supported(l)) { delete p; return fail(SDNS_ERR_UNSUPPORTED, "no kernel for line length %d", l); }
