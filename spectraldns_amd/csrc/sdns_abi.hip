@@ -866,7 +866,7 @@ template <typename Rt> int spectrum(sdns_plan* p, const void* u, int nb, double*
   EwArgs<Rt> a = ew_args<Rt>(p);
   a.a = u;
   launch_spectrum<Rt>(a, nb, part, nblk, p->stream);
-  if (launch_sum_rows(part, nblk, 2 * nb, out, p->stream)) return fail(SDNS_ERR_HIP, "sum rows");
+  if (launch_sum_cols(part, nblk, 2 * nb, out, p->stream)) return fail(SDNS_ERR_HIP, "sum columns");
   return 0;
 }
 template <typename Rt> int spectrum(sdns_plan* p, const void* u, int nb, double* out) {
@@ -904,15 +904,6 @@ int launch_sum_partials(const double* part, int nblk, double* out, double e_scal
   hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, s, part, nblk, out, e_scale, o_scale);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
-// out[j] = sum over b of part[b*width + j], fixed order (deterministic).
-__global__ void __launch_bounds__(256) k_sum_rows(const double* __restrict__ part, int nblk, int width,
-                                                  double* __restrict__ out) {
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= width) return;
-  double s = 0;
-  for (int b = 0; b < nblk; ++b) s += part[(long)b * width + j];
-  out[j] = s;
-}
 // Column sums of part[nblk][width] with one block per column: strided per-thread
 // sums, then a fixed-order tree in LDS (deterministic, no serial chain over nblk).
 __global__ void __launch_bounds__(256) k_sum_cols(const double* __restrict__ part, int nblk, int width,
@@ -931,10 +922,6 @@ __global__ void __launch_bounds__(256) k_sum_cols(const double* __restrict__ par
 }
 int launch_sum_cols(const double* part, int nblk, int width, double* out, hipStream_t s) {
   hipLaunchKernelGGL(k_sum_cols, dim3(width), dim3(256), 0, s, part, nblk, width, out);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-int launch_sum_rows(const double* part, int nblk, int width, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_sum_rows, dim3((width + 255) / 256), dim3(256), 0, s, part, nblk, width, out);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 // Per-box (energy, dissipation) of a batched ensemble: block b sums box b's

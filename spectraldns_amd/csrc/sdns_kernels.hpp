@@ -380,7 +380,9 @@ template <typename C> __device__ __forceinline__ C r2c_bin(C A, C Bz, C w) {
 // Post-process of the forward half-length FFT held in z (natural positions
 // t + P e); `my` is this line's LDS area.  Writes kept bins k < nk (and the
 // Nyquist bin n when nk > n).
-template <typename Rt, int n, int E, bool WAVE = false>
+// STREAM: non-temporal stores, for rows that start on 128-byte lines; rows that
+// do not share lines with their neighbours' through L2 and stay cached.
+template <typename Rt, int n, int E, bool WAVE = false, bool STREAM = true>
 __device__ __forceinline__ void r2c_post(cx<Rt> (&z)[E], cx<Rt>* my, cx<Rt>* __restrict__ out, int nk, bool valid,
                                          const cx<Rt>* __restrict__ rtw, int t, Rt scale) {
   using C = cx<Rt>;
@@ -392,8 +394,8 @@ __device__ __forceinline__ void r2c_post(cx<Rt> (&z)[E], cx<Rt>* my, cx<Rt>* __r
   for (int e = 0; e < E; ++e) {
     const int k = t + P * e;
     const C X = r2c_bin(z[e], my[(n - k) % n], rtw[k]);
-    if (valid && t < nk - P * e) st_stream(out + k, cscale(X, scale));
-    if (valid && k == 0 && nk > n) st_stream(out + n, mk<C>((z[e].x - z[e].y) * scale, Rt(0)));
+    if (valid && t < nk - P * e) st_pass<STREAM>(out + k, cscale(X, scale));
+    if (valid && k == 0 && nk > n) st_pass<STREAM>(out + n, mk<C>((z[e].x - z[e].y) * scale, Rt(0)));
   }
   lds_barrier<WAVE>();
 }
@@ -814,7 +816,8 @@ __global__ void __launch_bounds__((ZCfg<Rt, n, E>::THREADS / D), (occ_for(E + st
   lds_barrier<WL>();
   Ff::run(z, t, my, 1, tw);
   C* out = (C*)a.out + blockIdx.y * a.out_field + li * a.out_line;
-  r2c_post<Rt, n, E, WL>(z, my, out, a.nk, valid, rtw, t, a.scale);
+  if (a.out_line * (long)sizeof(C) % 128 == 0) r2c_post<Rt, n, E, WL, true>(z, my, out, a.nk, valid, rtw, t, a.scale);
+  else r2c_post<Rt, n, E, WL, false>(z, my, out, a.nk, valid, rtw, t, a.scale);
 }
 
 // ------------------------------------------------------------------ generic strided

@@ -87,8 +87,7 @@ template <typename Rt> int launch_force_scale(const EwArgs<Rt>& a, Rt kf2, const
 // Shell spectrum (demo/Isotropic.py:88-115): per-block partial sums of uiui and mode counts for
 // shells z = 1..nb (z = #{bins b_i = i + 1/2 : b_i < |K|}), out layout [nblk][2][nb].
 template <typename Rt> int launch_spectrum(const EwArgs<Rt>& a, int nb, double* partials, int nblk, hipStream_t s);
-int launch_sum_rows(const double* partials, int nblk, int width, double* out, hipStream_t s);
-// Same column sums, one block per column (for few columns over many rows).
+// Column sums of partials[nblk][width], one block per column.
 int launch_sum_cols(const double* partials, int nblk, int width, double* out, hipStream_t s);
 
 // ------------------------------------------------------------------ integrator updates

@@ -367,6 +367,15 @@ template <typename Rt> int launch_z(int n, int var, int dir, int nfields, const 
 }
 
 // ------------------------------------------------------------------ elementwise
+// Spectral point index i -> (ix, iy, kz).  In 32 bits (a component has fewer
+// than 2^31 points, checked when the plan is made): the 64-bit divisions took
+// more instructions than the rest of a reduction's loop.
+struct Mode { int ix, iy, kz; };
+__device__ __forceinline__ Mode mode_of(long i, int N1, int Nh) {
+  const unsigned u = (unsigned)i, r = u / (unsigned)Nh;
+  const unsigned ix = r / (unsigned)N1;
+  return {(int)ix, (int)(r - ix * (unsigned)N1), (int)(u - r * (unsigned)Nh)};
+}
 // Spectral point index i -> (ix, iy, kz) of the [N0][N1][Nh] grid.
 template <typename Rt, int OP>
 __global__ void __launch_bounds__(256) k_elementwise(EwArgs<Rt> a) {
@@ -423,10 +432,8 @@ __global__ void __launch_bounds__(256) k_elementwise(EwArgs<Rt> a) {
     ((C*)a.out)[i] = mk<C>(v.y, -v.x);
     return;
   } else {
-    const int kz = (int)(i % a.Nh);
-    const long r = i / a.Nh;
-    const int iy = (int)(r % a.N1);
-    const int ix = (int)(r / a.N1);
+    const Mode md = mode_of(i, a.N1, a.Nh);
+    const int ix = md.ix, iy = md.iy, kz = md.kz;
     const Rt K0 = a.kx[ix], K1 = a.ky[iy], K2 = a.kz[kz];
     const C* A = (const C*)a.a;
     C* O = (C*)a.out;
@@ -620,10 +627,8 @@ __global__ void __launch_bounds__(256) k_energy(EwArgs<Rt> a, double* __restrict
   const long n = a.n;
   double es = 0, os = 0;
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    const int kz = (int)(i % a.Nh);
-    const long r = i / a.Nh;
-    const int iy = (int)(r % a.N1);
-    const int ix = (int)(r / a.N1);
+    const Mode md = mode_of(i, a.N1, a.Nh);
+    const int ix = md.ix, iy = md.iy, kz = md.kz;
     const double k0 = a.kx[ix], k1 = a.ky[iy], k2 = a.kz[kz];
     const C* A = (const C*)a.a;
     const C u0 = A[i], u1 = A[n + i], u2 = A[2 * n + i];
@@ -662,10 +667,8 @@ __global__ void __launch_bounds__(256) k_force_reduce(EwArgs<Rt> a, Rt kf2, doub
   double s_all = 0, s_low = 0;
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
     if (i == 0) continue;  // the mean mode is set to zero first (Isotropic.py:163-164)
-    const int kz = (int)(i % a.Nh);
-    const long r = i / a.Nh;
-    const int iy = (int)(r % a.N1);
-    const int ix = (int)(r / a.N1);
+    const Mode md = mode_of(i, a.N1, a.Nh);
+    const int ix = md.ix, iy = md.iy, kz = md.kz;
     const Rt K0 = a.kx[ix], K1 = a.ky[iy], K2 = a.kz[kz];
     Rt k2 = K0 * K0;
     k2 += K1 * K1;
@@ -710,10 +713,8 @@ __global__ void __launch_bounds__(256) k_force_scale(EwArgs<Rt> a, Rt kf2, const
     if (Lo) { Lo[0] = czero<C>(); Lo[n] = czero<C>(); Lo[2 * n] = czero<C>(); }
     return;
   }
-  const int kz = (int)(i % a.Nh);
-  const long r = i / a.Nh;
-  const int iy = (int)(r % a.N1);
-  const int ix = (int)(r / a.N1);
+  const Mode md = mode_of(i, a.N1, a.Nh);
+  const int ix = md.ix, iy = md.iy, kz = md.kz;
   const Rt K0 = a.kx[ix], K1 = a.ky[iy], K2 = a.kz[kz];
   Rt k2 = K0 * K0;
   k2 += K1 * K1;
@@ -750,18 +751,20 @@ template <typename Rt> int launch_force_scale(const EwArgs<Rt>& a, Rt kf2, const
 }
 
 // ------------------------------------------------------------------ spectrum
+// One histogram per block of SPEC_THREADS threads: the partial rows limit the
+// blocks to about one per CU, so a block is 16 waves (with 4 the loads waited on
+// the shell sums: 109 us at 256^3 FP32).
+constexpr int SPEC_THREADS = 1024;
 template <typename Rt>
-__global__ void __launch_bounds__(256) k_spectrum(EwArgs<Rt> a, int nb, double* __restrict__ part) {
+__global__ void __launch_bounds__(SPEC_THREADS) k_spectrum(EwArgs<Rt> a, int nb, double* __restrict__ part) {
   using C = cx<Rt>;
   extern __shared__ double hist[];  // [2][nb]: uiui sums, counts
-  for (int b = threadIdx.x; b < 2 * nb; b += 256) hist[b] = 0.0;
+  for (int b = threadIdx.x; b < 2 * nb; b += SPEC_THREADS) hist[b] = 0.0;
   __syncthreads();
   const long n = a.n;
-  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    const int kz = (int)(i % a.Nh);
-    const long r = i / a.Nh;
-    const int iy = (int)(r % a.N1);
-    const int ix = (int)(r / a.N1);
+  for (long i = (long)blockIdx.x * SPEC_THREADS + threadIdx.x; i < n; i += (long)gridDim.x * SPEC_THREADS) {
+    const Mode md = mode_of(i, a.N1, a.Nh);
+    const int ix = md.ix, iy = md.iy, kz = md.kz;
     const Rt K0 = a.kx[ix], K1 = a.ky[iy], K2 = a.kz[kz];
     Rt k2 = K0 * K0;
     k2 += K1 * K1;
@@ -779,11 +782,11 @@ __global__ void __launch_bounds__(256) k_spectrum(EwArgs<Rt> a, int nb, double* 
     atomicAdd(&hist[nb + z - 1], 1.0);
   }
   __syncthreads();
-  for (int b = threadIdx.x; b < 2 * nb; b += 256) part[(long)blockIdx.x * 2 * nb + b] = hist[b];
+  for (int b = threadIdx.x; b < 2 * nb; b += SPEC_THREADS) part[(long)blockIdx.x * 2 * nb + b] = hist[b];
 }
 
 template <typename Rt> int launch_spectrum(const EwArgs<Rt>& a, int nb, double* partials, int nblk, hipStream_t s) {
-  hipLaunchKernelGGL((k_spectrum<Rt>), dim3(nblk), dim3(256), 2 * nb * sizeof(double), s, a, nb, partials);
+  hipLaunchKernelGGL((k_spectrum<Rt>), dim3(nblk), dim3(SPEC_THREADS), 2 * nb * sizeof(double), s, a, nb, partials);
   return 0;
 }
 

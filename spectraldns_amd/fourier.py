@@ -168,6 +168,7 @@ def spectrum(u_hat, T, N=None):
     Returns (Ek, bins) as NumPy arrays with the reference's definition: shells
     (k - 1/2, k + 1/2] for k = 1..Nb-1 with Nb = int(sqrt(sum((N/2)^2)/3)),
     Ek = (k_hi^3 - k_lo^3) * (4 pi/3) * sum(uiui) / count, Ek[Nb-1] = 0."""
+    import torch
     plan = T.plan
     N = np.array(plan.N if N is None else N)
     Nb = int(np.sqrt(np.sum((N / 2) ** 2) / 3))
@@ -175,12 +176,9 @@ def spectrum(u_hat, T, N=None):
     Ek = np.zeros(Nb)
     if Nb < 2:
         return Ek, bins
-    sums, counts = plan.spectrum_sums(u_hat.contiguous(), Nb - 1)
-    sums = sums.cpu().numpy() * (4.0 / 3.0 * np.pi)
-    counts = counts.cpu().numpy()
-    for i, k in enumerate(bins[1:]):
-        k0 = bins[i]
-        Ek[i] = (k ** 3 - k0 ** 3) * sums[i]
-        if counts[i] != 0:
-            Ek[i] = Ek[i] / counts[i]
+    out = torch.empty(2 * (Nb - 1), dtype=torch.float64, device=u_hat.device)
+    plan.spectrum_sums(u_hat.contiguous(), Nb - 1, out)
+    out = out.cpu().numpy()
+    sums, counts = out[:Nb - 1] * (4.0 / 3.0 * np.pi), out[Nb - 1:]
+    Ek[:-1] = (bins[1:] ** 3 - bins[:-1] ** 3) * sums / np.where(counts != 0, counts, 1)
     return Ek, bins
