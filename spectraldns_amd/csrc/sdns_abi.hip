@@ -90,6 +90,7 @@ struct sdns_plan {
   hipStream_t stream = nullptr;
   int in[3][2], out[3][2];
   int nky, nkz, nkyo, nkzo;
+  int nkz4;         // kz stride of W4
   int nkzp, nkzop;  // kz strides of the work buffers, padded to 16 elements
   bool plane = false;  // P2, P3 and P4 run as one launch per evaluation (sdns_plane.hpp)
   int var[6] = {0, 0, 0, 0, 0, 0};  // schedule variant per pass (see sdns_plan_set_variant)
@@ -213,11 +214,12 @@ void compute_sizes(sdns_plan* p) {
   const size_t M0 = p->M[0], M1 = p->M[1];
   const size_t state = 3ull * p->N[0] * p->N[1] * p->Nh;
   // W1 holds 6 fields when the vorticity is given (sdns_convection_uw)
-  const size_t w1 = 6ull * M0 * p->nky * p->nkzp, w3 = 3ull * M0 * M1 * p->nkzop;
-  const size_t w2 = 6ull * M0 * M1 * p->nkzp, w4 = 3ull * M0 * p->nkyo * p->nkzop;
+  const size_t w1 = 6ull * ((M0 + XB - 1) / XB * XB) * p->nky * p->nkzp, w3 = 3ull * M0 * M1 * p->nkzop;
+  const size_t w2 = 6ull * M0 * M1 * p->nkzp, w4 = 3ull * M0 * p->nkyo * p->nkzop;  // (nkz4 <= nkzop)
   p->szA = align256(std::max(std::max(w1, w3), state) * e);
   p->szB = align256(std::max(std::max(w2, w4), state) * e);
-  p->szS = align256(state * e);
+  const size_t tw = 128 / e;  // (stage arrays are tile-major)
+  p->szS = align256(3ull * p->N[0] * ((p->N[1] * p->Nh + tw - 1) / tw * tw) * e);
   // P5 blocks: columns N1*Nh over the smallest tile of the supported lengths
   p->max_blocks = p->N[1] * p->Nh;  // upper bound (>= 1 column per block)
   p->szPart = align256((size_t)std::max(p->max_blocks, 4096) * 2 * sizeof(double) + 4096);
@@ -230,6 +232,15 @@ void plan_layout(sdns_plan* p, bool plane) {
   p->plane = plane;
   p->nkzp = plane ? p->nkz : (p->nkz + 15) / 16 * 16;
   p->nkzop = plane ? p->nkzo : (p->nkzo + 15) / 16 * 16;
+  // W4 unpadded: its columns are the state's (every ky is kept unless mode 1
+  // truncates), so the x-forward tiles read whole lines, and the y-forward's
+  // tiles, which then straddle lines, store through the caches.  Measured while
+  // the three fields stay within about the last-level cache (256^3 FP32 3/2
+  // rule: y-forward 151 -> 132 us, step 4.95 -> 4.88 ms; 192^3 FP64 1.95 -> 1.93);
+  // larger ones lose more in the x-forward (384^3 FP32 7.06 -> 7.24 ms, 256^3 FP64
+  // 10.55 -> 10.69).
+  const size_t w4 = 3ull * p->M[0] * p->nkyo * p->nkzo * p->esz;
+  p->nkz4 = w4 <= (320ull << 20) ? p->nkzo : p->nkzop;
   compute_sizes(p);
 }
 
@@ -255,7 +266,7 @@ int default_variant(int pass, int len, int precision) {
       if (f32) return len == 256 ? 3 : (len == 512 ? 1 : (len >= 36 ? 2 : 0));
       return in({96, 192}) ? 2 : 0;
     case 3: return f32 ? 0 : in({128});
-    case 4: return f32 ? in({64, 128, 384, 512}) : in({128, 384});
+    case 4: return f32 ? in({64, 128, 384, 512}) : in({128});
     default: return 0;
   }
 }
@@ -451,7 +462,7 @@ template <typename Rt> StridedArgs<Rt> p4_args(const sdns_plan* p) {
   a.in = p->bufA; a.out = p->bufB; a.tw = p->tw.at(M1);
   a.Q = M0 * p->nkzop; a.cdiv = p->nkzop; a.cvalid = p->nkzo;
   a.in_hi = (long)M1 * p->nkzop; a.in_row = p->nkzop; a.in_field = (long)M0 * M1 * p->nkzop;
-  a.out_hi = (long)p->nkyo * p->nkzop; a.out_row = p->nkzop; a.out_field = (long)M0 * p->nkyo * p->nkzop;
+  a.out_hi = (long)p->nkyo * p->nkz4; a.out_row = p->nkz4; a.out_field = (long)M0 * p->nkyo * p->nkz4;
   a.rin = rmap(M1 / 2, M1 - M1 / 2 - 1, M1);
   a.rout = rmap(p->out[1][0], p->out[1][1], p->nkyo);
   a.scale = Rt(1);
@@ -487,9 +498,10 @@ template <typename Rt> PlaneArgs<Rt> plane_args(const sdns_plan* p) {
 // P1..P4 of one convection evaluation from the state of a1 into W4 (= bufB).  a1.w:
 // the vorticity of u when given (the velocity-vorticity solver), otherwise
 // null and the passes form curl(u).
-template <typename Rt> int conv_passes(sdns_plan* p, const P1Args<Rt>& a1) {
+template <typename Rt> int conv_passes(sdns_plan* p, P1Args<Rt> a1) {
   const int M0 = p->M[0], M1 = p->M[1];
   const void* w = a1.w;
+  a1.xb = !w && !p->plane;  // the y pass of a given vorticity and the plane kernel read plain rows
   tstart(p, 0);
   if (launch_p1<Rt>(M0, p->var[0], a1, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", M0);
   tstop(p);
@@ -505,8 +517,10 @@ template <typename Rt> int conv_passes(sdns_plan* p, const P1Args<Rt>& a1) {
   if (w) {
     if (launch_strided<Rt>(M1, p->var[1], +1, 6, p2_given_args<Rt>(p), p->stream))
       return fail(SDNS_ERR_UNSUPPORTED, "y length %d", M1);
-  } else if (launch_p2<Rt>(M1, p->var[1], p2_args<Rt>(p), p->stream)) {
-    return fail(SDNS_ERR_UNSUPPORTED, "y length %d", M1);
+  } else {
+    P2Args<Rt> a2 = p2_args<Rt>(p);
+    a2.xb = a1.xb;
+    if (launch_p2<Rt>(M1, p->var[1], a2, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "y length %d", M1);
   }
   tstop(p);
   tstart(p, 2);
@@ -526,7 +540,7 @@ template <typename Rt> P5Args<Rt> p5_args(const sdns_plan* p, double nu) {
   a.kx = (const Rt*)p->ktab[0]; a.ky = (const Rt*)p->ktab[1]; a.kz = (const Rt*)p->ktab[2];
   a.N0 = p->N[0]; a.N1 = p->N[1]; a.Nh = p->Nh; a.N2 = p->N[2];
   a.x = rmap(p->out[0][0], p->out[0][1], p->N[0]);
-  a.y_neg = p->out[1][0]; a.y_pos = p->out[1][1]; a.nkzo = p->nkzo; a.nkzop = p->nkzop;
+  a.y_neg = p->out[1][0]; a.y_pos = p->out[1][1]; a.nkzo = p->nkzo; a.nkzop = p->nkz4;
   a.mask_nyquist = p->mask_nyquist;
   a.nu = (Rt)nu;
   a.scale = (Rt)(1.0 / ((double)p->M[0] * p->M[1] * p->M[2]));
@@ -541,23 +555,27 @@ template <typename Rt> struct RkStage {
   static Rt a(int rk) { return rk == 0 || rk == 3 ? Rt(1. / 6.) : Rt(1. / 3.); }
   static Rt b(int rk) { return rk < 2 ? Rt(0.5) : Rt(1); }
   static int mode(int rk) { return rk == 0 ? P5_RK0 : (rk < 3 ? P5_RK12 : P5_RK3); }
-  static void p5(P5Args<Rt>& x, int keep, int rk, Rt dt, void* u, char* const st[3]) {
+  // tiled: the stage arrays are tile-major
+  static void p5(P5Args<Rt>& x, int keep, int rk, Rt dt, void* u, char* const st[3], int tiled) {
     const int n = keep == KEEP_SUM ? 1 : 3;  // KEEP_SUM: one stage state, st[0], and the sum, st[1]
     x.u = u;
     x.s = rk > 0 ? st[(rk - 1) % n] : nullptr;
     x.out = rk < 3 ? st[rk % n] : nullptr;
     x.b1 = keep == KEEP_SUM ? st[1] : st[0];
     x.b2 = st[1];
+    x.st_tiled = tiled;
     x.adt = a(rk) * dt;
     x.bdt = b(rk) * dt;
     x.sdt = rk > 0 ? b(rk - 1) * dt : Rt(0);
     x.a12 = a(1) * dt;
   }
   // the state that stage rk's RHS reads
-  static void p1(P1Args<Rt>& x, int keep, int rk, Rt dt, const void* u, char* const st[3]) {
+  static void p1(P1Args<Rt>& x, int keep, int rk, Rt dt, const void* u, char* const st[3], int tiled) {
     const void* s = rk > 0 ? st[keep == KEEP_SUM ? 0 : rk - 1] : nullptr;
     x.u = s && keep != KEEP_RHS ? s : u;
     x.d = keep == KEEP_RHS ? s : nullptr;
+    x.u_tiled = x.u != u && tiled;
+    x.d_tiled = x.d && tiled;
     x.ds = rk > 0 ? b(rk - 1) * dt : Rt(0);
   }
 };
@@ -594,12 +612,13 @@ bool fused_stages(const sdns_plan* p) {
 }
 
 // One right-hand side of the vorticity w and its stage (mode) into a's arrays.
-template <typename Rt> int vv_stage(sdns_plan* p, const void* w, int mode, const P5Args<Rt>& a) {
+template <typename Rt> int vv_stage(sdns_plan* p, const void* w, int tiled, int mode, const P5Args<Rt>& a) {
   P1Args<Rt> a1 = p1_args<Rt>(p, w);
   a1.w = w;
   a1.ky = (const Rt*)p->ktab[1];
   a1.kz = (const Rt*)p->ktab[2];
   a1.curl_inv = 1;
+  a1.w_tiled = tiled;
   int rc;
   if ((rc = conv_passes<Rt>(p, a1))) return rc;
   if (launch_p5vv<Rt>(p->M[0], mode, a, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", p->M[0]);
@@ -608,16 +627,16 @@ template <typename Rt> int vv_stage(sdns_plan* p, const void* w, int mode, const
 template <typename Rt> int vv_rhs(sdns_plan* p, const void* w, void* rhs, double nu, const void* src) {
   P5Args<Rt> a = p5_args<Rt>(p, nu);
   a.u = const_cast<void*>(w); a.rhs = rhs; a.source = src;
-  return vv_stage<Rt>(p, w, P5_RHS, a);
+  return vv_stage<Rt>(p, w, 0, P5_RHS, a);
 }
 template <typename Rt> int vv_rk4_steps(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* src) {
   using RK = RkStage<Rt>;
   for (int s = 0; s < nsteps; ++s)
     for (int rk = 0; rk < 4; ++rk) {
       P5Args<Rt> a = p5_args<Rt>(p, nu);
-      RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], w, p->st);
+      RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], w, p->st, 1);
       a.source = src;
-      const int rc = vv_stage<Rt>(p, rk == 0 ? w : p->st[rk - 1], RK::mode(rk), a);
+      const int rc = vv_stage<Rt>(p, rk == 0 ? w : p->st[rk - 1], rk > 0, RK::mode(rk), a);
       if (rc) return rc;
     }
   return 0;
@@ -701,7 +720,7 @@ template <typename Rt> int mhd_rk4_steps(sdns_plan* p, void* ub, const double* d
       const void* in[2];
       for (int h = 0; h < 2; ++h) {
         P5Args<Rt> a{};
-        RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], (char*)ub + h * half, st[h]);
+        RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], (char*)ub + h * half, st[h], 0);
         x.u[h] = a.u; x.s[h] = a.s; x.out[h] = a.out; x.b1[h] = a.b1; x.b2[h] = a.b2;
         x.adt = a.adt; x.bdt = a.bdt;
         in[h] = rk == 0 ? a.u : a.s;
@@ -767,13 +786,14 @@ template <typename Rt> int rk4_steps(sdns_plan* p, void* u, void* ulo, const dou
                                       float in_scale = 1.f, float out_scale = 1.f, int per_stage = 0) {
   using RK = RkStage<Rt>;
   const int keep = rk_keep<Rt>(p->M[0] != p->N[0], ulo != nullptr);
+  const int tiled = !(cl && per_stage);  // (the closure's transforms read a stage state as an array)
   const Rt nur = (Rt)nu;
   for (int s = 0; s < nsteps; ++s) {
     const Rt dt = (Rt)dts[s];
     for (int rk = 0; rk < 4; ++rk) {
       int rc;
       P1Args<Rt> a1 = p1_args<Rt>(p, u);
-      RK::p1(a1, keep, rk, dt, u, p->st);
+      RK::p1(a1, keep, rk, dt, u, p->st, tiled);
       if (cl && (per_stage || rk == 0)) {
         const void* state = a1.u;
         if (a1.d) {  // the closure's transform reads the stage state as an array
@@ -784,7 +804,7 @@ template <typename Rt> int rk4_steps(sdns_plan* p, void* u, void* ulo, const dou
       }
       if ((rc = conv_passes<Rt>(p, a1))) return rc;
       P5Args<Rt> pa = p5_args<Rt>(p, nu);
-      RK::p5(pa, keep, rk, dt, u, p->st);
+      RK::p5(pa, keep, rk, dt, u, p->st, tiled);
       pa.lo = ulo;
       pa.source = cl ? (const void*)cl->src : src;
       const int mode = RK::mode(rk);
@@ -1127,7 +1147,7 @@ template <typename Rt> int batch_upload(sdns_batch* b) {
     const int keep = rk_keep<Rt>(p->M[0] != p->N[0], false);
     for (int rk = 0; rk < 4; ++rk) {
       h1[rk].push_back(p1_args<Rt>(p, b->u[i]));
-      RkStage<Rt>::p1(h1[rk].back(), keep, rk, dt, b->u[i], p->st);
+      RkStage<Rt>::p1(h1[rk].back(), keep, rk, dt, b->u[i], p->st, 1);
     }
     h2.push_back(p2_args<Rt>(p));
     h3.push_back(p3_args<Rt>(p));
@@ -1140,7 +1160,7 @@ template <typename Rt> int batch_upload(sdns_batch* b) {
     }
     for (int rk = 0; rk < 4; ++rk) {
       P5Args<Rt> pa = p5_args<Rt>(p, b->nu[i]);
-      RkStage<Rt>::p5(pa, keep, rk, dt, b->u[i], p->st);
+      RkStage<Rt>::p5(pa, keep, rk, dt, b->u[i], p->st, 1);
       pa.partials = rk == 3 ? b->d_part + b->poff[i] : nullptr;
       h5[rk].push_back(pa);
     }

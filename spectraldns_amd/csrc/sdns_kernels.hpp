@@ -119,17 +119,27 @@ __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, c
   const bool given = a.w != nullptr;
   const int comp = given ? yb % 3 : 2 - yb;
   const long plane = (long)a.N1 * a.Nh;
-  const C* __restrict__ U = (const C*)(given && yb >= 3 ? a.w : a.u) + (long)comp * a.N0 * plane +
-                            (valid ? (long)iy * a.Nh + kzi : 0);
+  // component c of a state-shaped array at this column, and its row stride
+  constexpr int TW = tile_w<Rt>();
+  const int qs = valid ? iy * a.Nh + kzi : 0;
+  auto column = [&](const void* p, int c, int tiled) {
+    return (const C*)p + (tiled ? ((long)c * tiled_cols<Rt>(a.N1 * a.Nh) + qs / TW * TW) * a.N0 + qs % TW
+                                : (long)c * a.N0 * plane + qs);
+  };
+  auto stride = [&](int tiled) { return tiled ? (long)TW : plane; };
+  const int ut = given && yb >= 3 ? a.w_tiled : a.u_tiled;
+  const C* __restrict__ U = column(given && yb >= 3 ? a.w : a.u, comp, ut);
+  const long us = stride(ut);
   C v[E];
   if constexpr (INC) {
-    const C* __restrict__ D = (const C*)a.d + (U - (const C*)a.u);
+    const C* __restrict__ D = column(a.d, comp, a.d_tiled);
+    const long ds = stride(a.d_tiled);
     C d[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int r = bin_row(t + P * e, M, a.x);
-      v[e] = (valid && r >= 0) ? U[r * plane] : czero<C>();
-      d[e] = (valid && r >= 0) ? D[r * plane] : czero<C>();
+      v[e] = (valid && r >= 0) ? U[r * us] : czero<C>();
+      d[e] = (valid && r >= 0) ? D[r * ds] : czero<C>();
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = caxpy(v[e], a.ds, d[e]);
@@ -137,15 +147,15 @@ __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, c
     // velocity component `comp` of the vorticity: i (o_j w_k - o_k w_j), o = K / K^2,
     // K^2 = 0 taken as 1 (solvers/VV.py:71-72)
     const int cj = (comp + 1) % 3, ck = (comp + 2) % 3;
-    const C* __restrict__ B = (const C*)a.w + (valid ? (long)iy * a.Nh + kzi : 0);
-    const C *Wj = B + (long)cj * a.N0 * plane, *Wk = B + (long)ck * a.N0 * plane;
+    const C *Wj = column(a.w, cj, a.w_tiled), *Wk = column(a.w, ck, a.w_tiled);
+    const long ws = stride(a.w_tiled);
     const Rt K1 = a.ky[valid ? iy : 0], K2 = a.kz[valid ? kzi : 0];
     C d[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int r = bin_row(t + P * e, M, a.x);
-      v[e] = (valid && r >= 0) ? Wk[r * plane] : czero<C>();
-      d[e] = (valid && r >= 0) ? Wj[r * plane] : czero<C>();
+      v[e] = (valid && r >= 0) ? Wk[r * ws] : czero<C>();
+      d[e] = (valid && r >= 0) ? Wj[r * ws] : czero<C>();
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -162,7 +172,7 @@ __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, c
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int r = bin_row(t + P * e, M, a.x);
-      v[e] = (valid && r >= 0) ? U[r * plane] : czero<C>();
+      v[e] = (valid && r >= 0) ? U[r * us] : czero<C>();
     }
   }
   __syncthreads();
@@ -170,6 +180,17 @@ __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, c
   const long orow = a.Q, ofield = (long)M * a.Q;
   C* line = lds + c;
   auto store = [&](int f, C(&x)[E]) {
+    if (valid && a.xb) {
+      // row p of block p / XB, at p % XB within the columns of its ky
+      constexpr long MB = (M + XB - 1) / XB * XB;
+      C* __restrict__ o = (C*)a.w1 + f * MB * orow + (long)iyc * XB * a.nkzp + kzi;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int p = t + P * e;
+        o[(long)(p / XB) * XB * orow + p % XB * a.nkzp] = x[e];
+      }
+      return;
+    }
     if (valid) {
 #pragma unroll
       for (int e = 0; e < E; ++e) out[f * ofield + (long)(t + P * e) * orow] = x[e];
@@ -231,10 +252,11 @@ __device__ __forceinline__ void p2_body(const P2Args<Rt>& a, int tile, int yb, c
   const int x = q / a.nkzp, kzi = q - x * a.nkzp;
   const bool valid = q < a.Q && kzi < a.nkz;
   const int nky = a.y.base;
-  const long ifield = (long)a.M0 * nky * a.nkzp, ofield = (long)a.M0 * M * a.nkzp;
-  const C* __restrict__ in = (const C*)a.w1 + (valid ? (long)x * nky * a.nkzp + kzi : 0);
+  const long ifield = (long)(a.xb ? (a.M0 + XB - 1) / XB * XB : a.M0) * nky * a.nkzp, ofield = (long)a.M0 * M * a.nkzp;
+  const long xoff = a.xb ? ((long)(x / XB) * nky * XB + x % XB) * a.nkzp : (long)x * nky * a.nkzp;
+  const C* __restrict__ in = (const C*)a.w1 + (valid ? xoff + kzi : 0);
   C* __restrict__ out = (C*)a.w2 + (long)x * M * a.nkzp + kzi;
-  const int rs = a.nkzp;
+  const int rs = a.nkzp, irs = a.xb ? XB * a.nkzp : a.nkzp;
   const Rt kzv = a.kz[valid ? kzi : 0];
   C* line = lds + c;
   auto row = [&](int e) { return valid ? bin_row(t + P * e, M, a.y) : -1; };
@@ -247,7 +269,7 @@ __device__ __forceinline__ void p2_body(const P2Args<Rt>& a, int tile, int yb, c
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int r = row(e);
-      v[e] = r >= 0 ? ld_pass<STREAM>(in + f * ifield + (long)r * rs) : czero<C>();
+      v[e] = r >= 0 ? ld_pass<STREAM>(in + f * ifield + (long)r * irs) : czero<C>();
     }
   };
   auto store = [&](int f, C(&v)[E]) {
@@ -1023,6 +1045,10 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
   constexpr bool LOAD_B1 = MODE == P5_RK3 || (SUM && MODE == P5_RK12);
   constexpr bool LOAD_B2 = MODE == P5_RK3 && !SUM;
   constexpr bool LOAD_L = COMP && MODE == P5_RK3;
+  // stage arrays: component stride, row stride and column offset
+  constexpr int TW = tile_w<Rt>();
+  const long sfs = a.st_tiled ? (long)a.N0 * tiled_cols<Rt>(a.Q) : fs, srow = a.st_tiled ? TW : plane;
+  const long scol = a.st_tiled ? (long)(q / TW) * TW * a.N0 + q % TW : q;
 #pragma unroll
   for (int e0 = 0; e0 < E; e0 += G) {
     int ixs[G];
@@ -1052,9 +1078,10 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
       for (int i = 0; i < 3; ++i) {
         if constexpr (LOAD_U) su[g][i] = Uin[i * fs + off];
         if (src) sr[g][i] = src[i * fs + off];
-        if constexpr (LOAD_S) ss[g][i] = Sin[i * fs + off];
-        if constexpr (LOAD_B1) x1[g][i] = B1in[i * fs + off];
-        if constexpr (LOAD_B2) x2[g][i] = B2in[i * fs + off];
+        const long so = i * sfs + ix * srow + scol;
+        if constexpr (LOAD_S) ss[g][i] = Sin[so];
+        if constexpr (LOAD_B1) x1[g][i] = B1in[so];
+        if constexpr (LOAD_B2) x2[g][i] = B2in[so];
         if constexpr (LOAD_L) xl[g][i] = Lin[i * fs + off];
       }
     }
@@ -1105,8 +1132,9 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
         C* out = (C*)a.out;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-          st_pass<STREAM>(out + (i * fs + off), KEEP == KEEP_RHS ? r[i] : caxpy(su[g][i], a.bdt, r[i]));
-          if constexpr (SUM) st_pass<STREAM>((C*)a.b1 + (i * fs + off), caxpy(MODE == P5_RK0 ? su[g][i] : x1[g][i], a.adt, r[i]));
+          const long so = i * sfs + ix * srow + scol;
+          st_pass<STREAM>(out + so, KEEP == KEEP_RHS ? r[i] : caxpy(su[g][i], a.bdt, r[i]));
+          if constexpr (SUM) st_pass<STREAM>((C*)a.b1 + so, caxpy(MODE == P5_RK0 ? su[g][i] : x1[g][i], a.adt, r[i]));
         }
       } else {
         C* un = (C*)a.u;
@@ -1222,14 +1250,22 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
   const int nyq_ix = a.mask_nyquist ? a.N0 / 2 : -1;
   const double wz = (kz == 0 || kz == a.N2 / 2) ? 1.0 : 2.0;
   double esum = 0.0, osum = 0.0;
-  const auto ru = buf_rsrc(SUM && MODE == P5_RK3 ? a.s : a.u, span);
-  const auto rs = buf_rsrc(SUM && MODE == P5_RK3 ? a.b1 : a.s, span);
-  const auto rb1 = buf_rsrc(a.b1, span);
-  const auto rb2 = buf_rsrc(a.b2, span);
+  // stage arrays: row stride, component stride, span and this lane's offset; the
+  // first array is one with KEEP_SUM in stage 3, else it is u
+  constexpr int TW = tile_w<Rt>();
+  constexpr bool FIRST_S = SUM && MODE == P5_RK3;
+  const int srow = a.st_tiled ? TW : plane, sfs = a.st_tiled ? a.N0 * tiled_cols<Rt>(a.Q) : fs;
+  const long sspan = 3L * sfs * CS;
+  const int sso = a.st_tiled ? (q / TW * TW * a.N0 + q % TW + t * TW) * CS : so;
+  const auto ru = buf_rsrc(FIRST_S ? a.s : a.u, FIRST_S ? sspan : span);
+  const auto rs = buf_rsrc(FIRST_S ? a.b1 : a.s, sspan);
+  const auto rb1 = buf_rsrc(a.b1, sspan);
+  const auto rb2 = buf_rsrc(a.b2, sspan);
   const auto rlo = buf_rsrc(a.lo, span);
   const auto rsrc = buf_rsrc(a.source, a.source ? span : 0L);
   const auto rph = buf_rsrc(a.phat, a.phat ? (long)fs * CS : 0L);
-  const auto ro = buf_rsrc(MODE == P5_RHS ? a.rhs : (MODE == P5_RK3 ? a.u : a.out), span);
+  constexpr bool OUT_S = MODE == P5_RK0 || MODE == P5_RK12;
+  const auto ro = buf_rsrc(MODE == P5_RHS ? a.rhs : (MODE == P5_RK3 ? a.u : a.out), OUT_S ? sspan : span);
   if (valid) {
     C cur[G][NL + 1][3], nxt[G][NL + 1][3];  // state arrays, then the source
     Rt kcur[G], knxt[G];
@@ -1240,11 +1276,11 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
         kd[g] = a.kx[t + P * (j0 + g)];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-          const int o = (i * fs + eo) * CS;
-          d[g][0][i] = buf_load_so<C>(ru, so, o);
-          if constexpr (NL > 1) d[g][1][i] = buf_load_so<C>(rs, so, o);
-          if constexpr (NL > 2) d[g][2][i] = buf_load_so<C>(rb1, so, o);
-          if constexpr (NL > 3) d[g][3][i] = buf_load_so<C>(rb2, so, o);
+          const int o = (i * fs + eo) * CS, os = (i * sfs + P * (j0 + g) * srow) * CS;
+          d[g][0][i] = buf_load_so<C>(ru, FIRST_S ? sso : so, FIRST_S ? os : o);
+          if constexpr (NL > 1) d[g][1][i] = buf_load_so<C>(rs, sso, os);
+          if constexpr (NL > 2) d[g][2][i] = buf_load_so<C>(rb1, sso, os);
+          if constexpr (NL > 3) d[g][3][i] = buf_load_so<C>(rb2, sso, os);
           if constexpr (NL > 4) d[g][4][i] = buf_load_so<C>(rlo, so, o);
           d[g][NL][i] = buf_load_so<C>(rsrc, so, o);
         }
@@ -1289,7 +1325,7 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
           if constexpr (!VV) x = mk<C>(x.x - ph.x * Kv[i], x.y - ph.y * Kv[i]);
           x = mk<C>(x.x - z * st.x, x.y - z * st.y);
           x = cadd(x, d[NL][i]);  // rhs += Source (NS.py:256-258), every mode
-          const int o = (i * fs + eo) * CS;
+          const int o = (i * fs + eo) * CS, os = (i * sfs + P * j * srow) * CS;
           if constexpr (MODE == P5_RK3) {
             C l = d[NL > 4 ? 4 : 0][i];
             x = rk_last<KEEP, COMP>(a, u, SUM ? s : d[NL > 2 ? 2 : 0][i], d[NL > 3 ? 3 : 0][i], s, x, l);
@@ -1302,10 +1338,10 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
             }
           } else if constexpr (MODE != P5_RHS && KEEP != KEEP_RHS) {
             if constexpr (SUM)
-              buf_store_so_nt<C>(caxpy(d[MODE == P5_RK0 ? 0 : (NL > 2 ? 2 : 0)][i], a.adt, x), rb1, so, o);
+              buf_store_so_nt<C>(caxpy(d[MODE == P5_RK0 ? 0 : (NL > 2 ? 2 : 0)][i], a.adt, x), rb1, sso, os);
             x = caxpy(u, a.bdt, x);
           }
-          buf_store_so_nt<C>(x, ro, so, o);
+          buf_store_so_nt<C>(x, ro, OUT_S ? sso : so, OUT_S ? os : o);
         }
         if constexpr (!VV && (MODE == P5_RHS || MODE == P5_RK3)) buf_store_so_nt<C>(ph, rph, so, eo * CS);
         if constexpr (MODE == P5_RK3) energy_terms(v, Kv[0], K1, K2c, wz, esum, osum);

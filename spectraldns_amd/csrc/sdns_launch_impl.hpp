@@ -109,7 +109,7 @@ template <typename Rt, int n, int E> void p3c_go(const P3Args<Rt>& a, hipStream_
 // most BUF_OOB bytes (boxes up to about 640^3 in FP32).  Larger boxes run k_p5.
 template <typename Rt> bool p5b_fits(int M, int N0, int N1, int Nh, int nkyo, int nkzop) {
   const long esz = 2 * (long)sizeof(Rt);
-  return 3L * N0 * N1 * Nh * esz <= BUF_OOB && 3L * M * nkyo * nkzop * esz <= BUF_OOB;
+  return 3L * N0 * tiled_cols<Rt>(N1 * Nh) * esz <= BUF_OOB && 3L * M * nkyo * nkzop * esz <= BUF_OOB;
 }
 template <typename Rt> bool p5b_fits(int M, const P5Args<Rt>& a) {
   return p5b_fits<Rt>(M, a.N0, a.N1, a.Nh, a.y_neg + a.y_pos + 1, a.nkzop);
@@ -136,22 +136,15 @@ template <typename Rt, int M, int E, int MODE, bool PAD> void p5b_go(const P5Arg
     hipLaunchKernelGGL((k_p5b<Rt, M, E, MODE, PAD, false, D>), dim3(xcd_grid(nt)), dim3(Cfg::THREADS / D), 0, s, a);
   });
 }
-// Stages 1 and 2 with the accumulator (FP32, 3/2 rule: ten mixed read and write
-// streams) run p5_body: 0.313 ms at 256^3 against 0.336 ms of p5b_body, whose
-// prefetch only adds streams there; stages 0 and 3 take 0.246 against 0.248 and
-// 0.241 against 0.247 ms.
 template <typename Rt, int M, int V, int MODE> void p5_go(const P5Args<Rt>& a, hipStream_t s, int* nblk) {
   constexpr int EV = strided_E(M, V);
-  constexpr bool PADB = M % 3 == 0 && EV % 3 == 0;
-  constexpr bool PAD_SUM = PADB && MODE == P5_RK12 && rk_keep<Rt>(true, false) == KEEP_SUM;
   const bool fits = p5b_fits(M, a);
   if (fits && M == a.N0) return p5b_go<Rt, M, EV, MODE, false>(a, s, nblk);
-  if constexpr (PADB && !PAD_SUM) {
+  if constexpr (M % 3 == 0 && EV % 3 == 0) {
     // (the compensated stages of the 3/2 rule run p5_body)
     if (fits && p5b_padded(M, a) && (!a.lo || MODE == P5_RHS)) return p5b_go<Rt, M, EV, MODE, true>(a, s, nblk);
   }
-  // one schedule for the boxes beyond a descriptor's reach
-  constexpr int E0 = PAD_SUM ? EV : strided_E(M, 0);
+  constexpr int E0 = strided_E(M, 0);  // one schedule for the boxes beyond a descriptor's reach
   using Cfg = SCfg<Rt, M, E0>;
   const int nt = (a.Q + Cfg::T - 1) / Cfg::T;
   if (nblk) *nblk = nt;

@@ -43,6 +43,8 @@ template <typename Rt> struct P1Args {  // x-inverse of u_hat + kx products
   int nkz, nkzp;      // kept input kz count, padded kz stride of W1
   int Q;              // nky * nkzp columns (= W1 row stride)
   Rt ds;
+  int u_tiled, d_tiled, w_tiled;  // stage arrays (tile-major)
+  int xb;             // W1 blocked over x
 };
 
 template <typename Rt> struct P2Args {  // y-inverse + curl assembly
@@ -55,6 +57,7 @@ template <typename Rt> struct P2Args {  // y-inverse + curl assembly
   RowMap y;           // kept input modes of axis 1 (base = nky)
   int nkz, nkzp;
   int Q;              // M0 * nkzp
+  int xb;             // W1 blocked over x
 };
 
 template <typename Rt> struct P3Args {  // z C2R x6, cross product, z R2C x3
@@ -94,6 +97,20 @@ template <typename Rt> struct ZArgs {
   long in_line, in_field, out_line, out_field;  // element strides
   Rt scale;
 };
+
+// Layouts for the x passes, whose blocks walk a column tile through every x:
+// with x slowest, each row is 0.2 to 0.6 MB from the next, and the passes ran at
+// 4.0 TB/s where the y passes reach 5.3 (wider tiles did not help, data resident
+// in the last-level cache did not either: address translation).
+//   RK stage arrays, which only the x passes touch, are tile-major:
+//     [3][tile][N0][TW], TW = 128 bytes of columns, so that a block's rows are
+//     contiguous;
+//   W1 (not with a given vorticity) is blocked over x: [5][M0/XB][nky][XB][nkzp].
+// 256^3, before -> after: x-inverse FP64 3/2 rule 367 -> 307 us, FP32 160 -> 143;
+// x-forward + RK FP64 466 -> 442; 512^3 FP32 1800 -> 1600.
+template <typename Rt> constexpr int tile_w() { return 128 / (2 * (int)sizeof(Rt)); }
+template <typename Rt> constexpr int tiled_cols(int Q) { return (Q + tile_w<Rt>() - 1) / tile_w<Rt>() * tile_w<Rt>(); }
+constexpr int XB = 16;
 
 enum P5Mode { P5_RHS = 0, P5_RK0 = 1, P5_RK12 = 2, P5_RK3 = 3 };
 
@@ -136,6 +153,7 @@ template <typename Rt> struct P5Args {  // x-forward + mask + pressure + diffusi
   int y_neg, y_pos;   // kept output modes of axis 1
   int nkzo, nkzop;    // kept output kz count, padded kz stride of W4
   int mask_nyquist;
+  int st_tiled;       // s, out, b1, b2 are tile-major
   int conv_only;      // P5_RHS: write the scaled convection term only
   Rt nu, scale;
   Rt adt, bdt;        // a dt and b dt of this stage
