@@ -128,6 +128,7 @@ struct sdns_closure {
   float *y = nullptr, *wpart = nullptr, *gsum = nullptr;
   float *phys = nullptr, *tauphys = nullptr;
   char *tauhat = nullptr, *src = nullptr;  // 6 and 3 complex64 spectral fields
+  char *fftA = nullptr, *fftB = nullptr;   // 6 fields each: intermediates of tau's transform
   char* stage = nullptr;                   // 3 fields: the stage state of per-stage evaluations (in tauhat)
   double* lpart = nullptr;
   sdns::ClosureWeights w{};
@@ -348,21 +349,24 @@ template <typename Rt> int plain_backward(sdns_plan* p, const void* uh, void* up
   return 0;
 }
 
-template <typename Rt> int plain_forward(sdns_plan* p, const void* up, void* uh, int nc) {
+// bufA, bufB: nc fields each; the plan's workspace (three fields) unless given.
+template <typename Rt> int plain_forward(sdns_plan* p, const void* up, void* uh, int nc, void* bufA = nullptr,
+                                         void* bufB = nullptr) {
   const int N0 = p->N[0], N1 = p->N[1], Nh = p->Nh, N2 = p->N[2];
   const long plane = (long)N1 * Nh, fs = (long)N0 * plane;
+  if (!bufA) { bufA = p->bufA; bufB = p->bufB; }
   ZArgs<Rt> z{};
-  z.in = up; z.out = p->bufA; z.tw = p->tw[N2 / 2]; z.rtw = p->rtw[N2];
+  z.in = up; z.out = bufA; z.tw = p->tw[N2 / 2]; z.rtw = p->rtw[N2];
   z.L = N0 * N1; z.nk = Nh; z.in_line = N2 / 2; z.in_field = (long)N0 * N1 * (N2 / 2);
   z.out_line = Nh; z.out_field = fs; z.scale = Rt(1);
   if (launch_z<Rt>(N2 / 2, p->var[5], -1, nc, z, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "z length %d", N2);
   StridedArgs<Rt> a{};
-  a.in = p->bufA; a.out = p->bufB; a.tw = p->tw[N1];
+  a.in = bufA; a.out = bufB; a.tw = p->tw[N1];
   a.Q = N0 * Nh; a.cdiv = Nh; a.cvalid = Nh; a.in_hi = plane; a.out_hi = plane; a.in_row = Nh; a.out_row = Nh;
   a.in_field = fs; a.out_field = fs;
   a.rin = rmap(N1 / 2, N1 / 2 - 1, N1); a.rout = a.rin; a.scale = Rt(1);
   if (launch_strided<Rt>(N1, p->var[5], -1, nc, a, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "y length %d", N1);
-  a.in = p->bufB; a.out = uh; a.tw = p->tw[N0];
+  a.in = bufB; a.out = uh; a.tw = p->tw[N0];
   a.Q = (int)plane; a.cdiv = (int)plane; a.cvalid = (int)plane; a.in_hi = 0; a.out_hi = 0; a.in_row = plane;
   a.out_row = plane;
   a.rin = rmap(N0 / 2, N0 / 2 - 1, N0); a.rout = a.rin;
@@ -746,13 +750,15 @@ template <typename Rt> int form_state(sdns_plan* p, void* out, const P1Args<Rt>&
   return 0;
 }
 
-// Network forward on the closure's packed input x0.  Training (tau = null):
-// y = output, FP32 [P][8], 6 real, and the pre-activations z1, z2 that the
-// backward pass reads; inference: tau = out_scale * output, planar.
-int closure_net_forward(sdns_closure* c, hipStream_t st, float* tau, float out_scale) {
+// Network forward.  Training (tau = null): from the packed input x0, y = output,
+// FP32 [P][8], 6 real, and the pre-activations z1, z2 that the backward pass
+// reads.  Inference: from the planar velocity u, scaled as it is read, to
+// tau = out_scale * output, planar.
+int closure_net_forward(sdns_closure* c, hipStream_t st, const float* u, float in_scale, float* tau, float out_scale) {
   ConvArgs a{};
   a.n0 = c->n[0]; a.n1 = c->n[1]; a.n2 = c->n[2];
   a.x = c->x0; a.w = c->w.w1f; a.bias = c->w.b1; a.z = tau ? nullptr : c->z1; a.a = c->a1;
+  if (tau) { a.x = nullptr; a.u = u; a.scale = in_scale; }
   if (launch_conv(8, 32, CONV_EPI_SILU, a, st)) return fail(SDNS_ERR_UNSUPPORTED, "closure grid");
   a.x = c->a1; a.w = c->w.w2f; a.bias = c->w.b2; a.z = tau ? nullptr : c->z2; a.a = c->a2;
   if (launch_conv(32, 32, CONV_EPI_SILU, a, st)) return fail(SDNS_ERR_HIP, "closure layer 2");
@@ -767,11 +773,9 @@ int closure_net_forward(sdns_closure* c, hipStream_t st, float* tau, float out_s
 int closure_source(sdns_closure* c, sdns_plan* p, const void* u, float in_scale, float out_scale) {
   int rc;
   if ((rc = plain_backward<float>(p, u, c->phys, 3))) return rc;
-  launch_pack_input(c->phys, in_scale, c->x0, c->P, p->stream);
-  if ((rc = closure_net_forward(c, p->stream, c->tauphys, out_scale))) return rc;
-  const size_t fbytes = (size_t)p->N[0] * p->N[1] * p->Nh * p->esz;
-  if ((rc = plain_forward<float>(p, c->tauphys, c->tauhat, 3))) return rc;
-  if ((rc = plain_forward<float>(p, c->tauphys + 3 * c->P, c->tauhat + 3 * fbytes, 3))) return rc;
+  if ((rc = closure_net_forward(c, p->stream, c->phys, in_scale, c->tauphys, out_scale))) return rc;
+  // all six components in one launch per pass: at these sizes a launch costs its latency
+  if ((rc = plain_forward<float>(p, c->tauphys, c->tauhat, 6, c->fftA, c->fftB))) return rc;
   EwArgs<float> e = ew_args<float>(p);
   e.a = c->tauhat; e.out = c->src;
   if (launch_elementwise<float>(EW_SGS_FORCE, e, p->stream)) return fail(SDNS_ERR_HIP, "sgs force");
@@ -1853,6 +1857,7 @@ int sdns_closure_create(sdns_closure** out, const int32_t N[3], void* hip_stream
   c->gz2 = (__bf16*)(m + o_gz2); c->gz1 = (__bf16*)(m + o_gz1);
   c->y = (float*)(m + o_y); c->wpart = (float*)(m + o_wp); c->gsum = (float*)(m + o_gs); c->phys = (float*)(m + o_ph);
   c->tauphys = (float*)(m + o_tp); c->tauhat = m + o_th; c->src = m + o_src;
+  c->fftA = m + o_z1; c->fftB = m + o_z2;  // only training keeps z1, z2 (64 bytes a point; six fields take at most 26)
   c->stage = c->tauhat;  // read by the transform before tau's is written
   c->lpart = (double*)(m + o_lp);
   c->w.w1f = (__bf16*)(m + o_w1); c->w.w2f = (__bf16*)(m + o_w2); c->w.w3f = (__bf16*)(m + o_w3);
@@ -1878,8 +1883,7 @@ int sdns_closure_set_params(sdns_closure* c, const float* params) {
 int sdns_closure_forward(sdns_closure* c, const float* u_phys, float in_scale, float out_scale, float* tau_phys) {
   if (!c || !u_phys || !tau_phys) return fail(SDNS_ERR_INVALID, "bad argument");
   if (!c->have_params) return fail(SDNS_ERR_INVALID, "closure parameters not set");
-  launch_pack_input(u_phys, in_scale, c->x0, c->P, c->stream);
-  const int rc = closure_net_forward(c, c->stream, tau_phys, out_scale);
+  const int rc = closure_net_forward(c, c->stream, u_phys, in_scale, tau_phys, out_scale);
   return rc ? rc : check_launch();
 }
 
@@ -1891,7 +1895,7 @@ int sdns_closure_train_step(sdns_closure* c, const float* u_phys, const float* t
   const long P = c->P;
   const int n0 = c->n[0], n1 = c->n[1], n2 = c->n[2];
   launch_pack_input(u_phys, in_scale, c->x0, P, st);
-  const int rc = closure_net_forward(c, st, nullptr, 1.f);
+  const int rc = closure_net_forward(c, st, nullptr, 1.f, nullptr, 1.f);
   if (rc) return rc;
   launch_loss(c->y, tau_phys, 1.0f / out_scale, c->gyb, P, c->lpart, c->gsum, st);
   // layer 3

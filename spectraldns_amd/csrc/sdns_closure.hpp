@@ -38,7 +38,8 @@ struct ClosureWeights {
 enum { CONV_EPI_SILU = 0, CONV_EPI_LINEAR = 1, CONV_EPI_DSILU = 2, CONV_EPI_PLANAR = 3 };
 
 struct ConvArgs {
-  const __bf16* x;      // input [P][cin]
+  const __bf16* x;      // input [P][cin], or null (8 channels): u
+  const float* u;       // planar FP32 input [3][P], times scale (8 channels)
   const __bf16* w;      // [27][cout][cin]
   const float* bias;    // [cout] or null
   __bf16* z;            // SILU: pre-activation out [P][cout] (null: not stored)
@@ -47,7 +48,7 @@ struct ConvArgs {
   const __bf16* zprev;  // DSILU: stored pre-activation [P][cout] whose SiLU' multiplies the result
   int n0, n1, n2;
   int ystride, ncout;
-  float scale;
+  float scale;          // of u (8 channels) or of the PLANAR output
 };
 
 // cin in {8, 32}, cout in {16, 32}; N2 % 32 == 0, N0 and N1 at least 4.  Returns
