@@ -664,6 +664,7 @@ template <typename Rt> int mhd_stage(sdns_plan* p, const void* u, const void* b,
   char *A = ws, *B = ws + L.a;
   P1Args<Rt> a1 = p1_args<Rt>(p, u);
   a1.w = b; a1.w1 = A;
+  a1.u_tiled = a1.w_tiled = mode == P5_RK12 || mode == P5_RK3;  // stage states
   tstart(p, 0);
   if (launch_p1<Rt>(M0, p->var[0], a1, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", M0);
   tstop(p);

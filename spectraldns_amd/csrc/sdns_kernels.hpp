@@ -82,13 +82,22 @@ template <typename Rt> constexpr int esz_of() { return (int)sizeof(Rt); }
 constexpr int stage_k(int n, int P) { return (n + 1 + P - 1) / P; }
 
 // Column tile of this block.  Blocks are dispatched round-robin over the 8
-// XCDs; consecutive tiles go to blocks of the same XCD so that neighbouring
-// tiles, which share 128-byte lines of rows whose length is not a multiple
-// of 16 elements, meet in the same L2.  Launch 8*ceil(ntiles/8) blocks;
-// returns -1 for the padding blocks.
-__device__ __forceinline__ int xcd_tile(int ntiles) {
-  const int per = (ntiles + 7) >> 3;
-  const int t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+// XCDs; G consecutive tiles go to blocks of the same XCD, so that neighbouring
+// tiles, which share 128-byte lines of rows whose length is not a multiple of
+// 16 elements, meet in the same L2, and the next G to the next XCD.  The tiles
+// in flight then cover one range of every row, which spreads over all memory
+// channels, and columns without kept modes, which cost less, fall on all XCDs
+// alike.  (With one contiguous eighth of the tiles per XCD: 256^3 FP32 P2
+// 288 against 279 us, x-forward 287 against 257 us, 512^3 y-forward 606 against
+// 592 us, 256^3 FP64 y-forward 275 against 265 us, x-forward 444 against 427 us;
+// with G = 4 the y-forward takes 147 us instead of 131, with 32, which keeps the
+// tiles of a few whole planes together, MHD's takes 220 us against 237 with 16:
+// the strided passes use 32.)  Launch
+// 8*ceil(ntiles/8) blocks; returns -1 for the padding blocks.
+template <int G = 16> __device__ __forceinline__ int xcd_tile(int ntiles) {
+  const int per = (ntiles + 7) >> 3, full = per / G * G;
+  const int x = (int)(blockIdx.x & 7), s = (int)(blockIdx.x >> 3);
+  const int t = s < full ? (s / G * 8 + x) * G + s % G : 8 * full + x * (per - full) + (s - full);
   return t < ntiles ? t : -1;
 }
 inline int xcd_grid(int ntiles) { return ((ntiles + 7) / 8) * 8; }
@@ -104,7 +113,9 @@ __device__ __forceinline__ void table_to_lds(C* dst, const C* __restrict__ src, 
 // y = 1 -> v (fields 1 and 4 = X(kx v)), y = 2 -> u (field 0).  With a given
 // vorticity (a.w) there are six blocks rows y = 0..5, each the plain
 // x-inverse of one field: u, v, w from a.u, then wx, wy, wz from a.w.
-// INC: the state is u + ds d, formed on reading (the RK stages of KEEP_RHS).
+// INC: the state is u + ds d, formed on reading (the RK stages of KEEP_RHS; a
+// template, since a second loop behind a branch cost every stage its schedule).
+// Bound by its rows and stores: 3.1 TB/s at 256^3 3/2 rule FP32 (142 us).
 template <typename Rt, int M, int E, int T, bool INC>
 __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, cx<Rt>* lds, const cx<Rt>* tw) {
   using C = cx<Rt>;
@@ -886,7 +897,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (occ_for(E, esz
   constexpr int T = SCfg<Rt, M, E>::T / D;
   __shared__ C lds[M * T];
   __shared__ C tw[M];
-  const int tile = xcd_tile((a.Q + T - 1) / T);
+  const int tile = xcd_tile<32>((a.Q + T - 1) / T);
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
   strided_body<Rt, M, E, DIR, T>(a, tile, blockIdx.y, lds, tw);
@@ -1183,11 +1194,19 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
 // The host checks that the three components of a state array and of W4 span
 // at most BUF_OOB bytes (p5b_fits); larger boxes run p5_body.  The per-mode
 // arithmetic is p5_body's.
+// Bound by the strided rows (128 bytes each, 3..5 streams) at 2.4..3.6 TB/s, its
+// blocks alternating between loading W4, the transforms and the update.  Mean of
+// the four stages, p5_body -> now: 256^3 FP32 2/3 rule 245 -> 199 us (217 with
+// the skip and one eighth of the tiles per XCD), 3/2 rule 283 -> 258 us, FP64 3/2
+// rule 548 -> 427 us, 512^3 FP32 compensated 2.8 -> 1.5 ms.
+// EARLY: the first rows are loaded beside W4, before the transforms (divided
+// tiles: a grid of a few blocks per CU pays one latency less; in full grids the
+// 24..50 registers cost spills or occupancy).
 // VV: the velocity-vorticity right-hand side instead (solvers/VV.py:104-146): the
 // state is the vorticity, the convection term is i K x F(u x w) and there is no
 // pressure.
 template <typename Rt, int M, int E, int MODE, bool PAD, bool COMP, int T, int KEEP = rk_keep<Rt>(PAD, COMP),
-          bool VV = false>
+          bool VV = false, bool EARLY_ = false>
 __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* lds, const cx<Rt>* tw) {
   using C = cx<Rt>;
   static_assert(!PAD || (M % 3 == 0 && E % 3 == 0), "3/2-rule rows");
@@ -1210,40 +1229,26 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
   const auto rw = buf_rsrc(a.w4, 3L * wfield * CS);
   const int wo = colconv ? (t * wrow + kyc * a.nkzop + kz) * CS : BUF_OOB;
   C X0[E], X1[E], X2[E];
+  // a tile without kept modes (half of them under the 2/3 rule) skips the
+  // transforms; every wave holds all T columns, so all decide alike.  (In a grid
+  // of few blocks the kept tiles alone set the time, so no test there.)
+  static_assert(T <= 64 && TH % 64 == 0, "a wave holds every column");
+  const bool transform = EARLY_ || __any(colconv);
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    X0[e] = buf_load_so<C>(rw, wo, P * e * wrow * CS);
-    X1[e] = buf_load_so<C>(rw, wo, (wfield + P * e * wrow) * CS);
-    X2[e] = buf_load_so<C>(rw, wo, (2 * wfield + P * e * wrow) * CS);
+  for (int e = 0; e < E; ++e) X0[e] = X1[e] = X2[e] = czero<C>();
+  if (transform) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      X0[e] = buf_load_so<C>(rw, wo, P * e * wrow * CS);
+      X1[e] = buf_load_so<C>(rw, wo, (wfield + P * e * wrow) * CS);
+      X2[e] = buf_load_so<C>(rw, wo, (2 * wfield + P * e * wrow) * CS);
+    }
   }
-  __syncthreads();
-  C* line = lds + c;
-  F::run(X0, t, line, T, tw);
-  F::run(X1, t, line, T, tw);
-  F::run(X2, t, line, T, tw);
-
   const int plane = a.N1 * a.Nh, fs = a.N0 * plane;
   const long span = 3L * fs * CS;
   const int so = (t * plane + q) * CS;  // row t of the column
   // rows whose convection term is kept (every row with PAD)
   auto kept = [&](int ix) { return PAD || ix <= a.x.pos || ix >= a.N0 - a.x.neg; };
-  if constexpr (MODE == P5_RHS) {
-    if (a.conv_only) {
-      const auto ro = buf_rsrc(a.rhs, span);
-      if (valid) {
-#pragma unroll
-        for (int j = 0; j < NK; ++j) {
-          const int e = (!PAD || j < E3) ? j : j + E3;
-          const int eo = P * j * plane;
-          const Rt sc = kept(t + P * j) ? a.scale : Rt(0);
-          buf_store_so_nt<C>(cscale(X0[e], sc), ro, so, eo * CS);
-          buf_store_so_nt<C>(cscale(X1[e], sc), ro, so, (fs + eo) * CS);
-          buf_store_so_nt<C>(cscale(X2[e], sc), ro, so, (2 * fs + eo) * CS);
-        }
-      }
-      return;
-    }
-  }
   const Rt K1 = a.ky[iy], K2c = a.kz[kz];
   const Rt Kyz[2] = {K1, K2c};
   const bool colok = colconv && !(a.mask_nyquist && (iy == a.N1 / 2 || kz == a.N2 / 2));
@@ -1266,27 +1271,53 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
   const auto rph = buf_rsrc(a.phat, a.phat ? (long)fs * CS : 0L);
   constexpr bool OUT_S = MODE == P5_RK0 || MODE == P5_RK12;
   const auto ro = buf_rsrc(MODE == P5_RHS ? a.rhs : (MODE == P5_RK3 ? a.u : a.out), OUT_S ? sspan : span);
-  if (valid) {
-    C cur[G][NL + 1][3], nxt[G][NL + 1][3];  // state arrays, then the source
-    Rt kcur[G], knxt[G];
-    auto load = [&](C(&d)[G][NL + 1][3], Rt(&kd)[G], int j0) {
+  C cur[G][NL + 1][3], nxt[G][NL + 1][3];  // state arrays, then the source
+  Rt kcur[G], knxt[G];
+  auto load = [&](C(&d)[G][NL + 1][3], Rt(&kd)[G], int j0) {
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int eo = P * (j0 + g) * plane;
-        kd[g] = a.kx[t + P * (j0 + g)];
+    for (int g = 0; g < G; ++g) {
+      const int eo = P * (j0 + g) * plane;
+      kd[g] = a.kx[t + P * (j0 + g)];
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          const int o = (i * fs + eo) * CS, os = (i * sfs + P * (j0 + g) * srow) * CS;
-          d[g][0][i] = buf_load_so<C>(ru, FIRST_S ? sso : so, FIRST_S ? os : o);
-          if constexpr (NL > 1) d[g][1][i] = buf_load_so<C>(rs, sso, os);
-          if constexpr (NL > 2) d[g][2][i] = buf_load_so<C>(rb1, sso, os);
-          if constexpr (NL > 3) d[g][3][i] = buf_load_so<C>(rb2, sso, os);
-          if constexpr (NL > 4) d[g][4][i] = buf_load_so<C>(rlo, so, o);
-          d[g][NL][i] = buf_load_so<C>(rsrc, so, o);
+      for (int i = 0; i < 3; ++i) {
+        const int o = (i * fs + eo) * CS, os = (i * sfs + P * (j0 + g) * srow) * CS;
+        d[g][0][i] = buf_load_so<C>(ru, FIRST_S ? sso : so, FIRST_S ? os : o);
+        if constexpr (NL > 1) d[g][1][i] = buf_load_so<C>(rs, sso, os);
+        if constexpr (NL > 2) d[g][2][i] = buf_load_so<C>(rb1, sso, os);
+        if constexpr (NL > 3) d[g][3][i] = buf_load_so<C>(rb2, sso, os);
+        if constexpr (NL > 4) d[g][4][i] = buf_load_so<C>(rlo, so, o);
+        d[g][NL][i] = buf_load_so<C>(rsrc, so, o);
+      }
+    }
+  };
+  constexpr bool EARLY = EARLY_ && MODE != P5_RHS;
+  if (EARLY) load(cur, kcur, 0);
+  if (transform) {
+    __syncthreads();
+    C* line = lds + c;
+    F::run(X0, t, line, T, tw);
+    F::run(X1, t, line, T, tw);
+    F::run(X2, t, line, T, tw);
+  }
+  if constexpr (MODE == P5_RHS) {
+    if (a.conv_only) {
+      const auto ro = buf_rsrc(a.rhs, span);
+      if (valid) {
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+          const int e = (!PAD || j < E3) ? j : j + E3;
+          const int eo = P * j * plane;
+          const Rt sc = kept(t + P * j) ? a.scale : Rt(0);
+          buf_store_so_nt<C>(cscale(X0[e], sc), ro, so, eo * CS);
+          buf_store_so_nt<C>(cscale(X1[e], sc), ro, so, (fs + eo) * CS);
+          buf_store_so_nt<C>(cscale(X2[e], sc), ro, so, (2 * fs + eo) * CS);
         }
       }
-    };
-    load(cur, kcur, 0);
+      return;
+    }
+  }
+  if (valid) {
+    if (!EARLY) load(cur, kcur, 0);
 #pragma unroll
     for (int j0 = 0; j0 < NK; j0 += G) {
       if (j0 + G < NK) load(nxt, knxt, j0 + G);
@@ -1399,10 +1430,11 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, 
   const int tile = xcd_tile((a.Q + T - 1) / T);
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
-  p5b_body<Rt, M, E, MODE, PAD, COMP, T>(a, tile, lds, tw);
+  p5b_body<Rt, M, E, MODE, PAD, COMP, T, rk_keep<Rt>(PAD, COMP), false, (D > 1)>(a, tile, lds, tw);
 }
 
-// The VV stages (p5b_body).
+// The VV stages (p5b_body; 128^3 FP64 2/3 rule: elementwise tail, stage sums and
+// velocity in launches of their own took 400 of 1041 us a step, now 650 us).
 template <typename Rt, int M, int E, int MODE, bool PAD, int D = 1>
 __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, E, PAD>())) k_p5vv(P5Args<Rt> a) {
   using C = cx<Rt>;
@@ -1412,7 +1444,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, 
   const int tile = xcd_tile((a.Q + T - 1) / T);
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
-  p5b_body<Rt, M, E, MODE, PAD, false, T, KEEP_STATES, true>(a, tile, lds, tw);
+  p5b_body<Rt, M, E, MODE, PAD, false, T, KEEP_STATES, true, (D > 1)>(a, tile, lds, tw);
 }
 
 // ------------------------------------------------------------------ MHD
@@ -1426,7 +1458,8 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (p5_occ<Rt, M, 
 // z pass: the six real lines of u and b stay in registers, and each of the
 // nine products is formed, transformed and written from there.  Physical space
 // never touches HBM: as separate launches the same step wrote and read 6 + 9
-// physical fields.
+// physical fields (with the fused x pass below, 256^3 FP32 2/3 rule: 9.26 ->
+// 4.42 ms an RK4 step; this pass 226 us, 4.5 TB/s).
 __device__ constexpr int mhd_i(int f) { return f < 3 ? 0 : (f < 5 ? 1 : (f == 5 ? 2 : (f < 8 ? 0 : 1))); }
 __device__ constexpr int mhd_j(int f) { return f < 3 ? f : (f < 5 ? f - 2 : (f == 5 ? 2 : (f < 8 ? f - 5 : 2))); }
 template <typename Rt, int n, int E>
@@ -1486,9 +1519,15 @@ __global__ void __launch_bounds__((ZCfg<Rt, n, E>::THREADS), (occ_for(7 * E + st
 // done, so that three lines of sums, one line in work and the next one's loads
 // are live; then mask, pressure (U) and diffusion (MHD.py:135-176) and the RK4
 // stage as in p5b_body with KEEP_STATES.  Buffer descriptors span three fields
-// or components each.
+// or components each.  Bound like p5b_body; 256^3 FP32, mean of the stages: 553
+// us with linear stage arrays, every tile transformed and an eighth of the tiles
+// per XCD, 500 us now.  Two 8-wave blocks per CU need 128 registers (mhd_x_occ).
+template <typename Rt, int M, int E> constexpr int mhd_x_occ() {
+  const int o = occ_for(5 * E, esz_of<Rt>());
+  return sizeof(Rt) == 4 && E <= 8 ? 4 : o;
+}
 template <typename Rt, int M, int E, int MODE, bool PAD>
-__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz_of<Rt>()))) k_mhd_x(MhdXArgs<Rt> a) {
+__global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (mhd_x_occ<Rt, M, E>())) k_mhd_x(MhdXArgs<Rt> a) {
   using C = cx<Rt>;
   static_assert(!PAD || (M % 3 == 0 && E % 3 == 0), "3/2-rule rows");
   constexpr int T = SCfg<Rt, M, E>::T;
@@ -1497,9 +1536,11 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz
   using F = LineFFT<Rt, M, E, -1>;
   __shared__ C lds[M * T];
   __shared__ C tw[M];
+  __shared__ Rt kx[M];  // (held in registers over the six transforms they spill)
   const int tile = xcd_tile((a.Q + T - 1) / T);
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
+  table_to_lds(kx, a.kx, a.N0);
   const int c = threadIdx.x % T, t = threadIdx.x / T;
   const int q = tile * T + c;
   const bool valid = q < a.Q;
@@ -1519,9 +1560,6 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz
     for (int e = 0; e < E; ++e) d[e] = buf_load_so<C>(rw, wo, ((f % 3) * wfield + P * e * wrow) * CS);
   };
   const Rt K1 = a.ky[iy], K2c = a.kz[kz];
-  Rt k0[NK];
-#pragma unroll
-  for (int j = 0; j < NK; ++j) k0[j] = a.kx[t + P * j];
   C S[3][NK];
 #pragma unroll
   for (int f = 0; f < 3; ++f)
@@ -1529,7 +1567,6 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz
     for (int r = 0; r < NK; ++r) S[f][r] = czero<C>();
   C X[E], Y[E];
   load_field(X, f0);
-  __syncthreads();
   C* line = lds + c;
   // S[i] += +-K_j v, S[j] += +-K_i v of the field f
   auto add = [&](auto fc) {
@@ -1540,15 +1577,19 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz
     for (int r = 0; r < NK; ++r) {
       const int e = (!PAD || r < E3) ? r : r + E3;
       const C v = cscale(X[e], a.scale);
-      const Rt Kv[3] = {k0[r], K1, K2c};
+      const Rt Kv[3] = {kx[t + P * r], K1, K2c};
       S[i][r] = caxpy(S[i][r], Kv[j], v);
       if constexpr (i != j) S[j][r] = caxpy(S[j][r], f < 6 ? Kv[i] : -Kv[i], v);
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) X[e] = Y[e];
   };
-  if (h == 0) sfor<6>([&](auto fc) { add(fc); });
-  else sfor<3>([&](auto fc) { add(std::integral_constant<int, decltype(fc)::value + 6>{}); });
+  __syncthreads();
+  static_assert(T <= 64 && T * P % 64 == 0, "a wave holds every column");
+  if (__any(colconv)) {  // as in p5b_body
+    if (h == 0) sfor<6>([&](auto fc) { add(fc); });
+    else sfor<3>([&](auto fc) { add(std::integral_constant<int, decltype(fc)::value + 6>{}); });
+  }
   if (!valid) return;
   const int plane = a.N1 * a.Nh, fs = a.N0 * plane;
   const long span = 3L * fs * CS;
@@ -1556,23 +1597,29 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz
   const bool colok = colconv && !(a.mask_nyquist && (iy == a.N1 / 2 || kz == a.N2 / 2));
   const int nyq_ix = a.mask_nyquist ? a.N0 / 2 : -1;
   const auto rph = buf_rsrc(a.phat, a.phat && h == 0 ? (long)fs * CS : 0L);
+  // stage arrays (tile-major): row and component strides, span, this lane's offset
+  constexpr bool OUT_S = MODE == P5_RK0 || MODE == P5_RK12;
+  constexpr int TW = tile_w<Rt>();
+  const int sfs = a.N0 * tiled_cols<Rt>(a.Q);
+  const long sspan = 3L * sfs * CS;
+  const int sso = (q / TW * TW * a.N0 + q % TW + t * TW) * CS;
   const auto ru = buf_rsrc(a.u[h], span);
-  const auto rs = buf_rsrc(a.s[h], span);
-  const auto r1 = buf_rsrc(a.b1[h], span);
-  const auto r2 = buf_rsrc(a.b2[h], span);
-  const auto ro = buf_rsrc(MODE == P5_RK3 ? a.u[h] : a.out[h], span);
+  const auto rs = buf_rsrc(a.s[h], sspan);
+  const auto r1 = buf_rsrc(a.b1[h], sspan);
+  const auto r2 = buf_rsrc(a.b2[h], sspan);
+  const auto ro = buf_rsrc(MODE == P5_RK3 ? a.u[h] : a.out[h], OUT_S ? sspan : span);
   const Rt visc = a.visc[h], press = h == 0 ? Rt(1) : Rt(0);
   constexpr int NL = p5_arrays(MODE, false, KEEP_STATES);
   C cur[NL][3], nxt[NL][3];
   auto load = [&](C(&d)[NL][3], int r) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      const int o = (i * fs + P * r * plane) * CS;
-      d[0][i] = buf_load_so<C>(ru, so, o);
-      if constexpr (NL > 1) d[1][i] = buf_load_so<C>(rs, so, o);
+      const int o = (i * sfs + P * r * TW) * CS;
+      d[0][i] = buf_load_so<C>(ru, so, (i * fs + P * r * plane) * CS);
+      if constexpr (NL > 1) d[1][i] = buf_load_so<C>(rs, sso, o);
       if constexpr (NL > 2) {
-        d[2][i] = buf_load_so<C>(r1, so, o);
-        d[3][i] = buf_load_so<C>(r2, so, o);
+        d[2][i] = buf_load_so<C>(r1, sso, o);
+        d[3][i] = buf_load_so<C>(r2, sso, o);
       }
     }
   };
@@ -1583,7 +1630,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz
     const int ix = t + P * r;
     const int eo = P * r * plane;
     const bool conv = colok & (ix != nyq_ix) & (PAD || ix <= a.x.pos || ix >= a.N0 - a.x.neg);
-    const Rt Kv[3] = {k0[r], K1, K2c};
+    const Rt Kv[3] = {kx[t + P * r], K1, K2c};
     Rt k2 = Kv[0] * Kv[0];
     k2 += K1 * K1;
     k2 += K2c * K2c;
@@ -1607,7 +1654,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (occ_for(5 * E, esz
       x = mk<C>(x.x - z * st.x, x.y - z * st.y);
       if constexpr (MODE == P5_RK0 || MODE == P5_RK12) x = caxpy(u, a.bdt, x);
       if constexpr (MODE == P5_RK3) x = rk_add_states(u, cur[NL > 2 ? 2 : 0][i], cur[NL > 2 ? 3 : 0][i], st, a.adt, x);
-      buf_store_so_nt<C>(x, ro, so, (i * fs + eo) * CS);
+      buf_store_so_nt<C>(x, ro, OUT_S ? sso : so, (OUT_S ? i * sfs + P * r * TW : i * fs + eo) * CS);
     }
     if (r + 1 < NK) {
 #pragma unroll

@@ -176,7 +176,8 @@ template <typename Rt> struct MhdZArgs {  // z C2R x6, nine products, z R2C x9
 template <typename Rt> struct MhdXArgs {  // x-forward of the products, mask, pressure, diffusion, RK4 stage
   const void* w4;     // [9][M0][nkyo][nkzo]
   // arrays of three components, [0] of U and [1] of B; roles as in P5Args with
-  // KEEP_STATES (P5_RHS: u the input state, out the right-hand side)
+  // KEEP_STATES (P5_RHS: u the input state, out the right-hand side); s, out of
+  // stages 0..2, b1 and b2 are stage arrays, tile-major
   void* u[2];
   const void* s[2];
   void* out[2];
