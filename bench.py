@@ -36,9 +36,12 @@ def pass_bytes(N, dealias, esz):
     (3/2 rule) fields that went through the x (y) inverse are M0/N0 (M1/N1)
     times larger.  P1 reads u_hat (3F) and writes 5 fields; P2 reads 5 and
     writes 6; P3 reads 6 and writes 3; P4 reads 3 and writes 3; P5 reads 3 and
-    streams the RK4 state: stage 0 reads u (3F) and writes u0, u2 (6F);
-    stages 1-2 read u1, u0, u2 (9F) and write u0, u2 (6F); stage 3 reads u0,
-    u2 (6F) and writes u (3F)."""
+    streams the RK4 state.  FP64 keeps the stage states: stage 0 reads u and
+    writes the first (6F), stages 1-2 read u and one state and write the next
+    (9F each), stage 3 reads u and the three states and writes u (15F).  FP32
+    with the 2/3 rule keeps the stage right-hand sides: the same in P5, and P1
+    reads one beside u in stages 1-3 (9F per step); with the 3/2 rule it keeps
+    one state and the running sum (9F, 15F, 15F, 9F)."""
     F = N[0] * N[1] * (N[2] // 2 + 1) * esz
     rx = 1.5 if dealias == "3/2-rule" else 1.0
     rxy = rx * rx
@@ -48,7 +51,10 @@ def pass_bytes(N, dealias, esz):
         "z_cross": 6 * F * rxy + 3 * F * rxy,
         "y_forward": 3 * F * rxy + 3 * F * rx,
     }
-    rk = [9 * F, 15 * F, 15 * F, 9 * F]
+    keep_sum = esz == 8 and dealias == "3/2-rule"
+    rk = [9 * F, 15 * F, 15 * F, 9 * F] if keep_sum else [6 * F, 9 * F, 9 * F, 15 * F]
+    if esz == 8 and not keep_sum:
+        p["x_inverse"] += 9 * F / 4.0
     p["x_forward_rk"] = 3 * F * rx + sum(rk) / 4.0
     step = 4 * (p["x_inverse"] + p["y_inverse_curl"] + p["z_cross"] + p["y_forward"]) + 4 * 3 * F * rx + sum(rk)
     return p, step, F
@@ -164,7 +170,7 @@ def forced_main(args):
     plan.timing_enable(False)
     passes = plan.timing_read()
     F = N[0] * N[1] * (N[2] // 2 + 1) * 8
-    b_step = 214 * F  # 2/3 rule with compensated u_hat and u2 (hi, lo)
+    b_step = 202 * F  # 2/3 rule; the last stage also reads and writes the lo part of u_hat
     sps = args.steps / el
     d = diag[: 2 * args.steps].cpu().numpy().reshape(-1, 2)
     out = {
@@ -290,23 +296,19 @@ def closure_timing(steps=20, warmup=3):
 
 # Algorithmic HBM bytes per time step of the solver workloads, in units of
 # F = N0*N1*(N2/2+1)*esz (one complex spectral field; a real physical field is
-# counted as F too), 2/3 rule.  VV RHS: K/K^2 curl-inverse 6F, fused
-# convection passes 40F (P1-P4 34F + convection-only x-forward 6F), the
-# one-launch tail (cross2, mask, add_linear: reads F(u x w) and w_hat, writes
-# rhs) 9F = 55F; RK4 stage by stage: three stage values u0 + c rhs 27F, the
-# accumulator u2 = u0 + c rhs then three u2 (+)= c rhs 36F = 63F.  MHD RHS:
-# six inverse transforms of the kept modes 36F (x, y, z pass: 6F per field,
-# the 2/3-rule truncation inside them), Elsasser products 15F, nine forward
-# transforms 54F, set_Elsasser 15F, pressure/diffusion of U 10F, diffusion
-# of B 9F = 139F; RK4 over six
-# components 126F.  NS integrators: fused RHS 44F (P1-P4 34F; x-forward with
+# counted as F too), 2/3 rule.  VV, fused stages: x-inverse of the curl-inverse
+# velocity and the vorticity 3F + 6F, y 12F, z 9F, y-forward 6F, x-forward 3F =
+# 39F per RHS; RK4 with kept stage states 6F + 9F + 9F + 15F.  MHD, fused
+# stages: x-inverse and y 12F each, z pass of six fields and nine products 15F,
+# y-forward 18F, x-forward 9F = 66F per RHS; RK4 over six components 78F.  NS
+# integrators: fused RHS 44F (P1-P4 34F; x-forward with
 # the projection reads W4 and u_hat, writes rhs and P_hat: 10F);
 # ForwardEuler update 9F; AB2 updates 12F + 6F; BS5 (FSAL: 7 RHS per step
 # after the first) stage sums sum_{i=1..7} 3(i+2)F = 126F, solution sum 30F,
 # error sum 27F, error norm 9F, copy of the new state 6F.
 SOLVER_BYTES_F = {
-    ("VV", "RK4"): 4 * 55 + 63,
-    ("MHD", "RK4"): 4 * 139 + 126,
+    ("VV", "RK4"): 4 * 39 + 39,
+    ("MHD", "RK4"): 4 * 66 + 78,
     ("NS", "ForwardEuler"): 44 + 9,
     ("NS", "AB2"): 44 + 18,
     ("NS", "BS5_fixed"): 7 * 44 + 126 + 30 + 27 + 9 + 6,
