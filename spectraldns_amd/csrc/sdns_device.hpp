@@ -310,7 +310,14 @@ template <typename C> __device__ __forceinline__ C buf_load(__amdgpu_buffer_rsrc
 // With a uniform part of the offset in a scalar register (soff): the lane's
 // voff + soff addresses the element; the descriptor must cover voff + soff.
 // The store is non-temporal (the RK stage values are read once, by the next
-// stage).
+// stage).  A 16-byte store takes the sum in its lane offset: while it reads its
+// data registers, the next instructions may not write them, and the compiler
+// keeps that distance (2 wait states) only for stores without a scalar offset,
+// as if a scalar offset made it unnecessary.  It does not on this chip: with
+// `buffer_store_dwordx4 v[8:11], v38, s[8:11], s33 offen nt` followed by a
+// v_fma_f64 into v[8:9], some stores of the FP64 MHD pass wrote the low word of
+// the new v8 (16 to 1600 elements of a 128 x 64 x 128 right-hand side, other ones
+// in each run).
 template <typename C> __device__ __forceinline__ C buf_load_so(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
   if constexpr (sizeof(C) == 8) {
     return __builtin_bit_cast(C, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
@@ -324,7 +331,7 @@ template <typename C> __device__ __forceinline__ void buf_store_so_nt(C x, __amd
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(buf_u32x2, x), r, voff, soff, 2);
   } else {
     static_assert(sizeof(C) == 16, "complex of float or double");
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(buf_u32x4, x), r, voff, soff, 2);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(buf_u32x4, x), r, voff + soff, 0, 2);
   }
 }
 // Non-temporal variant (cache policy nt) for pass outputs read once by the next pass.
