@@ -163,7 +163,7 @@ def _fused(solver, c):
     """Whether the right-hand side is the module's own (no step of it replaced)
     and the fused passes reach the box."""
     plan = c["T"].plan
-    return (getattr(solver.conv, "mhd_fused", False) and solver.add_pressure_diffusion is add_pressure_diffusion and
+    return (getattr(solver.conv, "mhd_fused", False) and solver.add_pressure_diffusion is _module_pressure and
             solver.divergenceConvection is _module_convection and solver.set_Elsasser is _module_elsasser and
             plan.nyquist_masked == (c["mask"] is not None) and plan.fused_stages)
 
@@ -182,9 +182,11 @@ def ComputeRHS(rhs, ub_hat, solver, **context):
     return rhs
 
 
+# (kept apart: the solver may be this module, whose names a user replaces)
 _module_rhs = ComputeRHS
 _module_convection = divergenceConvection
 _module_elsasser = set_Elsasser
+_module_pressure = add_pressure_diffusion
 
 
 def fused_rk4_step(ub_hat, dt, solver, context):

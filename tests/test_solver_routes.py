@@ -1,0 +1,105 @@
+"""Which route the solvers' right-hand side and RK4 step take, with a plan that
+only records its calls: the fused route is for the module's own steps alone, and
+whatever it cannot serve goes step by step."""
+from functools import wraps
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+FUSED = ("compute_rhs", "rk4_steps", "vv_rhs", "vv_rk4_steps", "mhd_rhs", "mhd_rk4_steps")
+
+
+class _Plan:
+    """Stands for a Plan: notes the name of each method called on it."""
+    nyquist_masked, fused_stages, mhd_fused = True, True, True
+    dealiased_shape, real_dtype, device = (2, 2, 2), torch.float64, "cpu"
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        if name.startswith("__"):
+            raise AttributeError(name)
+
+        def method(*args, **kw):
+            self.calls.append(name)
+            return args[0] if args else None
+        return method
+
+
+def _setup(name):
+    import importlib
+    from spectraldns_amd import config
+    module = importlib.import_module("spectraldns_amd.solvers." + name)
+    plan = _Plan()
+    ncomp = 6 if name == "MHD" else 3
+    u, dU = (torch.zeros((ncomp, 2, 2, 2), dtype=torch.complex128) for _ in range(2))
+    space = SimpleNamespace(plan=plan, backward=lambda a, b: b)
+    c = config.AttributeDict(T=space, VT=space, Tp=space, VTp=space, VMp=space, mask=1, Source=torch.zeros_like(dU[:3]),
+                             P_hat=torch.zeros_like(u[0]), K=space, K2=space, K_over_K2=space, u=u, dU=dU, W_hat=u,
+                             work=_Work(), ub_dealias=None, u_dealias=u, ZZ_hat=torch.zeros((3, 3, 2, 2, 2)),
+                             float=np.float64)
+    solver = SimpleNamespace(**{k: v for k, v in vars(module).items() if not k.startswith("__")})
+    solver.conv = module.getConvection("Divergence" if name == "MHD" else "Vortex")
+    return module, solver, c, plan
+
+
+class _Work(dict):
+    def __missing__(self, key):
+        return torch.zeros_like(key[0])
+
+
+def _routes(plan):
+    fused = [n for n in plan.calls if n in FUSED]
+    plan.calls.clear()
+    return fused
+
+
+@pytest.fixture
+def rk4():
+    from spectraldns_amd import config
+    old = dict(config.params)
+    config.params.update(integrator="RK4", nu=0.1, eta=0.1, dt=0.1, compensated=False, precision="double")
+    yield config.params
+    config.params.clear()
+    config.params.update(old)
+
+
+@pytest.mark.parametrize("name,rhs,step", [("NS", "compute_rhs", "rk4_steps"), ("VV", "vv_rhs", "vv_rk4_steps"),
+                                           ("MHD", "mhd_rhs", "mhd_rk4_steps")])
+def test_own_steps_are_fused(name, rhs, step, rk4):
+    from spectraldns_amd.maths.integrators import getintegrator
+    module, solver, c, plan = _setup(name)
+    solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c)
+    assert _routes(plan) == [rhs]
+    getintegrator(c.dU, c.u, solver, c)()
+    assert _routes(plan) == [step]
+
+
+@pytest.mark.parametrize("name,hook", [("VV", "add_linear"), ("MHD", "add_pressure_diffusion")])
+@pytest.mark.parametrize("as_module", [True, False])
+def test_replaced_hook_is_called(name, hook, as_module, rk4, monkeypatch):
+    """Also where the solver is the module itself, whose name the hook then is."""
+    from spectraldns_amd.maths.integrators import getintegrator
+    module, solver, c, plan = _setup(name)
+    if as_module:
+        monkeypatch.setattr(module, "conv", solver.conv, raising=False)
+        solver = module
+    seen = []
+    monkeypatch.setattr(solver, hook, lambda rhs, *a, **k: seen.append(1) or rhs)
+    solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c)
+    assert seen == [1] and _routes(plan) == []
+    getintegrator(c.dU, c.u, solver, c)()
+    assert len(seen) == 5 and _routes(plan) == []
+
+
+def test_replaced_cross_product_is_called(rk4, monkeypatch):
+    """The VV convection calls the cross2 of its module."""
+    module, solver, c, plan = _setup("VV")
+    seen = []
+    monkeypatch.setattr(module, "cross2", lambda out, *a: seen.append(1) or out)
+    solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c)
+    assert seen == [1] and _routes(plan) == []
