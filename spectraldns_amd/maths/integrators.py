@@ -150,7 +150,7 @@ def getintegrator(rhs, u0, solver, context):
     if params.get("compensated", False) and params.integrator != "RK4":
         raise NotImplementedError("the compensated state is carried by the fused NS RK4 step only "
                                   "(integrator %r)" % params.integrator)
-    if params.integrator == "RK4" and not (getattr(solver.conv, "fused_vortex", False) and
+    if params.integrator == "RK4" and not (getattr(solver.conv, "fused_vortex", None) is solver.conv and
                                            solver.ComputeRHS is getattr(solver, "_ComputeRHS_fused", None)):
         if params.get("compensated", False):
             raise NotImplementedError("the compensated state is carried by the fused NS RK4 step only")

@@ -146,7 +146,7 @@ def getConvection(convection):
         return rhs
 
     Conv.convection = convection
-    Conv.mhd_fused = True
+    Conv.mhd_fused = Conv  # (itself: functools.wraps copies the attribute to a wrapper)
     return Conv
 
 
@@ -163,7 +163,7 @@ def _fused(solver, c):
     """Whether the right-hand side is the module's own (no step of it replaced)
     and the fused passes reach the box."""
     plan = c["T"].plan
-    return (getattr(solver.conv, "mhd_fused", False) and solver.add_pressure_diffusion is _module_pressure and
+    return (getattr(solver.conv, "mhd_fused", None) is solver.conv and solver.add_pressure_diffusion is _module_pressure and
             solver.divergenceConvection is _module_convection and solver.set_Elsasser is _module_elsasser and
             plan.nyquist_masked == (c["mask"] is not None) and plan.fused_stages)
 

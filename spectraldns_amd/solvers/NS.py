@@ -190,7 +190,7 @@ def getConvection(convection):
             return VTp.plan.convection(u_hat, rhs)
 
         Conv.convection = convection
-        Conv.fused_vortex = True
+        Conv.fused_vortex = Conv  # (itself: functools.wraps copies the attribute to a wrapper)
         return Conv
     if convection not in ("Standard", "Divergence", "Skewed"):
         raise NotImplementedError("convection %r" % convection)
@@ -228,7 +228,7 @@ def ComputeRHS(rhs, u_hat, solver, **context):
     c = context
     VT = c["VT"]
     src = c["Source"]
-    if getattr(solver.conv, "fused_vortex", False):
+    if getattr(solver.conv, "fused_vortex", None) is solver.conv:
         return VT.plan.compute_rhs(u_hat, rhs, params.nu, source=src, p_hat=c["P_hat"])
     u_dealias = c.get("u_dealias")
     if u_dealias is None:  # (the context builds it on first access; keyword unpacking skips it)

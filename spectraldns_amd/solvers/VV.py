@@ -114,7 +114,7 @@ def getConvection(convection):
         return rhs
 
     Conv.convection = convection
-    Conv.vv_fused_tail = True
+    Conv.vv_fused_tail = Conv  # (itself: functools.wraps copies the attribute to a wrapper)
     return Conv
 
 
@@ -138,7 +138,7 @@ def _fused(solver, c):
     """Whether the right-hand side is the module's own (Conv, cross2, mask and
     add_linear not replaced) and the fused passes reach the box."""
     plan = c["VT"].plan
-    return (getattr(solver.conv, "vv_fused_tail", False) and solver.add_linear is _module_linear and
+    return (getattr(solver.conv, "vv_fused_tail", None) is solver.conv and solver.add_linear is _module_linear and
             cross2 is _module_cross2 and plan.nyquist_masked == (c["mask"] is not None) and plan.fused_stages)
 
 
@@ -150,7 +150,7 @@ def ComputeRHS(rhs, w_hat, solver, **context):
     src = c["Source"]
     if _fused(solver, c) and rhs.data_ptr() != w_hat.data_ptr():
         return c["VT"].plan.vv_rhs(w_hat, rhs, params.nu, src)
-    if getattr(solver.conv, "vv_fused_tail", False) and solver.add_linear is _module_linear:
+    if getattr(solver.conv, "vv_fused_tail", None) is solver.conv and solver.add_linear is _module_linear:
         # the module's own Conv and add_linear: cross2, mask and add_linear in one launch
         v_hat = _cross_convection(w_hat, c["work"], c["VTp"], c["K_over_K2"])
         return c["VT"].plan.vv_rhs_tail(rhs, v_hat, w_hat, params.nu, src)
