@@ -161,10 +161,11 @@ def add_pressure_diffusion(rhs, ub_hat, nu, eta, K2, K, P_hat, K_over_K2):
 
 def _fused(solver, c):
     """Whether the right-hand side is the module's own (no step of it replaced)
-    and the fused passes reach the box."""
+    and the fused passes reach the box.  conv and add_pressure_diffusion are the
+    solver argument's, the others this module's, as the steps call them."""
     plan = c["T"].plan
     return (getattr(solver.conv, "mhd_fused", None) is solver.conv and solver.add_pressure_diffusion is _module_pressure and
-            solver.divergenceConvection is _module_convection and solver.set_Elsasser is _module_elsasser and
+            divergenceConvection is _module_convection and set_Elsasser is _module_elsasser and
             plan.nyquist_masked == (c["mask"] is not None) and plan.fused_stages)
 
 

@@ -121,3 +121,21 @@ def test_wrapped_convection_is_called(name, rk4):
     assert seen == [1] and _routes(plan) == []
     getintegrator(c.dU, c.u, solver, c)()
     assert len(seen) == 5 and _routes(plan) == []
+
+
+def test_mhd_solver_without_the_module_helpers(rk4):
+    """ComputeRHS needs conv and add_pressure_diffusion of its solver argument, no more."""
+    from spectraldns_amd.solvers import MHD
+    _, full, c, plan = _setup("MHD")
+    solver = SimpleNamespace(conv=full.conv, add_pressure_diffusion=MHD.add_pressure_diffusion)
+    MHD.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c)
+    assert _routes(plan) == ["mhd_rhs"]
+
+
+def test_mhd_replaced_helper_of_the_module(rk4, monkeypatch):
+    """The convection calls the helpers of its own module."""
+    module, solver, c, plan = _setup("MHD")
+    seen = []
+    monkeypatch.setattr(module, "set_Elsasser", lambda c, zz, K: seen.append(1) or c)
+    solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c)
+    assert seen == [1] and _routes(plan) == []
