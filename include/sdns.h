@@ -105,6 +105,10 @@ int sdns_vv_rhs(sdns_plan* plan, const void* w_hat, void* rhs, double nu, const 
 /* nsteps classical RK4 steps (integrators.py:149-159) of w_hat in place, the
  * stage updates in the last pass of each stage. */
 int sdns_vv_rk4_steps(sdns_plan* plan, void* w_hat, const double* dts, int nsteps, double nu, const void* source);
+/* The same; rhs (NULL: none) receives the last stage's right-hand side, as the
+ * stage-by-stage step leaves it, and may not alias w_hat. */
+int sdns_vv_rk4_steps_rhs(sdns_plan* plan, void* w_hat, const double* dts, int nsteps, double nu, const void* source,
+                          void* rhs);
 /* The VV right-hand side after the convection passes, in one launch:
  * rhs = 1j*(K x v_hat) (Conv, VV.py:104-106), Nyquist planes zeroed when the
  * plan masks them (VV.py:143-144), then rhs -= nu*K2*w_hat and rhs += source
@@ -157,6 +161,10 @@ int sdns_mhd_rhs(sdns_plan* plan, const void* ub_hat, void* rhs, double nu, doub
  * last stage's pressure. */
 int sdns_mhd_rk4_steps(sdns_plan* plan, void* ub_hat, const double* dts, int nsteps, double nu, double eta, void* p_hat,
                        void* workspace, size_t bytes);
+/* The same; rhs[6] (NULL: none) receives the last stage's right-hand side and may
+ * not alias ub_hat. */
+int sdns_mhd_rk4_steps_rhs(sdns_plan* plan, void* ub_hat, const double* dts, int nsteps, double nu, double eta,
+                           void* p_hat, void* rhs, void* workspace, size_t bytes);
 /* The Standard, Divergence and Skewed convection forms of the NS solver
  * (spectralDNS/solvers/NS.py:138-199), any dealiasing (physical arrays on the
  * plan's grid, or on the padded grid for the 3/2 rule):

@@ -38,10 +38,14 @@ _SIGS = {
     "sdns_fused_stages": (ctypes.c_int, [_P]),
     "sdns_vv_rhs": (ctypes.c_int, [_P, _P, _P, ctypes.c_double, _P]),
     "sdns_vv_rk4_steps": (ctypes.c_int, [_P, _P, ctypes.POINTER(ctypes.c_double), ctypes.c_int, ctypes.c_double, _P]),
+    "sdns_vv_rk4_steps_rhs": (ctypes.c_int, [_P, _P, ctypes.POINTER(ctypes.c_double), ctypes.c_int, ctypes.c_double, _P,
+                                             _P]),
     "sdns_mhd_workspace_bytes": (ctypes.c_size_t, [_P]),
     "sdns_mhd_rhs": (ctypes.c_int, [_P, _P, _P, ctypes.c_double, ctypes.c_double, _P, _P, ctypes.c_size_t]),
     "sdns_mhd_rk4_steps": (ctypes.c_int, [_P, _P, ctypes.POINTER(ctypes.c_double), ctypes.c_int, ctypes.c_double,
                                           ctypes.c_double, _P, _P, ctypes.c_size_t]),
+    "sdns_mhd_rk4_steps_rhs": (ctypes.c_int, [_P, _P, ctypes.POINTER(ctypes.c_double), ctypes.c_int, ctypes.c_double,
+                                              ctypes.c_double, _P, _P, _P, ctypes.c_size_t]),
     "sdns_dealias_truncate": (ctypes.c_int, [_P, _P, _P]),
     "sdns_backward_dealiased": (ctypes.c_int, [_P, _P, _P, ctypes.c_int]),
     "sdns_forward_dealiased": (ctypes.c_int, [_P, _P, _P, ctypes.c_int]),
@@ -463,15 +467,19 @@ class Plan:
                                      _ptr(source) if source is not None else None))
         return rhs
 
-    def vv_rk4_steps(self, w_hat, dts, nu, source=None):
+    def vv_rk4_steps(self, w_hat, dts, nu, source=None, rhs=None):
+        """rhs receives the last stage's right-hand side."""
         self._spec(w_hat, 3, "w_hat")
+        if rhs is not None:
+            self._spec(rhs, 3, "rhs")
         if source is not None:
             self._spec(source, 3, "Source")
         n = len(dts)
         arr = (ctypes.c_double * max(n, 1))(*[float(d) for d in dts])
         self._sync_stream()
-        _check(self._lib.sdns_vv_rk4_steps(self._h, _ptr(w_hat), arr, n, float(nu),
-                                           _ptr(source) if source is not None else None))
+        _check(self._lib.sdns_vv_rk4_steps_rhs(self._h, _ptr(w_hat), arr, n, float(nu),
+                                               _ptr(source) if source is not None else None,
+                                               _ptr(rhs) if rhs is not None else None))
         return w_hat
 
     def _mhd_workspace(self):
@@ -495,16 +503,20 @@ class Plan:
                                       _ptr(p_hat) if p_hat is not None else None, ws, nbytes))
         return rhs
 
-    def mhd_rk4_steps(self, ub_hat, dts, nu, eta, p_hat=None):
+    def mhd_rk4_steps(self, ub_hat, dts, nu, eta, p_hat=None, rhs=None):
+        """p_hat and rhs receive the last stage's pressure and right-hand side."""
         self._spec(ub_hat, 6, "ub_hat")
+        if rhs is not None:
+            self._spec(rhs, 6, "rhs")
         if p_hat is not None:
             self._spec(p_hat, 1, "P_hat")
         n = len(dts)
         arr = (ctypes.c_double * max(n, 1))(*[float(d) for d in dts])
         self._sync_stream()
         ws, nbytes = self._mhd_workspace()
-        _check(self._lib.sdns_mhd_rk4_steps(self._h, _ptr(ub_hat), arr, n, float(nu), float(eta),
-                                            _ptr(p_hat) if p_hat is not None else None, ws, nbytes))
+        _check(self._lib.sdns_mhd_rk4_steps_rhs(self._h, _ptr(ub_hat), arr, n, float(nu), float(eta),
+                                                _ptr(p_hat) if p_hat is not None else None,
+                                                _ptr(rhs) if rhs is not None else None, ws, nbytes))
         return ub_hat
 
     def lincomb(self, out, xs, cs):

@@ -633,13 +633,15 @@ template <typename Rt> int vv_rhs(sdns_plan* p, const void* w, void* rhs, double
   a.u = const_cast<void*>(w); a.rhs = rhs; a.source = src;
   return vv_stage<Rt>(p, w, 0, P5_RHS, a);
 }
-template <typename Rt> int vv_rk4_steps(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* src) {
+template <typename Rt> int vv_rk4_steps(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* src,
+                                        void* rhs) {
   using RK = RkStage<Rt>;
   for (int s = 0; s < nsteps; ++s)
     for (int rk = 0; rk < 4; ++rk) {
       P5Args<Rt> a = p5_args<Rt>(p, nu);
       RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], w, p->st, 1);
       a.source = src;
+      a.rhs = rk == 3 && s == nsteps - 1 ? rhs : nullptr;
       const int rc = vv_stage<Rt>(p, rk == 0 ? w : p->st[rk - 1], rk > 0, RK::mode(rk), a);
       if (rc) return rc;
     }
@@ -710,7 +712,7 @@ template <typename Rt> int mhd_rhs(sdns_plan* p, const void* ub, void* rhs, doub
   return mhd_stage<Rt>(p, x.u[0], x.u[1], P5_RHS, x, ws);
 }
 template <typename Rt> int mhd_rk4_steps(sdns_plan* p, void* ub, const double* dts, int nsteps, double nu, double eta,
-                                         void* ph, char* ws) {
+                                         void* ph, void* rhs, char* ws) {
   using RK = RkStage<Rt>;
   const size_t half = mhd_half(p);
   const MhdWs L(p);
@@ -728,6 +730,7 @@ template <typename Rt> int mhd_rk4_steps(sdns_plan* p, void* ub, const double* d
         RK::p5(a, KEEP_STATES, rk, (Rt)dts[s], (char*)ub + h * half, st[h], 0);
         x.u[h] = a.u; x.s[h] = a.s; x.out[h] = a.out; x.b1[h] = a.b1; x.b2[h] = a.b2;
         x.adt = a.adt; x.bdt = a.bdt;
+        if (rhs && rk == 3 && s == nsteps - 1) x.rhs[h] = (char*)rhs + h * half;
         in[h] = rk == 0 ? a.u : a.s;
       }
       x.phat = rk == 3 && s == nsteps - 1 ? ph : nullptr;
@@ -1540,13 +1543,18 @@ int sdns_vv_rhs(sdns_plan* p, const void* w, void* rhs, double nu, const void* s
 }
 
 int sdns_vv_rk4_steps(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* source) {
+  return sdns_vv_rk4_steps_rhs(p, w, dts, nsteps, nu, source, nullptr);
+}
+
+int sdns_vv_rk4_steps_rhs(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* source, void* rhs) {
+  if (rhs && rhs == w) return fail(SDNS_ERR_INVALID, "rhs may not alias the state");
   if (!p || !w || (!dts && nsteps > 0) || nsteps < 0) return fail(SDNS_ERR_INVALID, "bad argument");
   if (source && source == w) return fail(SDNS_ERR_INVALID, "the source may not alias the state");
   if (!fused_stages(p)) return fail(SDNS_ERR_UNSUPPORTED, "box beyond the fused stages");
   int rc = ensure_workspace(p);
   if (rc) return rc;
-  rc = p->precision == SDNS_DOUBLE ? vv_rk4_steps<double>(p, w, dts, nsteps, nu, source)
-                                   : vv_rk4_steps<float>(p, w, dts, nsteps, nu, source);
+  rc = p->precision == SDNS_DOUBLE ? vv_rk4_steps<double>(p, w, dts, nsteps, nu, source, rhs)
+                                   : vv_rk4_steps<float>(p, w, dts, nsteps, nu, source, rhs);
   return rc ? rc : check_launch();
 }
 
@@ -1570,11 +1578,17 @@ int sdns_mhd_rhs(sdns_plan* p, const void* ub, void* rhs, double nu, double eta,
 
 int sdns_mhd_rk4_steps(sdns_plan* p, void* ub, const double* dts, int nsteps, double nu, double eta, void* phat,
                        void* ws, size_t bytes) {
+  return sdns_mhd_rk4_steps_rhs(p, ub, dts, nsteps, nu, eta, phat, nullptr, ws, bytes);
+}
+
+int sdns_mhd_rk4_steps_rhs(sdns_plan* p, void* ub, const double* dts, int nsteps, double nu, double eta, void* phat,
+                           void* rhs, void* ws, size_t bytes) {
+  if (rhs && rhs == ub) return fail(SDNS_ERR_INVALID, "rhs may not alias the state");
   if (!p || !ub || (!dts && nsteps > 0) || nsteps < 0) return fail(SDNS_ERR_INVALID, "bad argument");
   int rc = mhd_check(p, ws, bytes);
   if (rc) return rc;
-  rc = p->precision == SDNS_DOUBLE ? mhd_rk4_steps<double>(p, ub, dts, nsteps, nu, eta, phat, (char*)ws)
-                                   : mhd_rk4_steps<float>(p, ub, dts, nsteps, nu, eta, phat, (char*)ws);
+  rc = p->precision == SDNS_DOUBLE ? mhd_rk4_steps<double>(p, ub, dts, nsteps, nu, eta, phat, rhs, (char*)ws)
+                                   : mhd_rk4_steps<float>(p, ub, dts, nsteps, nu, eta, phat, rhs, (char*)ws);
   return rc ? rc : check_launch();
 }
 

@@ -1269,6 +1269,7 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
   const auto rlo = buf_rsrc(a.lo, span);
   const auto rsrc = buf_rsrc(a.source, a.source ? span : 0L);
   const auto rph = buf_rsrc(a.phat, a.phat ? (long)fs * CS : 0L);
+  const auto rk = buf_rsrc(a.rhs, VV && a.rhs ? span : 0L);
   constexpr bool OUT_S = MODE == P5_RK0 || MODE == P5_RK12;
   const auto ro = buf_rsrc(MODE == P5_RHS ? a.rhs : (MODE == P5_RK3 ? a.u : a.out), OUT_S ? sspan : span);
   C cur[G][NL + 1][3], nxt[G][NL + 1][3];  // state arrays, then the source
@@ -1358,6 +1359,7 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
           x = cadd(x, d[NL][i]);  // rhs += Source (NS.py:256-258), every mode
           const int o = (i * fs + eo) * CS, os = (i * sfs + P * j * srow) * CS;
           if constexpr (MODE == P5_RK3) {
+            if constexpr (VV) buf_store_so_nt<C>(x, rk, so, o);
             C l = d[NL > 4 ? 4 : 0][i];
             x = rk_last<KEEP, COMP>(a, u, SUM ? s : d[NL > 2 ? 2 : 0][i], d[NL > 3 ? 3 : 0][i], s, x, l);
             v[2 * i] = x.x;
@@ -1608,6 +1610,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (mhd_x_occ<Rt, M, E
   const auto r1 = buf_rsrc(a.b1[h], sspan);
   const auto r2 = buf_rsrc(a.b2[h], sspan);
   const auto ro = buf_rsrc(MODE == P5_RK3 ? a.u[h] : a.out[h], OUT_S ? sspan : span);
+  const auto rk = buf_rsrc(a.rhs[h], a.rhs[h] ? span : 0L);
   const Rt visc = a.visc[h], press = h == 0 ? Rt(1) : Rt(0);
   constexpr int NL = p5_arrays(MODE, false, KEEP_STATES);
   C cur[NL][3], nxt[NL][3];
@@ -1652,6 +1655,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (mhd_x_occ<Rt, M, E
       const Rt pk = press * Kv[i];
       C x = mk<C>(g[i].x - ph.x * pk, g[i].y - ph.y * pk);
       x = mk<C>(x.x - z * st.x, x.y - z * st.y);
+      if constexpr (MODE == P5_RK3) buf_store_so_nt<C>(x, rk, so, (i * fs + eo) * CS);
       if constexpr (MODE == P5_RK0 || MODE == P5_RK12) x = caxpy(u, a.bdt, x);
       if constexpr (MODE == P5_RK3) x = rk_add_states(u, cur[NL > 2 ? 2 : 0][i], cur[NL > 2 ? 3 : 0][i], st, a.adt, x);
       buf_store_so_nt<C>(x, ro, OUT_S ? sso : so, (OUT_S ? i * sfs + P * r * TW : i * fs + eo) * CS);

@@ -142,7 +142,7 @@ template <typename Rt> struct P5Args {  // x-forward + mask + pressure + diffusi
   void* b1;           // stage 3: B1, B2 or k1, k2; KEEP_SUM: b1 is the accumulator of all stages
   const void* b2;
   void* lo;           // compensated mode: low part of u (caller's u_lo)
-  void* rhs;          // P5_RHS: rhs output
+  void* rhs;          // P5_RHS: rhs output; VV, P5_RK3: this stage's right-hand side (may be null)
   void* phat;         // P5_RHS: pressure output (may be null)
   const void* source; // P5_RHS: added source (may be null)
   double* partials;   // P5_RK3: per-block (energy, enstrophy) sums (may be null)
@@ -184,6 +184,7 @@ template <typename Rt> struct MhdXArgs {  // x-forward of the products, mask, pr
   const void* b1[2];
   const void* b2[2];
   void* phat;         // P5_RHS, P5_RK3: pressure output (may be null)
+  void* rhs[2];       // P5_RK3: this stage's right-hand side (may be null)
   const void* tw;
   const Rt *kx, *ky, *kz;
   int N0, N1, Nh, N2;

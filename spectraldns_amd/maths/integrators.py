@@ -161,7 +161,7 @@ def getintegrator(rhs, u0, solver, context):
         @wraps(RK4_stages)
         def func():
             fused = getattr(solver, "fused_rk4_step", None)
-            if fused is not None and fused(u0, params.dt, solver, context):
+            if fused is not None and fused(u0, rhs, params.dt, solver, context):
                 return u0, params.dt, params.dt
             if not work:
                 work.extend((u0.clone(), u0.clone()))

@@ -190,11 +190,11 @@ _module_elsasser = set_Elsasser
 _module_pressure = add_pressure_diffusion
 
 
-def fused_rk4_step(ub_hat, dt, solver, context):
-    """One RK4 step of ub_hat in place with the stage updates inside the passes
-    (P_hat of the last stage); False where the right-hand side is not the
-    module's own."""
+def fused_rk4_step(ub_hat, rhs, dt, solver, context):
+    """One RK4 step of ub_hat in place with the stage updates inside the passes,
+    the last stage's right-hand side in rhs and its pressure in P_hat; False
+    where the right-hand side is not the module's own."""
     if solver.ComputeRHS is not _module_rhs or not _fused(solver, context):
         return False
-    context.T.plan.mhd_rk4_steps(ub_hat, [dt], params.nu, params.eta, context.P_hat)
+    context.T.plan.mhd_rk4_steps(ub_hat, [dt], params.nu, params.eta, context.P_hat, rhs)
     return True

@@ -167,10 +167,11 @@ _module_linear = add_linear
 _module_cross2 = cross2
 
 
-def fused_rk4_step(w_hat, dt, solver, context):
-    """One RK4 step of w_hat in place with the stage updates inside the passes;
-    False where the right-hand side is not the module's own."""
+def fused_rk4_step(w_hat, rhs, dt, solver, context):
+    """One RK4 step of w_hat in place with the stage updates inside the passes,
+    the last stage's right-hand side in rhs; False where the right-hand side is
+    not the module's own."""
     if solver.ComputeRHS is not _module_rhs or not _fused(solver, context):
         return False
-    context.VT.plan.vv_rk4_steps(w_hat, [dt], params.nu, context.Source)
+    context.VT.plan.vv_rk4_steps(w_hat, [dt], params.nu, context.Source, rhs)
     return True

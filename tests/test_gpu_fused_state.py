@@ -1,0 +1,52 @@
+"""What a fused VV or MHD step leaves behind, and the sizes whose grids fill the
+chip: against the same module running step by step (a replaced hook sends it
+there), whose arithmetic the solver tests hold to the oracle.
+
+Tolerances: a step 1e-14 (FP64) or 1e-6 (FP32) of the state; a right-hand side,
+which two transforms of relative error about 3e-7 each way separate, 1e-13 or
+2e-6, and ten times that where the stage states differ by their own rounding."""
+import numpy as np
+import pytest
+
+from test_gpu_fused_solvers import _context, _rel
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def _start(c, N, seed=3, steep=2.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    phys = torch.randn((c.u.shape[0],) + tuple(N), generator=g, device="cuda", dtype=torch.float64)
+    u = torch.fft.rfftn(phys, dim=(1, 2, 3), norm="forward")
+    k = [torch.fft.fftfreq(n, 1.0 / n, device="cuda") for n in N[:2]] + \
+        [torch.fft.rfftfreq(N[2], 1.0 / N[2], device="cuda")]
+    k2 = k[0][:, None, None] ** 2 + k[1][None, :, None] ** 2 + k[2] ** 2
+    return u * (1 + k2) ** (-0.5 * steep)
+
+
+def _by_steps(solver, name, monkeypatch):
+    hook = "add_linear" if name == "VV" else "add_pressure_diffusion"
+    own = getattr(solver, hook)
+    monkeypatch.setattr(solver, hook, lambda *a, **k: own(*a, **k))
+
+
+@pytest.mark.parametrize("name", ["VV", "MHD"])
+@pytest.mark.parametrize("precision", ["double", "single"])
+def test_step_leaves_the_last_right_hand_side(name, precision, monkeypatch):
+    """context.dU after an RK4 step holds the last stage's right-hand side."""
+    for N, dealias in (((16, 32, 64), "2/3-rule"), ((32, 16, 16), "3/2-rule"), ((256, 16, 32), "2/3-rule")):
+        print("\n[case]", name, precision, N, dealias, flush=True)
+        solver, c, config = _context(name, N, precision, dealias, True)
+        start = _start(c, N).to(c.u.dtype)
+        c.u.copy_(start)
+        step = solver.getintegrator(c.dU, c.u, solver, c)
+        step()
+        got, after = c.dU.clone(), c.u.clone()
+        with monkeypatch.context() as m:
+            _by_steps(solver, name, m)
+            c.u.copy_(start)
+            c.dU.zero_()
+            solver.getintegrator(c.dU, c.u, solver, c)()
+            assert float(c.dU.abs().max()) > 0
+            assert _rel(got, c.dU) <= (1e-12 if precision == "double" else 2e-5)
+            assert _rel(after, c.u) <= (1e-14 if precision == "double" else 1e-6)
