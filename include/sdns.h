@@ -103,7 +103,9 @@ int sdns_fused_stages(const sdns_plan* plan);
  * last.  rhs may not alias w_hat. */
 int sdns_vv_rhs(sdns_plan* plan, const void* w_hat, void* rhs, double nu, const void* source);
 /* nsteps classical RK4 steps (integrators.py:149-159) of w_hat in place, the
- * stage updates in the last pass of each stage. */
+ * stage updates in the last pass of each stage.  The source may be w_hat itself
+ * (its value at the step's start: the last stage reads each mode of it before
+ * it writes that mode), but may not overlap it otherwise. */
 int sdns_vv_rk4_steps(sdns_plan* plan, void* w_hat, const double* dts, int nsteps, double nu, const void* source);
 /* The same; rhs (NULL: none) receives the last stage's right-hand side, as the
  * stage-by-stage step leaves it, and may not alias w_hat. */

@@ -1549,7 +1549,6 @@ int sdns_vv_rk4_steps(sdns_plan* p, void* w, const double* dts, int nsteps, doub
 int sdns_vv_rk4_steps_rhs(sdns_plan* p, void* w, const double* dts, int nsteps, double nu, const void* source, void* rhs) {
   if (rhs && rhs == w) return fail(SDNS_ERR_INVALID, "rhs may not alias the state");
   if (!p || !w || (!dts && nsteps > 0) || nsteps < 0) return fail(SDNS_ERR_INVALID, "bad argument");
-  if (source && source == w) return fail(SDNS_ERR_INVALID, "the source may not alias the state");
   if (!fused_stages(p)) return fail(SDNS_ERR_UNSUPPORTED, "box beyond the fused stages");
   int rc = ensure_workspace(p);
   if (rc) return rc;

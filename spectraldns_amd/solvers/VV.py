@@ -173,5 +173,8 @@ def fused_rk4_step(w_hat, rhs, dt, solver, context):
     not the module's own."""
     if solver.ComputeRHS is not _module_rhs or not _fused(solver, context):
         return False
-    context.VT.plan.vv_rk4_steps(w_hat, [dt], params.nu, context.Source, rhs)
+    src = context.Source
+    if 0 < abs(src.data_ptr() - w_hat.data_ptr()) < w_hat.nbytes:
+        return False  # the last stage would overwrite parts of the Source that it has yet to read
+    context.VT.plan.vv_rk4_steps(w_hat, [dt], params.nu, src, rhs)
     return True

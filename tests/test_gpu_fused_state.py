@@ -50,3 +50,25 @@ def test_step_leaves_the_last_right_hand_side(name, precision, monkeypatch):
             assert float(c.dU.abs().max()) > 0
             assert _rel(got, c.dU) <= (1e-12 if precision == "double" else 2e-5)
             assert _rel(after, c.u) <= (1e-14 if precision == "double" else 1e-6)
+
+
+@pytest.mark.parametrize("precision", ["double", "single"])
+def test_vv_source_is_the_state(precision, monkeypatch):
+    """A Source that is the vorticity itself acts as its value at the step's start."""
+    N = (16, 32, 64)
+    print("\n[case] VV", precision, N, flush=True)
+    solver, c, config = _context("VV", N, precision, "2/3-rule", True)
+    start = _start(c, N).to(c.u.dtype)
+    c.u.copy_(start)
+    c.Source = c.u
+    solver.getintegrator(c.dU, c.u, solver, c)()
+    after = c.u.clone()
+    with monkeypatch.context() as m:
+        _by_steps(solver, "VV", m)
+        c.u.copy_(start)
+        solver.getintegrator(c.dU, c.u, solver, c)()
+    assert _rel(after, c.u) <= (1e-14 if precision == "double" else 1e-6)
+    c.u.copy_(start)
+    c.Source = start.clone()
+    solver.getintegrator(c.dU, c.u, solver, c)()
+    assert torch.equal(after, c.u)

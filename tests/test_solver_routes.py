@@ -139,3 +139,17 @@ def test_mhd_replaced_helper_of_the_module(rk4, monkeypatch):
     monkeypatch.setattr(module, "set_Elsasser", lambda c, zz, K: seen.append(1) or c)
     solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c)
     assert seen == [1] and _routes(plan) == []
+
+
+def test_vv_source_that_overlaps_the_state(rk4):
+    """A Source shifted into the state is read after the state's update by no
+    stage-by-stage step; the fused last stage writes the state while it reads the
+    Source, so only an identical or a separate Source may take it."""
+    from spectraldns_amd.maths.integrators import getintegrator
+    module, solver, c, plan = _setup("VV")
+    both = torch.zeros((4,) + tuple(c.u.shape[1:]), dtype=c.u.dtype)
+    for source, fused in ((both[:3], True), (both[1:], False), (torch.zeros_like(c.u), True)):
+        c.u = c.W_hat = both[:3]
+        c.Source = source
+        getintegrator(c.dU, c.u, solver, c)()
+        assert (_routes(plan) == ["vv_rk4_steps"]) == fused
