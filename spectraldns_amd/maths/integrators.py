@@ -156,7 +156,10 @@ def getintegrator(rhs, u0, solver, context):
             raise NotImplementedError("the compensated state is carried by the fused NS RK4 step only")
         a = np.array([1. / 6., 1. / 3., 1. / 3., 1. / 6.], dtype=context.float)
         b = np.array([0.5, 0.5, 1.], dtype=context.float)
-        work = []
+        # the stage arrays: made here, not in a step that may be captured, unless the
+        # solver fuses its steps (then the first one that it cannot fuse makes them)
+        fuses = getattr(solver, "fuses_rk4", None)
+        work = [] if fuses is not None and fuses(solver, context) else [u0.clone(), u0.clone()]
 
         @wraps(RK4_stages)
         def func():

@@ -190,11 +190,16 @@ _module_elsasser = set_Elsasser
 _module_pressure = add_pressure_diffusion
 
 
+def fuses_rk4(solver, context):
+    """Whether fused_rk4_step runs for this solver and context."""
+    return solver.ComputeRHS is _module_rhs and _fused(solver, context)
+
+
 def fused_rk4_step(ub_hat, rhs, dt, solver, context):
     """One RK4 step of ub_hat in place with the stage updates inside the passes,
     the last stage's right-hand side in rhs and its pressure in P_hat; False
     where the right-hand side is not the module's own."""
-    if solver.ComputeRHS is not _module_rhs or not _fused(solver, context):
+    if not fuses_rk4(solver, context):
         return False
     context.T.plan.mhd_rk4_steps(ub_hat, [dt], params.nu, params.eta, context.P_hat, rhs)
     return True

@@ -167,11 +167,16 @@ _module_linear = add_linear
 _module_cross2 = cross2
 
 
+def fuses_rk4(solver, context):
+    """Whether fused_rk4_step runs for this solver and context."""
+    return solver.ComputeRHS is _module_rhs and _fused(solver, context)
+
+
 def fused_rk4_step(w_hat, rhs, dt, solver, context):
     """One RK4 step of w_hat in place with the stage updates inside the passes,
     the last stage's right-hand side in rhs; False where the right-hand side is
     not the module's own."""
-    if solver.ComputeRHS is not _module_rhs or not _fused(solver, context):
+    if not fuses_rk4(solver, context):
         return False
     src = context.Source
     if 0 < abs(src.data_ptr() - w_hat.data_ptr()) < w_hat.nbytes:
