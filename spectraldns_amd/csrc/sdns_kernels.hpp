@@ -1308,10 +1308,10 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
         for (int j = 0; j < NK; ++j) {
           const int e = (!PAD || j < E3) ? j : j + E3;
           const int eo = P * j * plane;
-          const Rt sc = kept(t + P * j) ? a.scale : Rt(0);
-          buf_store_so_nt<C>(cscale(X0[e], sc), ro, so, eo * CS);
-          buf_store_so_nt<C>(cscale(X1[e], sc), ro, so, (fs + eo) * CS);
-          buf_store_so_nt<C>(cscale(X2[e], sc), ro, so, (2 * fs + eo) * CS);
+          const bool cv = colconv & kept(t + P * j);
+          buf_store_so_nt<C>(cv ? cscale(X0[e], a.scale) : czero<C>(), ro, so, eo * CS);
+          buf_store_so_nt<C>(cv ? cscale(X1[e], a.scale) : czero<C>(), ro, so, (fs + eo) * CS);
+          buf_store_so_nt<C>(cv ? cscale(X2[e], a.scale) : czero<C>(), ro, so, (2 * fs + eo) * CS);
         }
       }
       return;
