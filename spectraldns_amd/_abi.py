@@ -492,6 +492,21 @@ class Plan:
         off = (-base) % 256
         return _P(base + off), self._mhd_ws.numel() - 256
 
+    @property
+    def mhd_fused(self):
+        """Whether the fused MHD stages serve this plan: the box within their reach
+        and memory for their workspace (asked for once: a plan that found none
+        stays with the step-by-step entries)."""
+        import torch
+        if getattr(self, "_mhd_no_memory", False) or not self.fused_stages:
+            return False
+        try:
+            self._mhd_workspace()
+        except torch.OutOfMemoryError:
+            self._mhd_no_memory = True
+            return False
+        return True
+
     def mhd_rhs(self, ub_hat, rhs, nu, eta, p_hat=None):
         self._spec(ub_hat, 6, "ub_hat")
         self._spec(rhs, 6, "rhs")

@@ -12,7 +12,7 @@ set_Elsasser, the Nyquist mask, pressure, diffusion and the stage update in
 the last pass; ub_dealias and ZZ_hat are not written then.  With a replaced
 step (conv, set_Elsasser, divergenceConvection, add_pressure_diffusion), or a
 box beyond the fused passes, each step is a launch of its own over those
-arrays.
+arrays; so do plans without memory left for the fused passes' workspace.
 
 Built for the 2/3 rule (shenfun's dealias_direct, dealias_mode 0), the 3/2
 rule (the six fields transformed onto the padded 3N/2 grid, the nine
@@ -161,12 +161,12 @@ def add_pressure_diffusion(rhs, ub_hat, nu, eta, K2, K, P_hat, K_over_K2):
 
 def _fused(solver, c):
     """Whether the right-hand side is the module's own (no step of it replaced)
-    and the fused passes reach the box.  conv and add_pressure_diffusion are the
+    and the fused passes serve the box.  conv and add_pressure_diffusion are the
     solver argument's, the others this module's, as the steps call them."""
     plan = c["T"].plan
     return (getattr(solver.conv, "mhd_fused", None) is solver.conv and solver.add_pressure_diffusion is _module_pressure and
             divergenceConvection is _module_convection and set_Elsasser is _module_elsasser and
-            plan.nyquist_masked == (c["mask"] is not None) and plan.fused_stages)
+            plan.nyquist_masked == (c["mask"] is not None) and plan.mhd_fused)
 
 
 def ComputeRHS(rhs, ub_hat, solver, **context):

@@ -188,3 +188,39 @@ def test_stage_arrays_of_the_other_convections(rk4):
             return super().clone(*a, **k)
     getintegrator(c.dU, c.u.as_subclass(State), solver, c)
     assert len(clones) == 2
+
+
+def test_mhd_without_memory_for_the_workspace(monkeypatch):
+    """No memory left for the fused workspace: the step-by-step arrays, which the
+    context holds, still serve."""
+    from spectraldns_amd._abi import Plan
+
+    def plan():
+        p = object.__new__(Plan)
+        p._h = None
+        p._lib = SimpleNamespace(sdns_mhd_workspace_bytes=lambda h: 1024, sdns_fused_stages=lambda h: 1)
+        p.device = torch.device("cpu")
+        return p
+    asked = []
+
+    def no_memory(*a, **k):
+        asked.append(1)
+        raise torch.OutOfMemoryError("out of memory")
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", no_memory)
+        p = plan()
+        assert not p.mhd_fused and not p.mhd_fused and asked == [1]
+    p = plan()
+    assert p.mhd_fused
+    ptr, nbytes = p._mhd_workspace()
+    assert ptr.value % 256 == 0 and nbytes >= 1024
+
+
+def test_mhd_plan_without_the_workspace_goes_step_by_step(rk4, monkeypatch):
+    from spectraldns_amd.maths.integrators import getintegrator
+    module, solver, c, plan = _setup("MHD")
+    plan.mhd_fused = False
+    solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c)
+    assert _routes(plan) == []
+    getintegrator(c.dU, c.u, solver, c)()
+    assert _routes(plan) == []
