@@ -255,7 +255,11 @@ void plan_layout(sdns_plan* p, bool plane) {
 //   16 -> 8 points).  In FP64 the LDS lines cost more than the registers, except
 //   at 96 and 192 points (256^3 3/2 rule 1.08 -> 1.02 ms).  Lines of 16 and 32
 //   points: more threads per line (64^3: 13.0 -> 10.1 us).
-//   x, y: the schedule with the block size that fills a CU's LDS better.
+//   x, y: the schedule with the block size that fills a CU's LDS better.  The
+//   x-forward's choice also holds for the boxes beyond a descriptor's reach (FP32:
+//   384 points 3.43 -> 3.25 ms a stage at 384 x 768 x 1024, 128 points 2.09 -> 2.05
+//   at 128 x 1536 x 1024; 0 at 512 points, 2.29 against 2.36 ms at 512 x 512 x 768
+//   and 2.52 against 2.68 compensated, where the descriptor form is the same with both).
 int default_variant(int pass, int len, int precision) {
   const bool f32 = precision == SDNS_SINGLE;
   auto in = [len](std::initializer_list<int> l) { return std::find(l.begin(), l.end(), len) != l.end() ? 1 : 0; };
@@ -267,7 +271,7 @@ int default_variant(int pass, int len, int precision) {
       if (f32) return len == 256 ? 3 : (len == 512 ? 1 : (len >= 36 ? 2 : 0));
       return in({96, 192}) ? 2 : 0;
     case 3: return f32 ? 0 : in({128});
-    case 4: return f32 ? in({64, 128, 384, 512}) : in({128});
+    case 4: return f32 ? in({64, 128, 384}) : in({128});
     default: return 0;
   }
 }

@@ -144,25 +144,24 @@ template <typename Rt, int M, int V, int MODE> void p5_go(const P5Args<Rt>& a, h
     // (the compensated stages of the 3/2 rule run p5_body)
     if (fits && p5b_padded(M, a) && (!a.lo || MODE == P5_RHS)) return p5b_go<Rt, M, EV, MODE, true>(a, s, nblk);
   }
-  constexpr int E0 = strided_E(M, 0);  // one schedule for the boxes beyond a descriptor's reach
-  using Cfg = SCfg<Rt, M, E0>;
+  using Cfg = SCfg<Rt, M, EV>;
   const int nt = (a.Q + Cfg::T - 1) / Cfg::T;
   if (nblk) *nblk = nt;
   const dim3 g(xcd_grid(nt)), b(Cfg::THREADS);
   constexpr bool RK = MODE != P5_RHS;
   if constexpr (sizeof(Rt) == 4 && RK) {
     if (a.lo) {
-      hipLaunchKernelGGL((k_p5<Rt, M, E0, MODE, rk_keep<Rt>(false, true), true>), g, b, 0, s, a);
+      hipLaunchKernelGGL((k_p5<Rt, M, EV, MODE, rk_keep<Rt>(false, true), true>), g, b, 0, s, a);
       return;
     }
   }
   if constexpr (RK && rk_keep<Rt>(true, false) != rk_keep<Rt>(false, false)) {
     if (M != a.N0) {
-      hipLaunchKernelGGL((k_p5<Rt, M, E0, MODE, rk_keep<Rt>(true, false), false>), g, b, 0, s, a);
+      hipLaunchKernelGGL((k_p5<Rt, M, EV, MODE, rk_keep<Rt>(true, false), false>), g, b, 0, s, a);
       return;
     }
   }
-  hipLaunchKernelGGL((k_p5<Rt, M, E0, MODE, rk_keep<Rt>(false, false), false>), g, b, 0, s, a);
+  hipLaunchKernelGGL((k_p5<Rt, M, EV, MODE, rk_keep<Rt>(false, false), false>), g, b, 0, s, a);
 }
 template <typename Rt, int M, int E> void strided_go(int dir, int nfields, const StridedArgs<Rt>& a0, hipStream_t s) {
   using Cfg = SCfg<Rt, M, E>;
