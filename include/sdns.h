@@ -54,12 +54,15 @@ int sdns_plan_destroy(sdns_plan* plan);
  * runs).  The z pass (id 2) has variants 2 and 3 too (its LDS-assisted scheme
  * with schedule 0 / 1) and 4 and 5 (rows staged HBM -> LDS by direct loads,
  * schedule 0 / 1; where the rows do not fit in LDS these run variant 2 / 3).
- * The x-forward + RK pass (id 4) has variants 2 and 3 too: schedules 0 / 1
- * whose plain RK stages under the 3/2 rule use kernels with the kept x rows
- * fixed at compile time (x lines of 96 to 768 points, arrays within 2 GiB;
- * other cases run as variants 0 / 1).
- * Set by the autotuner (spectraldns_amd/autotune.py). */
+ * The x-forward + RK pass (id 4) accepts 2 and 3 for schedules stored when it
+ * had such kernels; they mean 0 and 1.  Small boxes run the y, z and y passes
+ * (ids 1 to 3) as one launch, for which their variants have no effect (see
+ * sdns_plan_launches).  Set by the autotuner (spectraldns_amd/autotune.py). */
 int sdns_plan_set_variant(sdns_plan* plan, int pass, int variant);
+/* Whether a right-hand side or a step of the NS solver launches the pass (id 0
+ * to 4) by itself: 0 for the passes 1 to 3 of boxes whose x-planes fit in LDS,
+ * which run as one launch (timed as pass 2). */
+int sdns_plan_launches(const sdns_plan* plan, int pass);
 /* Rebind the plan to another HIP stream (NULL = null stream). */
 int sdns_plan_set_stream(sdns_plan* plan, void* hip_stream);
 /* Device workspace the plan needs; sdns_set_workspace hands it caller memory

@@ -22,6 +22,7 @@ _SIGS = {
                                         ctypes.c_int, ctypes.c_int, _P]),
     "sdns_plan_destroy": (ctypes.c_int, [_P]),
     "sdns_plan_set_stream": (ctypes.c_int, [_P, _P]),
+    "sdns_plan_launches": (ctypes.c_int, [_P, ctypes.c_int]),
     "sdns_plan_set_variant": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int]),
     "sdns_workspace_bytes": (ctypes.c_size_t, [_P]),
     "sdns_set_workspace": (ctypes.c_int, [_P, _P, ctypes.c_size_t]),
@@ -634,6 +635,11 @@ class Plan:
         being 0 and 1."""
         _check(self._lib.sdns_plan_set_variant(self._h, int(pass_id), int(variant)))
 
+    def launches(self, pass_id):
+        """Whether a right-hand side launches the pass (0..4) by itself: passes 1..3 of
+        small boxes are one launch, for which their variants have no effect."""
+        return bool(self._lib.sdns_plan_launches(self._h, int(pass_id)))
+
     # ---------------------------------------------------------------- timing
     PASS_NAMES = ("x_inverse", "y_inverse_curl", "z_cross", "y_forward", "x_forward_rk", "other")
 
@@ -724,6 +730,13 @@ class Batch:
             for k, l in enumerate((M[0], M[1], M[2] // 2, M[1], M[0])):
                 out.setdefault(k, set()).add(l)
         return {k: sorted(v) for k, v in out.items()}
+
+    def launches(self, pass_id):
+        """Whether an ensemble step launches the pass (0..4) by itself: with small boxes
+        alone, passes 1..3 are one launch per side."""
+        plan = _P()
+        _check(self._lib.sdns_batch_box_plan(self._h, 0, ctypes.byref(plan)))
+        return bool(self._lib.sdns_plan_launches(plan, int(pass_id)))
 
     def set_variant(self, pass_id, length, variant):
         """Schedule variant (0 or 1) of one batched pass for one line length."""

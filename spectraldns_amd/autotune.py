@@ -4,11 +4,11 @@ Every pass (0 x-inverse, 1 y-inverse + curl, 2 z + cross product, 3
 y-forward, 4 x-forward + RK stage) is compiled with up to two line-FFT
 schedules (points per thread and the radix sequence that follows from it,
 see sdns_device.hpp); the z pass also has three storage schemes (all in
-registers, LDS-assisted, LDS-DMA staging), six variants in all, and the
-x-forward + RK pass has its run-time row maps or its 3/2-rule stage kernels
-(kept rows fixed at compile time), four variants.  The tuner times each variant of each pass with HIP
-events inside real RK4 steps of the target box and keeps the fastest; the
-result is stored per box in ``schedules.json`` next to this file and applied
+registers, LDS-assisted, LDS-DMA staging), six variants in all.  The tuner
+times each variant of each pass with HIP events inside real RK4 steps of the
+target box and keeps the fastest; passes that the box does not launch by
+themselves (the y and z passes of small boxes) are left out.  The result is
+stored per box in ``schedules.json`` next to this file and applied
 by ``apply_schedule`` whenever a plan for that box is created.
 
     python -m spectraldns_amd.autotune --N 256 256 256 --precision single --dealias 3/2-rule
@@ -54,8 +54,8 @@ def apply_schedule(plan, path=SCHEDULE_FILE):
 
 
 def tune(N, L=(2 * np.pi,) * 3, precision="single", dealias="3/2-rule", mode=0, steps=3, seed=1234):
-    """Time every variant of every pass on RK4 steps of a random solenoidal
-    field; return {"variants": {pass: v}, "ms": {pass: [ms_v0, ms_v1, ...]}}."""
+    """Time every variant of every pass that the box launches on RK4 steps of a
+    random solenoidal field; return {"variants": {pass: v}, "ms": {pass: [ms_v0, ms_v1, ...]}}."""
     import torch
     from ._abi import Plan
     from .isotropic import random_solenoidal_field
@@ -64,8 +64,10 @@ def tune(N, L=(2 * np.pi,) * 3, precision="single", dealias="3/2-rule", mode=0, 
     u0 = torch.from_numpy(random_solenoidal_field(N, L, seed=seed, k0=4.0, energy=0.5)).to(cd).cuda()
     res = {"variants": {}, "ms": {}}
     for pid, name in enumerate(PASSES[:5]):
+        if not plan.launches(pid):
+            continue
         times = []
-        for var in ((0, 1, 2, 3, 4, 5) if pid == 2 else (0, 1, 2, 3) if pid == 4 else (0, 1)):
+        for var in ((0, 1, 2, 3, 4, 5) if pid == 2 else (0, 1)):
             plan.set_variant(pid, var)
             u = u0.clone()
             plan.rk4_steps(u, [1e-3], 1e-3)       # warm-up (first launch of this variant)
@@ -153,7 +155,7 @@ def tune_batch(sizes=None, precision="single", dealias="2/3-rule", mode=0, steps
     start = base
     chosen, ms = [], {}
     for k, lengths in sorted(ens.batch.line_lengths().items()):
-        for length in lengths:
+        for length in lengths if ens.batch.launches(k) else ():
             ens.reset()
             ens.batch.set_variant(k, length, 1)
             t1 = _time_ensemble(ens, steps)

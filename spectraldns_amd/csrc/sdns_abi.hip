@@ -1351,6 +1351,10 @@ int sdns_plan_set_variant(sdns_plan* p, int pass, int variant) {
   return 0;
 }
 
+int sdns_plan_launches(const sdns_plan* p, int pass) {
+  return p && pass >= 0 && pass <= 4 && !(p->plane && pass >= 1 && pass <= 3) ? 1 : 0;
+}
+
 int sdns_plan_set_stream(sdns_plan* p, void* s) {
   if (!p) return fail(SDNS_ERR_INVALID, "null plan");
   p->stream = (hipStream_t)s;
