@@ -247,14 +247,19 @@ template <typename Rt> int launch_plane(int M1, int n, const PlaneArgs<Rt>& a, h
   });
 }
 // Whether a box of M0 planes runs launch_plane (its plan lays out the work buffers
-// for it): where the plane fits in LDS, except few planes of 64 x 64 points, whose
-// 64 blocks leave the chip idle longer than three launches take.  Per
+// for it): where the plane fits in LDS, except few planes of the largest sizes,
+// whose few blocks leave the chip idle longer than three launches take.  Per
 // evaluation, three passes against the plane launch, with M0 = M1: FP32 32^2 18
 // against 10 us, 48^2 24 against 15, 64^2 16 against 19; FP64 21 against 11, 30
 // against 19, 22 against 34; the plane launch's time stays the same up to 256
-// planes (FP64 64^2: 38 us at 256).
+// planes (FP64 64^2: 38 us at 256).  Steps of 8 to 512 planes of every compiled
+// pair, both precisions, with the 2/3 rule and without (496 boxes): the plane
+// launch takes 0.48 to 1.0 of the three passes' step, but for FP64 planes of 32 or
+// 48 rows with 64-point z lines: 8 planes 116 against 108 us (32 rows) and 131
+// against 117 (48), 32 planes 125 against 122 and 143 against 138, even from 48 on.
 template <typename Rt> bool plane_fits(int M0, int M1, int n, int nkz) {
   if (M1 == 64 && n == 32 && M0 < (sizeof(Rt) == 4 ? 128 : 192)) return false;
+  if (sizeof(Rt) == 8 && M1 >= 32 && n == 32 && M0 < 48) return false;
   return plane_dispatch(M1, n, [&](auto mm, auto nn) {
            constexpr int m = decltype(mm)::value, h = decltype(nn)::value, TH = plane_threads(m, (int)sizeof(cx<Rt>));
            return plane_lds<m, h, TH>(nkz, (int)sizeof(cx<Rt>)) <= PLANE_LDS_MAX ? 0 : -1;
