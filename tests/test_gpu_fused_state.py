@@ -72,3 +72,51 @@ def test_vv_source_is_the_state(precision, monkeypatch):
     c.Source = start.clone()
     solver.getintegrator(c.dU, c.u, solver, c)()
     assert torch.equal(after, c.u)
+
+
+@pytest.mark.parametrize("name", ["VV", "MHD"])
+@pytest.mark.parametrize("precision", ["double", "single"])
+@pytest.mark.parametrize("N,dealias", [((256, 32, 64), "2/3-rule"), ((64, 128, 256), "2/3-rule"),
+                                       ((128, 64, 128), "None"), ((128, 32, 64), "3/2-rule")])
+def test_whole_tiles(name, precision, N, dealias, monkeypatch):
+    """x lines of 128 points and more, and grids of 512 blocks and more, whose
+    column tiles are not divided."""
+    print("\n[case]", name, N, precision, dealias, flush=True)
+    solver, c, config = _context(name, N, precision, dealias, True)
+    start = _start(c, N).to(c.u.dtype)
+    c.u.copy_(start)
+    fused = solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c).clone()
+    solver.getintegrator(c.dU, c.u, solver, c)()
+    after = c.u.clone()
+    with monkeypatch.context() as m:
+        _by_steps(solver, name, m)
+        c.u.copy_(start)
+        ref = solver.ComputeRHS(torch.empty_like(c.dU), c.u, solver, **c).clone()
+        assert _rel(fused, ref) <= (1e-13 if precision == "double" else 2e-6)
+        solver.getintegrator(c.dU, c.u, solver, c)()
+        assert _rel(after, c.u) <= (1e-14 if precision == "double" else 1e-6)
+
+
+@pytest.mark.parametrize("name", ["VV", "MHD"])
+def test_many_single_precision_steps(name, monkeypatch):
+    """50 FP32 steps of a smooth field: no further from FP64 than the stage by
+    stage step with its accumulator, whose error is the yardstick (1.5 times it:
+    the two round differently)."""
+    N = (32, 32, 32)
+    print("\n[case]", name, N, "50 steps", flush=True)
+
+    def run(precision, by_steps):
+        solver, c, config = _context(name, N, precision, "2/3-rule", True)
+        u = _start(c, N, 5, 4.0).to(torch.complex64)
+        c.u.copy_(u * (0.5 / float(u.abs().pow(2).sum().sqrt())))
+        with monkeypatch.context() as m:
+            if by_steps:
+                _by_steps(solver, name, m)
+            step = solver.getintegrator(c.dU, c.u, solver, c)
+            for _ in range(50):
+                step()
+        return c.u.to(torch.complex128).clone()
+    ref = run("double", True)
+    fused, steps = _rel(run("single", False), ref), _rel(run("single", True), ref)
+    print("fused %.2e, stage by stage %.2e" % (fused, steps), flush=True)
+    assert fused <= 1.5 * steps and fused <= 1e-5
