@@ -1226,6 +1226,25 @@ void batch_drop_graph(sdns_batch* b) {
   b->graph = nullptr;
 }
 
+// Whether an ensemble whose boxes all fit the plane kernel is faster with it.  The
+// sides' launches follow each other (a side's code and registers are its own), so
+// every further side adds a launch's latency, 8 to 23 us by its size, against the
+// three passes over all boxes; many planes hide it.  Two steps, plane against
+// passes, k boxes of each side, 2/3 rule: 32 246 / 345 us FP32 (k = 1); 64 485 /
+// 431 FP64 (k = 1), 527 / 525 (k = 2); 16 + 32 310 / 344; 32 + 48 427 / 397 FP32
+// (k = 1), 477 / 487 (k = 4); 48 + 64 755 / 623 FP64 (k = 2), 901 / 994 (k = 4);
+// 32 + 48 + 64 682 / 453 (k = 1), 773 / 747 (k = 4), 1003 / 1243 (k = 8);
+// 16 + 24 + 32 + 48 646 / 532 FP32 (k = 4), 711 / 738 (k = 8), 997 / 948 FP64
+// (k = 8), 1423 / 1674 (k = 16).
+bool batch_planes_pay(const std::map<int, int>& sides, int precision) {
+  int planes = 0;
+  for (const auto& s : sides) planes += s.second;
+  const int n = (int)sides.size(), largest = sides.rbegin()->first;
+  if (n == 1) return largest < 64 || planes >= 128;
+  if (n == 2 && largest <= 32) return true;
+  return planes >= (n > 3 && precision == SDNS_DOUBLE ? 400 : 320) * (n - 1);
+}
+
 int batch_capture(sdns_batch* b) {
   HIP_TRY(hipStreamBeginCapture(b->own, hipStreamCaptureModeThreadLocal));
   const int rc = batch_step_any(b, b->own);
@@ -1736,9 +1755,13 @@ int sdns_batch_create(sdns_batch** out, int nbox, const int32_t* N, const double
   }
   // plane launches for all boxes or for none: the passes run over whole ensembles
   bool planes = true;
-  for (const sdns_plan* p : b->box)
+  std::map<int, int> sides;  // x-planes by side
+  for (const sdns_plan* p : b->box) {
     planes = planes && (precision == SDNS_DOUBLE ? batch_plane_fits<double>(p->M[1], p->n2h, p->nkz)
                                                  : batch_plane_fits<float>(p->M[1], p->n2h, p->nkz));
+    sides[p->M[1]] += p->M[0];
+  }
+  planes = planes && batch_planes_pay(sides, precision);
   for (sdns_plan* p : b->box) {
     plan_layout(p, planes);
     const int rc = ensure_workspace(p);
