@@ -413,8 +413,7 @@ template <typename C> __device__ __forceinline__ C r2c_bin(C A, C Bz, C w) {
 // Post-process of the forward half-length FFT held in z (natural positions
 // t + P e); `my` is this line's LDS area.  Writes kept bins k < nk (and the
 // Nyquist bin n when nk > n).
-// STREAM: non-temporal stores, for rows that start on 128-byte lines; rows that
-// do not share lines with their neighbours' through L2 and stay cached.
+// STREAM: non-temporal stores (see r2c_streams).
 template <typename Rt, int n, int E, bool WAVE = false, bool STREAM = true>
 __device__ __forceinline__ void r2c_post(cx<Rt> (&z)[E], cx<Rt>* my, cx<Rt>* __restrict__ out, int nk, bool valid,
                                          const cx<Rt>* __restrict__ rtw, int t, Rt scale) {
@@ -849,7 +848,7 @@ __global__ void __launch_bounds__((ZCfg<Rt, n, E>::THREADS / D), (occ_for(E + st
   lds_barrier<WL>();
   Ff::run(z, t, my, 1, tw);
   C* out = (C*)a.out + blockIdx.y * a.out_field + li * a.out_line;
-  if (a.out_line * (long)sizeof(C) % 128 == 0) r2c_post<Rt, n, E, WL, true>(z, my, out, a.nk, valid, rtw, t, a.scale);
+  if (a.stream) r2c_post<Rt, n, E, WL, true>(z, my, out, a.nk, valid, rtw, t, a.scale);
   else r2c_post<Rt, n, E, WL, false>(z, my, out, a.nk, valid, rtw, t, a.scale);
 }
 

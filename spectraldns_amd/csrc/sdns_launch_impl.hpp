@@ -177,8 +177,22 @@ template <typename Rt, int M, int E> void strided_go(int dir, int nfields, const
     else hipLaunchKernelGGL((k_strided<Rt, M, E, 1, D>), gd, bd, 0, s, a);
   });
 }
-template <typename Rt, int n, int E> void z_go(int dir, int nfields, const ZArgs<Rt>& a, hipStream_t s) {
+// Whether the R2C pass writes its rows with non-temporal stores: where they start on
+// 128-byte lines; other rows share a line with each neighbour, which cached stores
+// complete in L2 (forward transform of three components, non-temporal against
+// cached: 256^3 FP32 266 / 231 us, FP64 539 / 502, 96^3 FP64 35.9 / 31.2), unless
+// the shared lines are few (rows of 6 KB: 128 x 128 x 1536 FP32 326 / 336) or the
+// output is small, where the next pass waits for the dirty lines (64^3 FP64, 6 MB
+// of 528-byte rows: 17.8 / 18.4; 72^3 FP64 23.7 / 25.2; 32 x 32 x 1024 FP32, 12 MB
+// of 4 KB rows: 27.0 / 29.0).
+inline bool r2c_streams(long row, long bytes) {
+  return row % 128 == 0 || row >= 6144 || (row >= 256 && bytes < (10L << 20)) || (row >= 2048 && bytes < (16L << 20));
+}
+template <typename Rt, int n, int E> void z_go(int dir, int nfields, const ZArgs<Rt>& a0, hipStream_t s) {
   using Cfg = ZCfg<Rt, n, E>;
+  ZArgs<Rt> a = a0;
+  const long row = a.out_line * (long)sizeof(cx<Rt>);
+  a.stream = dir < 0 && r2c_streams(row, row * a.L * nfields);
   constexpr int MD = max_div(n, 64, Cfg::LPB, Cfg::THREADS);
   with_div<MD>(tile_div((long)nfields * ((a.L + Cfg::LPB - 1) / Cfg::LPB), MD), [&](auto dd) {
     constexpr int D = decltype(dd)::value, LPB = Cfg::LPB / D;

@@ -95,6 +95,7 @@ template <typename Rt> struct ZArgs {
   int L;
   int nk;             // spectral bins kept (input of C2R / output of R2C)
   long in_line, in_field, out_line, out_field;  // element strides
+  int stream;         // R2C: non-temporal stores (set by the launcher)
   Rt scale;
 };
 
