@@ -323,6 +323,8 @@ void tstop(sdns_plan* p) {
 }
 
 // ---------------------------------------------------------------- transforms
+// Tile order of the y passes by the bins of a row (see xcd_tile_run).
+int y_run(int Nh) { return Nh >= 96 ? 5 : XCD_EIGHTHS; }
 // With trunc, each pass reads only the plan's kept input modes of its axis (the
 // others count as zero): the tensor-product truncation of a 2/3-rule
 // dealiased backward transform, inside the transform.
@@ -333,6 +335,7 @@ template <typename Rt> int plain_backward(sdns_plan* p, const void* uh, void* up
   // x inverse: columns (iy, kz) contiguous
   a.in = uh; a.out = p->bufA; a.tw = p->tw[N0];
   a.Q = (int)plane; a.cdiv = (int)plane; a.cvalid = (int)plane; a.in_hi = 0; a.out_hi = 0;
+  a.run = XCD_EIGHTHS;
   a.in_row = plane; a.out_row = plane; a.in_field = fs; a.out_field = fs;
   a.rout = rmap(N0 / 2, N0 / 2 - 1, N0);
   a.rin = trunc ? rmap(p->in[0][0], p->in[0][1], N0) : a.rout;
@@ -341,6 +344,7 @@ template <typename Rt> int plain_backward(sdns_plan* p, const void* uh, void* up
   // y inverse: columns (x, kz)
   a.in = p->bufA; a.out = p->bufB; a.tw = p->tw[N1];
   a.Q = N0 * Nh; a.cdiv = Nh; a.cvalid = Nh; a.in_hi = plane; a.out_hi = plane; a.in_row = Nh; a.out_row = Nh;
+  a.run = y_run(Nh);
   a.rout = rmap(N1 / 2, N1 / 2 - 1, N1);
   a.rin = trunc ? rmap(p->in[1][0], p->in[1][1], N1) : a.rout;
   if (launch_strided<Rt>(N1, p->var[5], +1, nc, a, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "y length %d", N1);
@@ -367,11 +371,13 @@ template <typename Rt> int plain_forward(sdns_plan* p, const void* up, void* uh,
   StridedArgs<Rt> a{};
   a.in = bufA; a.out = bufB; a.tw = p->tw[N1];
   a.Q = N0 * Nh; a.cdiv = Nh; a.cvalid = Nh; a.in_hi = plane; a.out_hi = plane; a.in_row = Nh; a.out_row = Nh;
+  a.run = y_run(Nh);
   a.in_field = fs; a.out_field = fs;
   a.rin = rmap(N1 / 2, N1 / 2 - 1, N1); a.rout = a.rin; a.scale = Rt(1);
   if (launch_strided<Rt>(N1, p->var[5], -1, nc, a, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "y length %d", N1);
   a.in = bufB; a.out = uh; a.tw = p->tw[N0];
   a.Q = (int)plane; a.cdiv = (int)plane; a.cvalid = (int)plane; a.in_hi = 0; a.out_hi = 0; a.in_row = plane;
+  a.run = XCD_EIGHTHS;
   a.out_row = plane;
   a.rin = rmap(N0 / 2, N0 / 2 - 1, N0); a.rout = a.rin;
   a.scale = (Rt)(1.0 / ((double)N0 * N1 * N2));
@@ -394,6 +400,7 @@ template <typename Rt> int padded_backward(sdns_plan* p, const void* uh, void* u
   StridedArgs<Rt> a{};
   a.in = uh; a.out = p->bufA; a.tw = p->tw.at(M0);
   a.Q = (int)plane; a.cdiv = (int)plane; a.cvalid = (int)plane; a.in_hi = 0; a.out_hi = 0;
+  a.run = XCD_EIGHTHS;
   a.in_row = plane; a.out_row = plane; a.in_field = (long)N0 * plane; a.out_field = (long)M0 * plane;
   a.rin = rmap(p->in[0][0], p->in[0][1], N0);
   a.rout = rmap(M0 / 2, M0 / 2 - 1, M0);
@@ -401,6 +408,7 @@ template <typename Rt> int padded_backward(sdns_plan* p, const void* uh, void* u
   if (launch_strided<Rt>(M0, p->var[5], +1, nc, a, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "x length %d", M0);
   a.in = p->bufA; a.out = p->bufB; a.tw = p->tw.at(M1);
   a.Q = M0 * Nh; a.cdiv = Nh; a.cvalid = Nh; a.in_hi = plane; a.out_hi = (long)M1 * Nh; a.in_row = Nh;
+  a.run = y_run(Nh);
   a.out_row = Nh; a.in_field = (long)M0 * plane; a.out_field = (long)M0 * M1 * Nh;
   a.rin = rmap(p->in[1][0], p->in[1][1], N1);
   a.rout = rmap(M1 / 2, M1 / 2 - 1, M1);
@@ -425,6 +433,7 @@ template <typename Rt> int padded_forward(sdns_plan* p, const void* up, void* uh
   StridedArgs<Rt> a{};
   a.in = p->bufA; a.out = p->bufB; a.tw = p->tw.at(M1);
   a.Q = M0 * Nh; a.cdiv = Nh; a.cvalid = Nh; a.in_hi = (long)M1 * Nh; a.out_hi = plane; a.in_row = Nh;
+  a.run = y_run(Nh);
   a.out_row = Nh; a.in_field = (long)M0 * M1 * Nh; a.out_field = (long)M0 * plane;
   a.rin = rmap(M1 / 2, M1 / 2 - 1, M1);
   a.rout = rmap(p->out[1][0], p->out[1][1], N1);
@@ -432,6 +441,7 @@ template <typename Rt> int padded_forward(sdns_plan* p, const void* up, void* uh
   if (launch_strided<Rt>(M1, p->var[5], -1, nc, a, p->stream)) return fail(SDNS_ERR_UNSUPPORTED, "y length %d", M1);
   a.in = p->bufB; a.out = uh; a.tw = p->tw.at(M0);
   a.Q = (int)plane; a.cdiv = (int)plane; a.cvalid = (int)plane; a.in_hi = 0; a.out_hi = 0; a.in_row = plane;
+  a.run = XCD_EIGHTHS;
   a.out_row = plane; a.in_field = (long)M0 * plane; a.out_field = (long)N0 * plane;
   a.rin = rmap(M0 / 2, M0 / 2 - 1, M0);
   a.rout = rmap(p->out[0][0], p->out[0][1], N0);

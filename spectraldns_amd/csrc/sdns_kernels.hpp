@@ -90,14 +90,27 @@ constexpr int stage_k(int n, int P) { return (n + 1 + P - 1) / P; }
 // alike.  (With one contiguous eighth of the tiles per XCD: 256^3 FP32 P2
 // 288 against 279 us, x-forward 287 against 257 us, 512^3 y-forward 606 against
 // 592 us, 256^3 FP64 y-forward 275 against 265 us, x-forward 444 against 427 us;
-// with G = 4 the y-forward takes 147 us instead of 131, with 32, which keeps the
-// tiles of a few whole planes together, MHD's takes 220 us against 237 with 16:
-// the strided passes use 32.)  Launch
+// with G = 4 the y-forward takes 147 us instead of 131.)  Launch
 // 8*ceil(ntiles/8) blocks; returns -1 for the padding blocks.
 template <int G = 16> __device__ __forceinline__ int xcd_tile(int ntiles) {
   const int per = (ntiles + 7) >> 3, full = per / G * G;
   const int x = (int)(blockIdx.x & 7), s = (int)(blockIdx.x >> 3);
   const int t = s < full ? (s / G * 8 + x) * G + s % G : 8 * full + x * (per - full) + (s - full);
+  return t < ntiles ? t : -1;
+}
+// The same with 1 << run tiles per run, for the strided passes: with 32, which
+// keeps the tiles of a few whole planes together, MHD's y-forward takes 214 us
+// against 235 with 16 and 219 in eighths, 512 x 512 x 64 FP32 y-inverse 149 against
+// 162 in eighths.  The plain transforms' x pass, one range of columns whose rows
+// are a plane apart, and their y pass on short rows (under 96 bins: a run is many
+// planes) go in eighths: backward transform of three components 256^3 FP64 547 ->
+// 505 us, 384^3 FP64 1624 -> 1564, 512 x 512 x 64 FP64 541 -> 531, 1024 x 128 x 128
+// FP32 forward 382 -> 365.
+__device__ __forceinline__ int xcd_tile_run(int ntiles, int run) {
+  const int per = (ntiles + 7) >> 3, full = per >> run << run;
+  const int x = (int)(blockIdx.x & 7), s = (int)(blockIdx.x >> 3);
+  const int t = s < full ? ((((s >> run) << 3) + x) << run) + (s & ((1 << run) - 1))
+                         : 8 * full + x * (per - full) + (s - full);
   return t < ntiles ? t : -1;
 }
 inline int xcd_grid(int ntiles) { return ((ntiles + 7) / 8) * 8; }
@@ -896,7 +909,7 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS / D), (occ_for(E, esz
   constexpr int T = SCfg<Rt, M, E>::T / D;
   __shared__ C lds[M * T];
   __shared__ C tw[M];
-  const int tile = xcd_tile<32>((a.Q + T - 1) / T);
+  const int tile = xcd_tile_run((a.Q + T - 1) / T, a.run);
   if (tile < 0) return;
   table_to_lds(tw, (const C*)a.tw, M);
   strided_body<Rt, M, E, DIR, T>(a, tile, blockIdx.y, lds, tw);

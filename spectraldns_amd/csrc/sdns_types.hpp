@@ -69,6 +69,10 @@ template <typename Rt> struct P3Args {  // z C2R x6, cross product, z R2C x3
   int L;              // M0 * M1 lines
 };
 
+// Order of a strided pass's tiles on the XCDs (StridedArgs::run): no runs, each XCD
+// one contiguous eighth.
+constexpr int XCD_EIGHTHS = 30;
+
 // Generic batched strided-axis transform: columns q = hi*cdiv + lo live at
 // offset hi*hi_stride + lo; row r of a column at offset r*row_stride; field f
 // (blockIdx.y) at offset f*field_stride.
@@ -81,6 +85,7 @@ template <typename Rt> struct StridedArgs {
   long out_hi, out_row, out_field;
   RowMap rin, rout;
   Rt scale;           // applied to every output (1 = none)
+  int run = 5;        // log2 of the tiles per run on one XCD (xcd_tile_run)
   int stream_in, stream_out;  // non-temporal loads / stores (set by the launcher
                               // when every column tile covers whole 128-byte lines)
 };
