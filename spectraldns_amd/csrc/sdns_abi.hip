@@ -253,8 +253,8 @@ void plan_layout(sdns_plan* p, bool plane) {
 //   parking two of them in LDS (2, 3) is 1.1 to 1.7 times faster from 36-point
 //   lines on (256^3 3/2 rule 0.63 -> 0.37 ms, 512^3 2/3 rule 1.69 -> 1.10 ms with
 //   16 -> 8 points).  In FP64 the LDS lines cost more than the registers, except
-//   at 96 and 192 points (256^3 3/2 rule 1.08 -> 1.02 ms).  Lines of 16 and 32
-//   points: more threads per line (64^3: 13.0 -> 10.1 us).
+//   at 96 and 192 points (256^3 3/2 rule 1.08 -> 1.02 ms).  Lines of 32 points:
+//   more threads per line (64^3: 13.0 -> 10.1 us).
 //   x, y: the schedule with the block size that fills a CU's LDS better.  The
 //   x-forward's choice also holds for the boxes beyond a descriptor's reach (FP32:
 //   384 points 3.43 -> 3.25 ms a stage at 384 x 768 x 1024, 128 points 2.09 -> 2.05
@@ -267,7 +267,7 @@ int default_variant(int pass, int len, int precision) {
     case 0: return f32 ? in({128, 192, 256, 384}) : in({128});
     case 1: return f32 ? in({128, 256, 512}) : in({64, 128, 256});
     case 2:
-      if (in({16, 32})) return 1;
+      if (len == 32) return 1;
       if (f32) return len == 256 ? 3 : (len == 512 ? 1 : (len >= 36 ? 2 : 0));
       return in({96, 192}) ? 2 : 0;
     case 3: return f32 ? 0 : in({128});

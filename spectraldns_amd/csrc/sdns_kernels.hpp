@@ -1534,8 +1534,7 @@ __global__ void __launch_bounds__((ZCfg<Rt, n, E>::THREADS), (occ_for(7 * E + st
 // are live; then mask, pressure (U) and diffusion (MHD.py:135-176) and the RK4
 // stage as in p5b_body with KEEP_STATES.  Buffer descriptors span three fields
 // or components each.  Bound like p5b_body; 256^3 FP32, mean of the stages: 553
-// us with linear stage arrays, every tile transformed and an eighth of the tiles
-// per XCD, 500 us now.  Two 8-wave blocks per CU need 128 registers (mhd_x_occ).
+// us with linear stage arrays and an eighth of the tiles per XCD, 500 us now.  Two 8-wave blocks per CU need 128 registers (mhd_x_occ).
 template <typename Rt, int M, int E> constexpr int mhd_x_occ() {
   const int o = occ_for(5 * E, esz_of<Rt>());
   return sizeof(Rt) == 4 && E <= 8 ? 4 : o;
@@ -1599,11 +1598,8 @@ __global__ void __launch_bounds__((SCfg<Rt, M, E>::THREADS), (mhd_x_occ<Rt, M, E
     for (int e = 0; e < E; ++e) X[e] = Y[e];
   };
   __syncthreads();
-  static_assert(T <= 64 && T * P % 64 == 0, "a wave holds every column");
-  if (__any(colconv)) {  // as in p5b_body
-    if (h == 0) sfor<6>([&](auto fc) { add(fc); });
-    else sfor<3>([&](auto fc) { add(std::integral_constant<int, decltype(fc)::value + 6>{}); });
-  }
+  if (h == 0) sfor<6>([&](auto fc) { add(fc); });
+  else sfor<3>([&](auto fc) { add(std::integral_constant<int, decltype(fc)::value + 6>{}); });
   if (!valid) return;
   const int plane = a.N1 * a.Nh, fs = a.N0 * plane;
   const long span = 3L * fs * CS;
