@@ -248,7 +248,9 @@ void plan_layout(sdns_plan* p, bool plane) {
 // Schedule variant of each pass for a box that the autotuner's table does not
 // hold, by line length: variant 1 (and for the z pass 2 and 3, the LDS-assisted
 // scheme) where it measured faster on cubes of 32..512 points with either
-// dealiasing rule, by more than 2%; 0 elsewhere.  What decides:
+// dealiasing rule, by more than 2%; 0 elsewhere.  (Timed again with the present x
+// passes: every alternative it takes is still faster or even, at worst 1.2% slower.)
+// What decides:
 //   z: six lines of 12 to 16 points per thread take 200 to 256 registers in FP32;
 //   parking two of them in LDS (2, 3) is 1.1 to 1.7 times faster from 36-point
 //   lines on (256^3 3/2 rule 0.63 -> 0.37 ms, 512^3 2/3 rule 1.69 -> 1.10 ms with

@@ -128,7 +128,7 @@ __device__ __forceinline__ void table_to_lds(C* dst, const C* __restrict__ src, 
 // x-inverse of one field: u, v, w from a.u, then wx, wy, wz from a.w.
 // INC: the state is u + ds d, formed on reading (the RK stages of KEEP_RHS; a
 // template, since a second loop behind a branch cost every stage its schedule).
-// Bound by its rows and stores: 3.1 TB/s at 256^3 3/2 rule FP32 (142 us).
+// Bound by its rows and stores: 10.5 F in 142 us at 256^3 3/2 rule FP32, 5.0 TB/s.
 template <typename Rt, int M, int E, int T, bool INC>
 __device__ __forceinline__ void p1_body(const P1Args<Rt>& a, int tile, int yb, cx<Rt>* lds, const cx<Rt>* tw) {
   using C = cx<Rt>;
@@ -1206,11 +1206,11 @@ __device__ __forceinline__ void p5_body(const P5Args<Rt>& a, int tile, cx<Rt>* l
 // The host checks that the three components of a state array and of W4 span
 // at most BUF_OOB bytes (p5b_fits); larger boxes run p5_body.  The per-mode
 // arithmetic is p5_body's.
-// Bound by the strided rows (128 bytes each, 3..5 streams) at 2.4..3.6 TB/s, its
-// blocks alternating between loading W4, the transforms and the update.  Mean of
-// the four stages, p5_body -> now: 256^3 FP32 2/3 rule 245 -> 199 us (217 with
-// the skip and one eighth of the tiles per XCD), 3/2 rule 283 -> 258 us, FP64 3/2
-// rule 548 -> 427 us, 512^3 FP32 compensated 2.8 -> 1.5 ms.
+// Bound by the strided rows (128 bytes each, 3..5 streams) at 4.3 TB/s (12.75 F in
+// 199 us, 16.5 F in 258 us), its blocks alternating between loading W4, the
+// transforms and the update.  Mean of the four stages, p5_body -> now: 256^3 FP32
+// 2/3 rule 245 -> 199 us (217 with one eighth of the tiles per XCD), 3/2 rule
+// 283 -> 258 us, FP64 3/2 rule 548 -> 427 us, 512^3 FP32 compensated 2.8 -> 1.6 ms.
 // EARLY: the first rows are loaded beside W4, before the transforms (divided
 // tiles: a grid of a few blocks per CU pays one latency less; in full grids the
 // 24..50 registers cost spills or occupancy).
@@ -1241,9 +1241,12 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
   const auto rw = buf_rsrc(a.w4, 3L * wfield * CS);
   const int wo = colconv ? (t * wrow + kyc * a.nkzop + kz) * CS : BUF_OOB;
   C X0[E], X1[E], X2[E];
-  // a tile without kept modes (half of them under the 2/3 rule) skips the
-  // transforms; every wave holds all T columns, so all decide alike.  (In a grid
-  // of few blocks the kept tiles alone set the time, so no test there.)
+  // a tile without kept modes skips the transforms; every wave holds all T columns,
+  // so all decide alike.  Only a rule that masks the output (dealias_mode 1) has
+  // such tiles, the others keep every mode here: mean of the stages at 256^3, mode 1,
+  // FP32 175 -> 162 us, FP64 330 -> 319, 192^3 64 -> 62 and 134 -> 126 (with mode 0
+  // the test is never false, 198 -> 193 and 373 -> 376 us as the loop is compiled).
+  // In a grid of few blocks the kept tiles alone set the time, so no test there.
   static_assert(T <= 64 && TH % 64 == 0, "a wave holds every column");
   const bool transform = EARLY_ || __any(colconv);
 #pragma unroll
@@ -1389,6 +1392,8 @@ __device__ __forceinline__ void p5b_body(const P5Args<Rt>& a, int tile, cx<Rt>* 
           buf_store_so_nt<C>(x, ro, OUT_S ? sso : so, OUT_S ? os : o);
         }
         if constexpr (!VV && (MODE == P5_RHS || MODE == P5_RK3)) buf_store_so_nt<C>(ph, rph, so, eo * CS);
+        // (also without partials: behind a test of them the stages took longer, 256^3 FP32
+        // 2/3 rule 193 -> 201 us, FP64 3/2 rule 426 -> 442)
         if constexpr (MODE == P5_RK3) energy_terms(v, Kv[0], K1, K2c, wz, esum, osum);
       }
       if (j0 + G < NK) {

@@ -106,7 +106,8 @@ template <typename Rt, int n, int E> void p3c_go(const P3Args<Rt>& a, hipStream_
 }
 // P5 through buffer descriptors (k_p5b) wherever they reach: byte offsets are
 // 31 bits, so the three components of a state array and of W4 have to span at
-// most BUF_OOB bytes (boxes up to about 640^3 in FP32).  Larger boxes run k_p5.
+// most BUF_OOB bytes (FP32 boxes up to about 560^3, with the 3/2 rule, whose W4 is
+// 3/2 times the state, up to about 480^3: 512^3 is beyond).  Larger boxes run k_p5.
 template <typename Rt> bool p5b_fits(int M, int N0, int N1, int Nh, int nkyo, int nkzop) {
   const long esz = 2 * (long)sizeof(Rt);
   return 3L * N0 * tiled_cols<Rt>(N1 * Nh) * esz <= BUF_OOB && 3L * M * nkyo * nkzop * esz <= BUF_OOB;

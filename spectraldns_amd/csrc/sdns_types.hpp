@@ -132,9 +132,11 @@ enum P5Mode { P5_RHS = 0, P5_RK0 = 1, P5_RK12 = 2, P5_RK3 = 3 };
 //     and the last stage adds the terms with the accumulator's roundings, plain
 //     or compensated: 39 F, 12 F written, and 9 F more in the x-inverse pass times
 //     the share of the modes that it reads (0.3 with the 2/3 rule).
-// FP64 keeps the states.  FP32 keeps the accumulator's roundings: right-hand
-// sides, except with the 3/2 rule, whose x-inverse reads every mode (256^3:
-// 4.95 ms per step with the sum, 5.12 ms with right-hand sides).
+// FP64 keeps the states, and so do VV and MHD in FP32 (50 steps of 32^3: 1.3e-7 and
+// 1.4e-7 from FP64, with an accumulator 2.6e-7 and 2.0e-7).  FP32 NS keeps the
+// accumulator's roundings: right-hand sides, except with the 3/2 rule, whose
+// x-inverse reads every mode (256^3: 4.95 ms per step with the sum, 5.12 ms with
+// right-hand sides).
 enum RkKeep { KEEP_SUM = 0, KEEP_STATES = 1, KEEP_RHS = 2 };
 template <typename Rt> constexpr int rk_keep(bool padded, bool comp) {
   return sizeof(Rt) == 8 ? KEEP_STATES : (padded && !comp ? KEEP_SUM : KEEP_RHS);
