@@ -298,17 +298,18 @@ def closure_timing(steps=20, warmup=3):
 # F = N0*N1*(N2/2+1)*esz (one complex spectral field; a real physical field is
 # counted as F too), 2/3 rule.  VV, fused stages: x-inverse of the curl-inverse
 # velocity and the vorticity 3F + 6F, y 12F, z 9F, y-forward 6F, x-forward 3F =
-# 39F per RHS; RK4 with kept stage states 6F + 9F + 9F + 15F.  MHD, fused
+# 39F per RHS; RK4 with kept stage states 6F + 9F + 9F + 15F, and the last
+# stage's right-hand side 3F.  MHD, fused
 # stages: x-inverse and y 12F each, z pass of six fields and nine products 15F,
-# y-forward 18F, x-forward 9F = 66F per RHS; RK4 over six components 78F.  NS
+# y-forward 18F, x-forward 9F = 66F per RHS; RK4 over six components 78F + 6F.  NS
 # integrators: fused RHS 44F (P1-P4 34F; x-forward with
 # the projection reads W4 and u_hat, writes rhs and P_hat: 10F);
 # ForwardEuler update 9F; AB2 updates 12F + 6F; BS5 (FSAL: 7 RHS per step
 # after the first) stage sums sum_{i=1..7} 3(i+2)F = 126F, solution sum 30F,
 # error sum 27F, error norm 9F, copy of the new state 6F.
 SOLVER_BYTES_F = {
-    ("VV", "RK4"): 4 * 39 + 39,
-    ("MHD", "RK4"): 4 * 66 + 78,
+    ("VV", "RK4"): 4 * 39 + 39 + 3,
+    ("MHD", "RK4"): 4 * 66 + 78 + 6,
     ("NS", "ForwardEuler"): 44 + 9,
     ("NS", "AB2"): 44 + 18,
     ("NS", "BS5_fixed"): 7 * 44 + 126 + 30 + 27 + 9 + 6,

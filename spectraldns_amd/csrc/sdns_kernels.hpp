@@ -1539,7 +1539,8 @@ __global__ void __launch_bounds__((ZCfg<Rt, n, E>::THREADS), (occ_for(7 * E + st
 // are live; then mask, pressure (U) and diffusion (MHD.py:135-176) and the RK4
 // stage as in p5b_body with KEEP_STATES.  Buffer descriptors span three fields
 // or components each.  Bound like p5b_body; 256^3 FP32, mean of the stages: 553
-// us with linear stage arrays and an eighth of the tiles per XCD, 500 us now.  Two 8-wave blocks per CU need 128 registers (mhd_x_occ).
+// us with linear stage arrays and an eighth of the tiles per XCD, 500 us now, 525
+// with the last right-hand side stored.  Two 8-wave blocks per CU need 128 registers (mhd_x_occ).
 template <typename Rt, int M, int E> constexpr int mhd_x_occ() {
   const int o = occ_for(5 * E, esz_of<Rt>());
   return sizeof(Rt) == 4 && E <= 8 ? 4 : o;

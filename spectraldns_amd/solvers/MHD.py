@@ -9,7 +9,8 @@ The module keeps the reference's protocol (``get_context`` with its keys,
 (sdns_mhd_rhs, sdns_mhd_rk4_steps): dealiased inverse transforms of the six
 fields, the nine products formed in the z pass, and the sums of
 set_Elsasser, the Nyquist mask, pressure, diffusion and the stage update in
-the last pass; ub_dealias and ZZ_hat are not written then.  With a replaced
+the last pass; the work arrays ub_dealias and ZZ_hat are not written then (dU and
+P_hat are: the last stage's right-hand side and pressure).  With a replaced
 step (conv, set_Elsasser, divergenceConvection, add_pressure_diffusion), or a
 box beyond the fused passes, each step is a launch of its own over those
 arrays; so do plans without memory left for the fused passes' workspace.

@@ -13,6 +13,10 @@ reference's w_dealias = VTp.backward(w_hat) for any W_hat, including one with
 a mean or a gradient part (a random start, a Source with a mean).  K2 and
 K_over_K2 are handles that carry the plan; the kernels form K^2 on the fly,
 and indexing a handle materialises the array.
+
+The right-hand side and RK4 run in fused passes (sdns_vv_rhs, sdns_vv_rk4_steps),
+which leave the last stage's right-hand side in dU; with a replaced step (conv,
+add_linear, ComputeRHS) each is a launch of its own.
 """
 from .NS import *  # noqa: F401,F403
 from .NS import config, params, HDF5File, optimizer, cross2, end_of_tstep  # noqa: F401
